@@ -6,6 +6,7 @@
 // (k_minmax_fold); the statistics pass folds its own in the last workgroup
 // to finish (ticket on a control counter that it resets).
 #include <algorithm>
+#include <cstddef>
 #include <vector>
 #include <limits>
 
@@ -39,17 +40,6 @@ __device__ __forceinline__ uint64_t block_reduce_max(uint64_t v, uint64_t* sm) {
     __syncthreads();
     return r;
 }
-template <typename A> __device__ __forceinline__ A block_reduce_sum(A v, A* sm) {
-    v = wave_sum(v);
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-    if (lane == 0) sm[wid] = v;
-    __syncthreads();
-    A r = 0;
-    for (int w = 0; w < kBlock / kWave; w++) r += sm[w];
-    __syncthreads();
-    return r;
-}
-
 __device__ __forceinline__ uint64_t rd(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -375,9 +365,14 @@ struct StatsAcc {
     uint32_t prec, dmax;
 };
 
+// LDS copies of the bit-width histogram: lane l counts in copy l % 32, so the
+// rows of a wave, which mostly share a width, never meet in a bank (two lanes
+// of the wave share a copy).
+constexpr int kHistCopies = 32;
+
 template <typename T>
 __device__ __forceinline__ void stats_elem(StatsAcc& a, T v, T next, bool has_next, bool has_next2, size_t row,
-                                           uint32_t* sm_hist, uint32_t* sm_hll) {
+                                           uint32_t* sm_hist, volatile uint32_t* sm_hll) {
     if constexpr (std::is_floating_point<T>::value) {
         FoldKeys<T> fk;
         fk.kmn = a.mn;
@@ -412,25 +407,67 @@ __device__ __forceinline__ void stats_elem(StatsAcc& a, T v, T next, bool has_ne
         }
     }
     if (has_next2 && rl_equal(v, next)) a.rl_eq++;
-    atomicAdd(&sm_hist[bitwidth64(zigzag_bits(v))], 1u);
+    atomicAdd(&sm_hist[bitwidth64(zigzag_bits(v)) * kHistCopies + (threadIdx.x & (kHistCopies - 1))], 1u);
     const uint64_t h = mix64(ubits(v) + 0x9e3779b97f4a7c15ull);
     const uint32_t reg = (uint32_t)(h >> 58);
     const uint32_t rank = (uint32_t)__clzll((h << 6) | (1ull << 5)) + 1;
-    atomicMax(&sm_hll[reg], rank);
+    // registers only grow: after a few rows nearly every row reads a register
+    // at or above its rank and skips the atomic
+    if (rank > sm_hll[reg]) atomicMax(const_cast<uint32_t*>(&sm_hll[reg]), rank);
 }
 
+// The scalar fields of the threads' accumulators reduced over the workgroup
+// (one barrier for all of them); every thread gets the result.
+__device__ __forceinline__ StatsAcc block_fold(StatsAcc a, StatsAcc* sm /* kBlock / kWave */) {
+    a.mn = wave_min(a.mn);
+    a.mx = wave_max(a.mx);
+    a.zf = wave_min(a.zf);
+    a.unsorted = __ballot(a.unsorted != 0) != 0;
+    a.rl_eq = wave_sum(a.rl_eq);
+    a.runs = wave_sum(a.runs);
+    a.sum_bits = wave_sum(a.sum_bits);
+    a.sum_f = wave_sum(a.sum_f);
+    a.prec = wave_max(a.prec);
+    a.dmax = wave_max(a.dmax);
+    if ((threadIdx.x & (kWave - 1)) == 0) sm[threadIdx.x / kWave] = a;
+    __syncthreads();
+    StatsAcc r{~0ull, 0, ~0ull, 0, 0, 0, 0, 0.0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < kBlock / kWave; w++) {
+        const StatsAcc q = sm[w];
+        r.mn = q.mn < r.mn ? q.mn : r.mn;
+        r.mx = q.mx > r.mx ? q.mx : r.mx;
+        r.zf = q.zf < r.zf ? q.zf : r.zf;
+        r.unsorted |= q.unsorted;
+        r.rl_eq += q.rl_eq;
+        r.runs += q.runs;
+        r.sum_bits += q.sum_bits;
+        r.sum_f += q.sum_f;
+        r.prec = q.prec > r.prec ? q.prec : r.prec;
+        r.dmax = q.dmax > r.dmax ? q.dmax : r.dmax;
+    }
+    __syncthreads();  // sm may be rewritten
+    return r;
+}
+
+// Bound by latency on the planner's blocks of 10^4..10^5 rows.  The last
+// workgroup folds the others' 129 histogram and HyperLogLog words with all
+// its threads, consecutive lanes on consecutive words and kFold loads in
+// flight each (one thread per workgroup, walking that workgroup's 129 words
+// one atomic load at a time, took 112 us on 65,537 int32 rows, now 13, and
+// 34 us on 10,000 rows, now 10).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_stats(const T* __restrict__ x, size_t n, DevStats* __restrict__ partials,
                                                   uint32_t* counter, DevStats* out) {
-    __shared__ uint64_t sm[kBlock / kWave];
-    __shared__ double smd[kBlock / kWave];
-    __shared__ uint32_t sm_hist[65];
-    __shared__ uint32_t sm_hll[64];
-    __shared__ uint32_t fin_hist[65];
-    __shared__ uint32_t fin_hll[64];
+    constexpr int kBins = 65, kRegs = 64;
+    __shared__ StatsAcc sm[kBlock / kWave];
+    __shared__ uint32_t sm_hist[kBins * kHistCopies];
+    __shared__ uint32_t sm_hll[kRegs];
+    __shared__ uint32_t fin[kBins + kRegs];  // the folded bins, then the registers
     __shared__ bool last;
-    for (int i = threadIdx.x; i < 65; i += kBlock) sm_hist[i] = 0;
-    for (int i = threadIdx.x; i < 64; i += kBlock) sm_hll[i] = 0;
+    for (int i = threadIdx.x; i < kBins * kHistCopies; i += kBlock) sm_hist[i] = 0;
+    for (int i = threadIdx.x; i < kRegs; i += kBlock) sm_hll[i] = 0;
+    for (int i = threadIdx.x; i < kBins + kRegs; i += kBlock) fin[i] = 0;
     __syncthreads();
     StatsAcc a{~0ull, 0, ~0ull, 0, 0, 0, 0, 0.0, 0, 0};
     const size_t tid = (size_t)blockIdx.x * kBlock + threadIdx.x, stride = (size_t)gridDim.x * kBlock;
@@ -456,33 +493,32 @@ __global__ __launch_bounds__(kBlock) void k_stats(const T* __restrict__ x, size_
         T nx = (i + 1 < n) ? x[i + 1] : T(0);
         stats_elem(a, v, nx, i + 1 < n, i + 2 < n, i, sm_hist, sm_hll);
     }
-    uint64_t mn = block_reduce_min(a.mn, sm);
-    uint64_t mx = block_reduce_max(a.mx, sm);
-    uint64_t zf = block_reduce_min(a.zf, sm);
-    uint64_t uns = block_reduce_max(a.unsorted, sm);
-    uint64_t rl = block_reduce_sum<uint64_t>(a.rl_eq, sm);
-    uint64_t runs = block_reduce_sum<uint64_t>(a.runs, sm);
-    uint64_t sb = block_reduce_sum<uint64_t>(a.sum_bits, sm);
-    double sf = block_reduce_sum<double>(a.sum_f, smd);
-    uint64_t pr = block_reduce_max((uint64_t)a.prec, sm);
-    uint64_t dm = block_reduce_max((uint64_t)a.dmax, sm);
+    a = block_fold(a, sm);  // its barriers also complete sm_hist and sm_hll
     DevStats* p = partials + blockIdx.x;
+    static_assert(offsetof(DevStats, hll) == offsetof(DevStats, bit_hist) + 4 * kBins, "bins and registers adjoin");
     if (threadIdx.x == 0) {
-        st_agent(&p->min_key, mn);
-        st_agent(&p->max_key, mx);
-        st_agent(&p->first_zero, zf);
-        st_agent(&p->unsorted, uns);
-        st_agent(&p->rl_eq, rl);
-        st_agent(&p->runs, runs);
-        st_agent(&p->sum_bits, sb);
+        st_agent(&p->min_key, a.mn);
+        st_agent(&p->max_key, a.mx);
+        st_agent(&p->first_zero, a.zf);
+        st_agent(&p->unsorted, a.unsorted);
+        st_agent(&p->rl_eq, a.rl_eq);
+        st_agent(&p->runs, a.runs);
+        st_agent(&p->sum_bits, a.sum_bits);
         uint64_t sfb;
-        __builtin_memcpy(&sfb, &sf, 8);
+        __builtin_memcpy(&sfb, &a.sum_f, 8);
         st_agent(reinterpret_cast<uint64_t*>(&p->sum_f), sfb);
-        st_agent(&p->precision, (uint32_t)pr);
-        st_agent(&p->delta_bits_max, (uint32_t)dm);
+        st_agent(&p->precision, a.prec);
+        st_agent(&p->delta_bits_max, a.dmax);
     }
-    for (int i = threadIdx.x; i < 65; i += kBlock) st_agent(&p->bit_hist[i], sm_hist[i]);
-    for (int i = threadIdx.x; i < 64; i += kBlock) st_agent(&p->hll[i], sm_hll[i]);
+    for (int i = threadIdx.x; i < kBins + kRegs; i += kBlock) {
+        uint32_t v = 0;
+        if (i < kBins) {  // rotated, so that the lanes' reads spread over the banks
+            for (int k = 0; k < kHistCopies; k++) v += sm_hist[i * kHistCopies + ((i + k) & (kHistCopies - 1))];
+        } else {
+            v = sm_hll[i - kBins];
+        }
+        st_agent(&p->bit_hist[0] + i, v);
+    }
     if (!last_block_arrives(counter, &last)) return;
     StatsAcc f{~0ull, 0, ~0ull, 0, 0, 0, 0, 0.0, 0, 0};
     for (uint32_t b = threadIdx.x; b < gridDim.x; b += kBlock) {
@@ -504,39 +540,40 @@ __global__ __launch_bounds__(kBlock) void k_stats(const T* __restrict__ x, size_
         f.prec = pp > f.prec ? pp : f.prec;
         f.dmax = dd > f.dmax ? dd : f.dmax;
     }
-    mn = block_reduce_min(f.mn, sm);
-    mx = block_reduce_max(f.mx, sm);
-    zf = block_reduce_min(f.zf, sm);
-    uns = block_reduce_max(f.unsorted, sm);
-    rl = block_reduce_sum<uint64_t>(f.rl_eq, sm);
-    runs = block_reduce_sum<uint64_t>(f.runs, sm);
-    sb = block_reduce_sum<uint64_t>(f.sum_bits, sm);
-    sf = block_reduce_sum<double>(f.sum_f, smd);
-    pr = block_reduce_max((uint64_t)f.prec, sm);
-    dm = block_reduce_max((uint64_t)f.dmax, sm);
-    for (int i = threadIdx.x; i < 65; i += kBlock) fin_hist[i] = 0;
-    for (int i = threadIdx.x; i < 64; i += kBlock) fin_hll[i] = 0;
-    __syncthreads();
-    for (uint32_t b = threadIdx.x; b < gridDim.x; b += kBlock) {
-        const DevStats* q = partials + b;
-        for (int e = 0; e < 65; e++) atomicAdd(&fin_hist[e], rd32(&q->bit_hist[e]));
-        for (int e = 0; e < 64; e++) atomicMax(&fin_hll[e], rd32(&q->hll[e]));
+    constexpr int kFold = 8;
+    const uint32_t words = gridDim.x * (kBins + kRegs);
+    for (uint32_t i0 = threadIdx.x; i0 < words; i0 += kFold * kBlock) {
+        uint32_t v[kFold];
+#pragma unroll
+        for (int u = 0; u < kFold; u++) {
+            const uint32_t i = i0 + u * kBlock, b = i / (kBins + kRegs), e = i - b * (kBins + kRegs);
+            v[u] = i < words ? rd32(&partials[b].bit_hist[0] + e) : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < kFold; u++) {
+            const uint32_t i = i0 + u * kBlock, e = i % (kBins + kRegs);
+            if (i >= words) break;
+            if (e < (uint32_t)kBins)
+                atomicAdd(&fin[e], v[u]);
+            else
+                atomicMax(&fin[e], v[u]);
+        }
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < 65; i += kBlock) out->bit_hist[i] = fin_hist[i];
-    for (int i = threadIdx.x; i < 64; i += kBlock) out->hll[i] = fin_hll[i];
+    f = block_fold(f, sm);  // its barriers also complete fin
+    for (int i = threadIdx.x; i < kBins; i += kBlock) out->bit_hist[i] = fin[i];
+    for (int i = threadIdx.x; i < kRegs; i += kBlock) out->hll[i] = fin[kBins + i];
     if (threadIdx.x == 0) {
-        fold_fixup(x, mn, mx, zf);
-        out->min_key = mn;
-        out->max_key = mx;
-        out->first_zero = zf;
-        out->unsorted = uns;
-        out->rl_eq = rl;
-        out->runs = runs + (n > 0 ? 1 : 0);
-        out->sum_bits = sb;
-        out->sum_f = sf;
-        out->precision = (uint32_t)pr;
-        out->delta_bits_max = (uint32_t)dm;
+        fold_fixup(x, f.mn, f.mx, f.zf);
+        out->min_key = f.mn;
+        out->max_key = f.mx;
+        out->first_zero = f.zf;
+        out->unsorted = f.unsorted;
+        out->rl_eq = f.rl_eq;
+        out->runs = f.runs + (n > 0 ? 1 : 0);
+        out->sum_bits = f.sum_bits;
+        out->sum_f = f.sum_f;
+        out->precision = f.prec;
+        out->delta_bits_max = f.dmax;
         __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }

@@ -1,0 +1,63 @@
+"""Kernels at the sizes where their work splits can go wrong (edges of tiles,
+of workgroups and of the ranges a dispatch rule covers), against NumPy or the
+oracle.  Every comparison is exact."""
+import math
+
+import numpy as np
+import pytest
+
+import gputimeseriescompressionoptimizer_amd as g
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+INT_TYPES = [g.D_CHAR, g.D_SHORT, g.D_INT, g.D_TIME]
+
+
+def _mix64(z):
+    z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+    z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+    return z ^ (z >> np.uint64(31))
+
+
+def _bit_lengths(u):
+    return np.array([int(v).bit_length() for v in u])
+
+
+def _distinct_estimate(x):
+    """The 64-register HyperLogLog estimate of the statistics pass."""
+    u = np.unique(x)
+    u = u.view(f"u{u.itemsize}").astype(np.uint64)
+    with np.errstate(over="ignore"):
+        h = _mix64(u + np.uint64(0x9E3779B97F4A7C15))
+    reg = (h >> np.uint64(58)).astype(np.int64)
+    rank = 64 - _bit_lengths((h << np.uint64(6)) | np.uint64(1 << 5)) + 1
+    regs = np.zeros(64, np.int64)
+    np.maximum.at(regs, reg, rank)
+    est = 0.709 * 64 * 64 / sum(math.ldexp(1.0, -int(r)) for r in regs)
+    zeros = int((regs == 0).sum())
+    if est <= 160 and zeros:
+        est = 64.0 * math.log(64.0 / zeros)
+    return min(est, float(x.size))
+
+
+# one workgroup takes 4096 bytes x 4 of rows; 256 and 512 workgroups are the
+# fold's own thread count and the largest grid
+@pytest.mark.parametrize("dtype", INT_TYPES)
+@pytest.mark.parametrize("n", [1, 2, 255, 4096, 4097, 65_537, 2_200_003])
+def test_stats_features(ctx, dtype, n):
+    npdt = g.NP_DTYPE[dtype]
+    r = np.random.default_rng(n)
+    info = np.iinfo(npdt)
+    x = r.integers(info.min, info.max, n, dtype=npdt, endpoint=True) >> r.integers(0, 8 * npdt().itemsize, n).astype(npdt)
+    x[n // 3: n // 2] = 7  # a run: one width, one register
+    s = ctx.stats(ctx.upload(x), dtype)
+    w = x.astype(np.int64)
+    zig = ((w << 1) ^ (w >> 63)).view(np.uint64)
+    width = lambda u: np.where(u == 0, 0, np.floor(np.log2(np.maximum(u, 1).astype(np.longdouble))).astype(np.int64) + 1)
+    assert list(s.bit_hist) == list(np.bincount(width(zig), minlength=65))
+    with np.errstate(over="ignore"):
+        d = (x[1:] - x[:-1]).astype(np.int64) if n > 1 else np.zeros(1, np.int64)  # wraps in the type
+    assert s.delta_bits_max == (int(width(((d << 1) ^ (d >> 63)).view(np.uint64)).max()) if n > 1 else 0)
+    assert s.runs == 1 + int(np.count_nonzero(x[1:] != x[:-1]))
+    assert abs(s.distinct_est - _distinct_estimate(x)) <= 0.5 + 1e-9 * s.distinct_est  # rounded to a whole number
