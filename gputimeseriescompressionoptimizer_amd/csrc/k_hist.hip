@@ -59,28 +59,31 @@ template <typename T> __device__ __forceinline__ uint64_t hist_key(T v, bool& ne
     return ubits(v);
 }
 
-__device__ bool global_insert(unsigned long long* keys, unsigned long long* counts, uint64_t cap_mask, uint64_t key,
-                              unsigned long long cnt, HistCtl* ctl) {
+// Adds cnt rows of `key` to the global table; returns 1 when the key is new
+// (the caller sums these: a counter bumped once per new key serializes every
+// workgroup on one address, which for a column of 10^4 distinct rows was most
+// of the count's time).
+__device__ uint32_t global_insert(unsigned long long* keys, unsigned long long* counts, uint64_t cap_mask, uint64_t key,
+                                  unsigned long long cnt, HistCtl* ctl) {
     uint64_t h = hmix(key) & cap_mask;
     for (uint64_t p = 0; p <= cap_mask && p < 4096; p++) {
         const uint64_t s = (h + p) & cap_mask;
         unsigned long long k = __hip_atomic_load(&keys[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (k == key) {
             atomicAdd(&counts[s], cnt);
-            return true;
+            return 0;
         }
         if (k == kEmpty) {
             unsigned long long prev = atomicCAS(&keys[s], kEmpty, (unsigned long long)key);
             if (prev == kEmpty || prev == key) {
                 atomicAdd(&counts[s], cnt);
-                if (prev == kEmpty) atomicAdd(&ctl->distinct, 1ull);
-                return true;
+                return prev == kEmpty ? 1u : 0u;
             }
         }
     }
     atomicOr(&ctl->overflow, 1u);
     atomicAdd(&ctl->dropped, cnt);
-    return false;
+    return 0;
 }
 
 // Ascending list of the (up to) four smallest keys seen, with multiplicity.
@@ -167,12 +170,15 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
     __shared__ uint32_t scnt[kLdsSlots];
     __shared__ uint64_t s_nk[kHistThreads / kWave * kMaxK];
     __shared__ int s_nc[kHistThreads / kWave];
+    __shared__ uint32_t s_new;  // keys this workgroup brought into the global table
+    uint32_t fresh = 0;
     Small4 nan4;
     unsigned long long nans = 0;
     for (int i = threadIdx.x; i < kLdsSlots; i += kHistThreads) {
         skey[i] = kEmpty;
         scnt[i] = 0;
     }
+    if (threadIdx.x == 0) s_new = 0;
     __syncthreads();
     bool negzero = false;
     unsigned long long special = 0;
@@ -189,7 +195,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
                 return;
             }
         }
-        global_insert(keys, counts, cap_mask, key, (unsigned long long)add, ctl);
+        fresh += global_insert(keys, counts, cap_mask, key, (unsigned long long)add, ctl);
     };
     // Two keys per thread counted in registers (the first two distinct keys
     // the thread meets): on skewed columns most rows hit them and skip the
@@ -251,7 +257,11 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
     if (rk1 != kEmpty) lds_add(rk1, rc1);
     __syncthreads();
     for (int s = threadIdx.x; s < kLdsSlots; s += kHistThreads)
-        if (skey[s] != kEmpty) global_insert(keys, counts, cap_mask, skey[s], scnt[s], ctl);
+        if (skey[s] != kEmpty) fresh += global_insert(keys, counts, cap_mask, skey[s], scnt[s], ctl);
+    fresh = wave_sum(fresh);
+    if ((threadIdx.x & (kWave - 1)) == 0 && fresh) atomicAdd(&s_new, fresh);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_new) atomicAdd(&ctl->distinct, (unsigned long long)s_new);
     const uint64_t nz = wave_or((uint64_t)negzero);
     const unsigned long long sp = wave_sum(special);
     const unsigned long long nn = wave_sum(nans);
@@ -296,32 +306,49 @@ template <typename T> __device__ __forceinline__ void push(Cand* top, int K, Can
         if (i == pos) top[i] = c;
 }
 
-// a = the best K of the sorted lists a and b (empty entries have count 0).
-template <typename T> __device__ __forceinline__ void merge_lists(Cand* a, const Cand* b, int K) {
-    Cand o[kMaxK];
-    int i = 0, j = 0;
+// The best K candidates of a wave whose lanes hold sorted lists of K: K
+// rounds, each taking the largest head (by count; the heads that tie by the
+// smaller order key) off its lane's list.  Lane 0 writes round r's to out[r]
+// (count 0 when the lists are empty).  One wave maximum and one ballot a
+// round: a pairwise merge of the lists through LDS, with its lists indexed by
+// data, took 13-18 us a launch, this 5.
+template <typename T> __device__ __forceinline__ void wave_best(Cand* top, int K, Cand* out) {
+    const int lane = threadIdx.x & (kWave - 1);
+    for (int r = 0; r < K; r++) {  // uniform
+        const unsigned long long m = wave_max(top[0].count);
+        uint64_t who = __ballot(top[0].count == m);
+        if (m != 0 && (who & (who - 1)) != 0) {  // a tie (uniform)
+            T v;
+            using U = typename UnsignedOf<T>::type;
+            const U u = (U)top[0].key;
+            __builtin_memcpy(&v, &u, sizeof(T));
+            const bool mine = top[0].count == m;
+            const uint64_t ok = mine ? order_key(v) : ~0ull;
+            const uint64_t k = wave_min(ok);
+            who = __ballot(mine && ok == k);
+        }
+        if (lane == __builtin_ctzll(who)) {
+            out[r] = m ? top[0] : Cand{0, 0};
 #pragma unroll
-    for (int k = 0; k < kMaxK; k++) {
-        if (k >= K) break;
-        const bool ta = i < K && a[i].count != 0, tb = j < K && b[j].count != 0;
-        if (ta && (!tb || better<T>(a[i], b[j])))
-            o[k] = a[i++];
-        else if (tb)
-            o[k] = b[j++];
-        else
-            o[k] = Cand{0, 0};
+            for (int i = 0; i + 1 < kMaxK; i++) top[i] = top[i + 1];
+            top[kMaxK - 1] = Cand{0, 0};
+        }
     }
-#pragma unroll
-    for (int k = 0; k < kMaxK; k++)
-        if (k < K) a[k] = o[k];
 }
 
-// Pairwise tree merge of nl sorted lists of K in LDS into list 0.
-template <typename T> __device__ void block_merge(Cand* sc, int nl, int K) {
-    for (int s = 1; s < nl; s <<= 1) {
-        __syncthreads();
+// The best K of the workgroup's sorted lists into out[0..K), by wave 0 (sc:
+// LDS for K candidates per wave); the other waves only contribute.
+template <typename T> __device__ void block_best(Cand* top, int K, Cand* sc, Cand* out) {
+    const int wid = threadIdx.x / kWave;
+    wave_best<T>(top, K, sc + wid * kMaxK);
+    __syncthreads();
+    if (wid == 0) {
+        Cand one[kMaxK];
+#pragma unroll
+        for (int i = 0; i < kMaxK; i++) one[i] = Cand{0, 0};
         const int t = threadIdx.x;
-        if (t < nl && t % (2 * s) == 0 && t + s < nl) merge_lists<T>(sc + t * K, sc + (t + s) * K, K);
+        if (t < kBlock / kWave * kMaxK && (t & (kMaxK - 1)) < K) one[0] = sc[t];
+        wave_best<T>(one, K, out);
     }
     __syncthreads();
 }
@@ -331,36 +358,38 @@ __global__ __launch_bounds__(kBlock) void k_hist_topk(const unsigned long long* 
                                                       uint64_t cap, int K, Cand* partials, uint32_t* counter,
                                                       const HistCtl* ctl, const uint64_t* nan_keys,
                                                       const uint32_t* nan_n, uint32_t nan_blocks, Cand* out) {
-    __shared__ Cand sc[kBlock * kMaxK];
+    __shared__ Cand sc[kBlock / kWave * kMaxK];
+    __shared__ Cand best[kMaxK];
     __shared__ bool last;
     Cand top[kMaxK];
+#pragma unroll
     for (int i = 0; i < kMaxK; i++) top[i] = Cand{0, 0};
     const size_t stride = (size_t)gridDim.x * kBlock;
     for (size_t s = (size_t)blockIdx.x * kBlock + threadIdx.x; s < cap; s += stride) {
         const uint64_t k = keys[s];
         if (k != kEmpty) push<T>(top, K, Cand{counts[s], k});
     }
-#pragma unroll
-    for (int i = 0; i < kMaxK; i++)
-        if (i < K) sc[threadIdx.x * K + i] = top[i];
-    block_merge<T>(sc, kBlock, K);
-    if (threadIdx.x == 0)
-        for (int i = 0; i < K; i++) {
-            st_agent(reinterpret_cast<uint64_t*>(&partials[blockIdx.x * K + i].count), (uint64_t)sc[i].count);
-            st_agent(&partials[blockIdx.x * K + i].key, sc[i].key);
-        }
+    block_best<T>(top, K, sc, best);
+    if (threadIdx.x < K) {
+        st_agent(reinterpret_cast<uint64_t*>(&partials[blockIdx.x * K + threadIdx.x].count),
+                 (uint64_t)best[threadIdx.x].count);
+        st_agent(&partials[blockIdx.x * K + threadIdx.x].key, best[threadIdx.x].key);
+    }
     if (!last_block_arrives(counter, &last)) return;
-    // the last workgroup gathers every workgroup's list into LDS and merges
+    // the last workgroup takes the best of every workgroup's list
+#pragma unroll
+    for (int i = 0; i < kMaxK; i++) top[i] = Cand{0, 0};
     for (uint32_t i = threadIdx.x; i < gridDim.x * (uint32_t)K; i += kBlock) {
         Cand c;
         c.count = __hip_atomic_load(&partials[i].count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         c.key = __hip_atomic_load(&partials[i].key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        sc[i] = c;
+        push<T>(top, K, c);
     }
-    block_merge<T>(sc, (int)gridDim.x, K);
+    block_best<T>(top, K, sc, best);
     if (threadIdx.x != 0) return;
     Cand b[kMaxK];
-    for (int i = 0; i < kMaxK; i++) b[i] = i < K ? sc[i] : Cand{0, 0};
+#pragma unroll
+    for (int i = 0; i < kMaxK; i++) b[i] = i < K ? best[i] : Cand{0, 0};
     if (ctl->special) push<T>(b, K, Cand{ctl->special, kEmpty});
     if constexpr (std::is_floating_point<T>::value) {
         if (ctl->nans)  // every NaN row is a bin of count 1

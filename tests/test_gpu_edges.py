@@ -61,3 +61,32 @@ def test_stats_features(ctx, dtype, n):
     assert s.delta_bits_max == (int(width(((d << 1) ^ (d >> 63)).view(np.uint64)).max()) if n > 1 else 0)
     assert s.runs == 1 + int(np.count_nonzero(x[1:] != x[:-1]))
     assert abs(s.distinct_est - _distinct_estimate(x)) <= 0.5 + 1e-9 * s.distinct_est  # rounded to a whole number
+
+
+def _top(x, k):
+    """The k most frequent values, equal counts by the smaller value."""
+    v, c = np.unique(x, return_counts=True)
+    return [int(v[i]) for i in np.lexsort((v, -c))[:k]]
+
+
+# 2048 LDS slots a workgroup, 16384 rows a workgroup, 64K slots in the first
+# global table (70% of it full makes the count run again)
+@pytest.mark.parametrize("distinct", [1, 3, 4, 63, 2_047, 2_048, 2_049, 45_875, 45_876, 70_000, 300_000])
+@pytest.mark.parametrize("dtype", [g.D_INT, g.D_TIME])
+def test_most_frequent(ctx, dtype, distinct):
+    npdt = g.NP_DTYPE[dtype]
+    r = np.random.default_rng(distinct)
+    values = r.permutation(np.arange(-(distinct // 2), distinct - distinct // 2, dtype=np.int64) * 1_000_003 + 7)
+    x = np.concatenate([values, values[r.integers(0, min(distinct, 40), 20_011)]]).astype(npdt)
+    r.shuffle(x)
+    meta = g.Encoding(ctx, g.DICT).Encode(ctx.upload(x), dtype)[1].to_bytes()
+    want = O.encode(g.DICT, dtype, x)
+    assert meta == want[1]
+    found = np.frombuffer(meta[16:16 + npdt().itemsize * min(distinct, 4)], npdt)
+    assert sorted(int(v) for v in found) == sorted(_top(x, 4))
+
+
+def test_most_frequent_all_counts_tie(ctx):
+    x = np.random.default_rng(1).permutation(np.arange(-50_000, 50_000, dtype=np.int32))
+    meta = g.Encoding(ctx, g.DICT).Encode(ctx.upload(x), g.D_INT)[1].to_bytes()
+    assert sorted(np.frombuffer(meta[16:32], np.int32)) == [-50_000, -49_999, -49_998, -49_997]
