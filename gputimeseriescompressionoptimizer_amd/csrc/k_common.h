@@ -73,33 +73,6 @@ template <typename T> __device__ __host__ __forceinline__ T from_order_key(uint6
 }
 
 // ---------------------------------------------------------- wave reductions
-template <typename T> __device__ __forceinline__ T wave_sum(T v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-    return v;
-}
-template <typename T> __device__ __forceinline__ T wave_min(T v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-        T w = __shfl_xor(v, o, kWave);
-        v = w < v ? w : v;
-    }
-    return v;
-}
-template <typename T> __device__ __forceinline__ T wave_max(T v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-        T w = __shfl_xor(v, o, kWave);
-        v = w > v ? w : v;
-    }
-    return v;
-}
-__device__ __forceinline__ uint64_t wave_or(uint64_t v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v |= __shfl_xor(v, o, kWave);
-    return v;
-}
-
 // Minimum (MAX: maximum) of a 32-bit value over the 64 lanes of a wave:
 // DPP steps inside every row of 16 lanes (swap neighbours, swap pairs, mirror
 // half-rows, mirror rows), then the four rows' results by readlane.  The
@@ -113,6 +86,17 @@ template <bool MAX> __device__ __forceinline__ int32_t wave_extreme_i32(int32_t 
     const int32_t r0 = __builtin_amdgcn_readlane(v, 0), r1 = __builtin_amdgcn_readlane(v, 16);
     const int32_t r2 = __builtin_amdgcn_readlane(v, 32), r3 = __builtin_amdgcn_readlane(v, 48);
     return op(op(r0, r1), op(r2, r3));
+}
+
+// The same for 64-bit unsigned values: the high halves first, then the low
+// halves of the lanes that hold the extreme one.
+template <bool MAX> __device__ __forceinline__ uint64_t wave_extreme_u64(uint64_t v) {
+    constexpr uint32_t kFlip = 0x80000000u;  // unsigned order as signed order
+    const uint32_t hi = (uint32_t)(v >> 32);
+    const uint32_t mh = (uint32_t)wave_extreme_i32<MAX>((int32_t)(hi ^ kFlip)) ^ kFlip;
+    const uint32_t lo = hi == mh ? (uint32_t)v : (MAX ? 0u : ~0u);
+    const uint32_t ml = (uint32_t)wave_extreme_i32<MAX>((int32_t)(lo ^ kFlip)) ^ kFlip;
+    return ((uint64_t)mh << 32) | ml;
 }
 
 // v shifted across lanes by a DPP control (lanes the control or the row /
@@ -144,6 +128,42 @@ template <typename T> __device__ __forceinline__ T wave_inclusive_scan(T v) {
     x += dpp_shift<0x142, 0xA, 0xF>(x);       // row_bcast:15, rows 1 and 3
     x += dpp_shift<0x143, 0xC, 0xF>(x);       // row_bcast:31, rows 2 and 3
     return x;
+}
+
+// Reductions over the 64 lanes of a wave (the result in every lane), by DPP:
+// a chain of six ds_bpermute shuffles waits on LDS at every step.
+template <bool MAX, typename T> __device__ __forceinline__ T wave_extreme(T v) {
+    static_assert(std::is_integral<T>::value && sizeof(T) <= 8, "integers");
+    if constexpr (sizeof(T) == 8) {
+        constexpr uint64_t kSign = std::is_signed<T>::value ? 1ull << 63 : 0ull;
+        return (T)(wave_extreme_u64<MAX>((uint64_t)v ^ kSign) ^ kSign);
+    } else {
+        constexpr uint32_t kSign = std::is_signed<T>::value ? 0u : 1u << 31;
+        return (T)((uint32_t)wave_extreme_i32<MAX>((int32_t)((uint32_t)v ^ kSign)) ^ kSign);
+    }
+}
+template <typename T> __device__ __forceinline__ T wave_min(T v) { return wave_extreme<false>(v); }
+template <typename T> __device__ __forceinline__ T wave_max(T v) { return wave_extreme<true>(v); }
+template <typename T> __device__ __forceinline__ T wave_sum(T v) {
+    if constexpr (std::is_integral<T>::value) {
+        const T s = wave_inclusive_scan(v);  // lane 63 holds the sum
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(uint64_t)s, kWave - 1);
+        if constexpr (sizeof(T) == 8) {
+            const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)s >> 32), kWave - 1);
+            return (T)(((uint64_t)hi << 32) | lo);
+        } else {
+            return (T)lo;
+        }
+    } else {
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+        return v;
+    }
+}
+__device__ __forceinline__ uint64_t wave_or(uint64_t v) {
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) v |= __shfl_xor(v, o, kWave);
+    return v;
 }
 
 // Block-wide exclusive scan of one value per thread (NT threads).
