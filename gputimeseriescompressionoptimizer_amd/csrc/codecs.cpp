@@ -79,17 +79,7 @@ template <typename T> uint64_t tbits(T v) {
     return (uint64_t)u;
 }
 
-struct MinMax {
-    DevBuf buf;
-    MinMaxResult host;
-};
-MinMax minmax(Ctx* c, int dtype, const void* x, size_t n) {
-    if (dtype != DDJ_D_FLOAT && dtype != DDJ_D_DOUBLE) return MinMax{DevBuf(), minmax_to_host(c, dtype, x, n, false)};
-    MinMax m{DevBuf(c, sizeof(MinMaxResult)), {}};
-    launch_minmax(c, dtype, x, n, m.buf.get<MinMaxResult>());
-    d2h(c, &m.host, m.buf.get(), sizeof(MinMaxResult));
-    return m;
-}
+MinMaxResult minmax(Ctx* c, int dtype, const void* x, size_t n) { return minmax_to_host(c, dtype, x, n, false); }
 
 // ------------------------------------------------------------------- none
 // NoneEncoding (reference compression/none/none_encoding.cu:13-49)
@@ -145,11 +135,11 @@ std::vector<Part> scale_encode(Ctx* c, int dtype, DView in) {
     const size_t es = dtype_size(dtype), n = rows(dtype, in.n);
     if (n == 0) return {empty(), empty()};
     Part x = aligned_view(c, in, es);
-    MinMax mm = minmax(c, iv, x.p, n);
+    const MinMaxResult mm = minmax(c, iv, x.p, n);
     return dispatch_int((int)es, [&](auto tag) -> std::vector<Part> {
         using T = decltype(tag);
         T mn, mx;
-        decode_minmax(iv, mm.host, &mn, &mx);
+        decode_minmax(iv, mm, &mn, &mx);
         T m = scale_min(mn, mx);
         DevBuf data(c, n * es);
         launch_sub_scalar(c, (int)es, x.p, n, tbits(m), data.get());
@@ -217,14 +207,15 @@ std::vector<Part> afl_encode_int(Ctx* c, int dtype, DView in, const MinMaxResult
     DevBuf mmb;
     const MinMaxResult* mm = known;
     MinMaxResult h;
-    if (!mm && defer) {  // the width only, folded on the host
-        h = minmax_to_host(c, dtype, x.p, n, false);
+    HostOut pending;
+    if (!mm) {
+        if (!defer) mmb = DevBuf(c, sizeof(MinMaxResult));  // the pack reads the width there
+        pending = launch_minmax(c, dtype, x.p, n, false, mmb.get<MinMaxResult>());
         kernel_bytes(c, "k_minmax", (double)(n * es));
-    } else if (!mm) {
-        mmb = DevBuf(c, sizeof(MinMaxResult));
-        launch_minmax(c, dtype, x.p, n, mmb.get<MinMaxResult>());
-        kernel_bytes(c, "k_minmax", (double)(n * es));
-        mm = mmb.get<MinMaxResult>();
+        if (defer)
+            h = wait_minmax(c, pending);
+        else
+            mm = mmb.get<MinMaxResult>();
     }
     const uint64_t W = 8 * es;
     Part data;
@@ -240,7 +231,10 @@ std::vector<Part> afl_encode_int(Ctx* c, int dtype, DView in, const MinMaxResult
     } else {
         DevBuf buf(c, (size_t)((W * n + W - 1) / W) * es);  // worst case b = W
         launch_fl_pack(c, dtype, x.p, n, mm, 0, buf.get());
-        d2h(c, &h, mm, sizeof h);
+        if (pending.dst)
+            h = wait_minmax(c, pending);  // the pack is not waited for
+        else
+            d2h(c, &h, mm, sizeof h);
         buf.set_size((size_t)fl_bytes(es, bits_of(dtype, h), n));
         kernel_bytes(c, "k_fl_pack", (double)(n * es + buf.size()));
         data = own(std::move(buf));
@@ -277,9 +271,9 @@ std::vector<Part> afl_encode_float(Ctx* c, DView in) {
     const size_t n = rows(DDJ_D_FLOAT, in.n);
     if (n == 0) return {empty(), empty()};
     Part x = aligned_view(c, in, 4);
-    MinMax mm = minmax(c, DDJ_D_FLOAT, x.p, n);
+    const MinMaxResult mm = minmax(c, DDJ_D_FLOAT, x.p, n);
     float mn, mx;
-    decode_minmax(DDJ_D_FLOAT, mm.host, &mn, &mx);
+    decode_minmax(DDJ_D_FLOAT, mm, &mn, &mx);
     const char sign = (char)((mn >= 0 ? 1 : 0) + (mx < 0 ? 2 : 0));
     DevBuf mant(c, 4 * n), expo(c, 4 * n), sgn(c, 4 * n);
     launch_float_split(c, reinterpret_cast<const float*>(x.p), n, mant.get<int32_t>(), expo.get<int32_t>(),
@@ -395,12 +389,12 @@ size_t stencil_rows(Ctx* c, DView st) {
 // (compression/patch/patch_encoding_factory.hpp:40-57, lower_patch_encoding.cu:22-66,
 // outside_patch_encoding.cu:22-60)
 PredArgs patch_pred(Ctx* c, int dtype, const uint8_t* x, size_t n, bool outside) {
-    MinMax mm = minmax(c, dtype, x, n);
+    const MinMaxResult mm = minmax(c, dtype, x, n);
     PredArgs p{};
     dispatch_native(dtype, [&](auto tag) {
         using T = decltype(tag);
         T mnT, mxT;
-        decode_minmax(dtype, mm.host, &mnT, &mxT);
+        decode_minmax(dtype, mm, &mnT, &mxT);
         volatile double mn = (double)mnT, mx = (double)mxT, factor = 0.1;
         const T dist = (T)(mx - mn);
         volatile double prod = factor * (double)dist;
@@ -626,14 +620,11 @@ std::vector<Part> float_encode(Ctx* c, int dtype, DView in) {
     int precision = 0;
     MinMaxResult mmr;
     if (dtype == DDJ_D_FLOAT || dtype == DDJ_D_DOUBLE) {
-        DevBuf s(c, sizeof(FloatScanResult));
-        launch_float_scan(c, dtype, x.p, n, s.get<FloatScanResult>());
-        FloatScanResult h;
-        d2h(c, &h, s.get(), sizeof h);
+        const FloatScanResult h = float_scan(c, dtype, x.p, n);
         precision = (int)h.precision;
         mmr = h.mm;
     } else {
-        mmr = minmax(c, dtype, x.p, n).host;  // float(integer) always has precision 0
+        mmr = minmax(c, dtype, x.p, n);  // float(integer) always has precision 0
     }
     bool transform = false;
     if (precision < 10) {
@@ -903,12 +894,9 @@ std::vector<Part> delta_afl_encode(Ctx* c, int dtype, DView in, bool defer) {
     const size_t m = n - 1;
     DevBuf mmb;
     MinMaxResult h;
-    if (defer) {  // the width only, folded on the host
-        h = minmax_to_host(c, dtype, x.p, n, true);
-    } else {
-        mmb = DevBuf(c, sizeof(MinMaxResult));
-        launch_minmax_delta(c, (int)es, x.p, n, mmb.get<MinMaxResult>());
-    }
+    if (!defer) mmb = DevBuf(c, sizeof(MinMaxResult));  // the pack reads the width there
+    const HostOut pending = launch_minmax(c, dtype, x.p, n, true, mmb.get<MinMaxResult>());
+    if (defer) h = wait_minmax(c, pending);
     kernel_bytes(c, "k_minmax_delta", (double)(n * es));
     const uint64_t W = 8 * es;
     Part data;
@@ -924,7 +912,7 @@ std::vector<Part> delta_afl_encode(Ctx* c, int dtype, DView in, bool defer) {
     } else {
         DevBuf buf(c, (size_t)((W * m + W - 1) / W) * es);  // worst case b = W
         launch_fl_pack_delta(c, (int)es, x.p, m, mmb.get<MinMaxResult>(), buf.get());
-        d2h(c, &h, mmb.get(), sizeof h);
+        h = wait_minmax(c, pending);
         buf.set_size((size_t)fl_bytes(es, bits_of(dtype, h), m));
         kernel_bytes(c, "k_fl_pack", (double)(n * es + buf.size()));
         data = own(std::move(buf));
@@ -1105,10 +1093,7 @@ ddj_stats_t stats(Ctx* c, int dtype, DView in) {
     s.size = n;
     if (n == 0) return s;
     Part x = aligned_view(c, in, es);
-    DevBuf d(c, sizeof(DevStats));
-    launch_stats(c, dtype, x.p, n, d.get<DevStats>());
-    DevStats h;
-    d2h(c, &h, d.get(), sizeof h);
+    const DevStats h = device_stats(c, dtype, x.p, n);
     dispatch_native(dtype, [&](auto tag) {
         using T = decltype(tag);
         MinMaxResult r{h.min_key, h.max_key};

@@ -66,7 +66,25 @@ struct Control {
     uint32_t counters[64];
     uint32_t error_flag;
     uint32_t pad[63];
+    // Tickets of the "last workgroup" reductions of large grids: word 0 the
+    // root, word 32 (1 + g) group g, each on a cache line of its own.
+    uint32_t tickets[32 * 17];
+    // Where a kernel's results go when the runtime gives pinned memory no
+    // device address: kHostOutBytes bytes, then the completion flag.
+    uint8_t host_out[8192 + 64];
 };
+
+// Where the last workgroup of a kernel leaves a small result for the host:
+// the context's pinned landing area through its device address (dst), then
+// `seq` at *flag, which the host polls.  One is outstanding at a time: it is
+// waited for before the next read-back of any kind.
+struct HostOut {
+    uint8_t* dst = nullptr;  // null: no result wanted
+    uint32_t* flag = nullptr;
+    uint32_t seq = 0;
+};
+constexpr size_t kHostOutBytes = 8192;
+static_assert(sizeof(Control::host_out) == kHostOutBytes + 64, "the slot and its flag");
 
 // Per-kernel HIP-event timings, recorded on the context stream around each
 // launch while profiling is enabled.
@@ -205,6 +223,11 @@ struct ReadBack {
 // that writes the landing area directly).  d2h_any is for pointers a
 // caller passed in, which the runtime's copy checks.
 void d2h_many(Ctx* c, const ReadBack* rb, size_t count);
+// A result slot for the next kernel (at most kHostOutBytes), and the wait for
+// it: returns the landed bytes.  Launches made between the two are not waited
+// for.
+HostOut host_out(Ctx* c);
+const uint8_t* wait_host_out(Ctx* c, const HostOut& h);
 void d2h_any(Ctx* c, void* dst, const void* src, size_t bytes);
 void h2d(Ctx* c, void* dst, const void* src, size_t bytes);  // stream-ordered
 // A slot of `bytes` in the staging ring for a small table that kernels read

@@ -211,15 +211,38 @@ __device__ __forceinline__ void st_agent(uint32_t* p, uint32_t v) {
 // makes those stores complete at the device coherence point before the
 // barrier, and only then does thread 0 take a ticket.  The last workgroup
 // reads the partials with relaxed agent-scope loads, which go to that point.
-__device__ __forceinline__ bool last_block_arrives(uint32_t* counter, bool* sm_flag) {
+// Past 64 workgroups the tickets are taken on 16 group counters first (one
+// address would serialize the arrivals: 7 us for 1024, 28 us for 4096), whose
+// last arrivals go on to the root.  The last workgroup leaves every counter at
+// zero.  Kernels of one context run on one stream, so they share the counters.
+__device__ __forceinline__ bool last_of_grid(uint32_t* tickets, bool* sm_flag) {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (threadIdx.x == 0) {
-        const uint32_t prev = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *sm_flag = (prev == gridDim.x - 1);
+        auto arrive = [&](uint32_t* t, uint32_t members) {
+            if (__hip_atomic_fetch_add(t, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != members - 1) return false;
+            st_agent(t, 0u);
+            return true;
+        };
+        const uint32_t grid = gridDim.x, g = blockIdx.x & 15;
+        bool l;
+        if (grid <= 64)
+            l = arrive(tickets, grid);
+        else
+            l = arrive(tickets + 32 * (1 + g), (grid - g + 15) / 16) && arrive(tickets, 16);
+        *sm_flag = l;
     }
     __syncthreads();
     return *sm_flag;
+}
+
+// Completes a HostOut that the calling workgroup's threads have written:
+// every thread releases its stores at system scope (a release alone: the
+// full fence would also invalidate the L2), then thread 0 sets the flag.
+__device__ __forceinline__ void host_out_done(const HostOut& h) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(h.flag, h.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // -------------------------------------------------------------- bit helpers

@@ -238,9 +238,7 @@ __global__ __launch_bounds__(kBlock) void k_to_host(ToHostPieces t, uint8_t* __r
             for (uint32_t i = tid; i < nb; i += kBlock) d[i] = s[i];
         }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-    __syncthreads();
-    if (tid == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    host_out_done(HostOut{dst, flag, seq});
 }
 
 template <typename T>

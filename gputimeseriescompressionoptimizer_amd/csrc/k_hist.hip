@@ -279,6 +279,12 @@ struct Cand {
     uint64_t key;
 };
 
+// What the host gets: the table's state and the best K (the rest empty).
+struct HistResult {
+    HistCtl ctl;
+    Cand top[kMaxK];
+};
+
 template <typename T> __device__ __forceinline__ bool better(const Cand& a, const Cand& b) {
     if (a.count != b.count) return a.count > b.count;
     T va, vb;
@@ -355,9 +361,9 @@ template <typename T> __device__ void block_best(Cand* top, int K, Cand* sc, Can
 
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_hist_topk(const unsigned long long* keys, const unsigned long long* counts,
-                                                      uint64_t cap, int K, Cand* partials, uint32_t* counter,
+                                                      uint64_t cap, int K, Cand* partials, uint32_t* tickets,
                                                       const HistCtl* ctl, const uint64_t* nan_keys,
-                                                      const uint32_t* nan_n, uint32_t nan_blocks, Cand* out) {
+                                                      const uint32_t* nan_n, uint32_t nan_blocks, HostOut host) {
     __shared__ Cand sc[kBlock / kWave * kMaxK];
     __shared__ Cand best[kMaxK];
     __shared__ bool last;
@@ -375,7 +381,7 @@ __global__ __launch_bounds__(kBlock) void k_hist_topk(const unsigned long long* 
                  (uint64_t)best[threadIdx.x].count);
         st_agent(&partials[blockIdx.x * K + threadIdx.x].key, best[threadIdx.x].key);
     }
-    if (!last_block_arrives(counter, &last)) return;
+    if (!last_of_grid(tickets, &last)) return;
     // the last workgroup takes the best of every workgroup's list
 #pragma unroll
     for (int i = 0; i < kMaxK; i++) top[i] = Cand{0, 0};
@@ -386,23 +392,25 @@ __global__ __launch_bounds__(kBlock) void k_hist_topk(const unsigned long long* 
         push<T>(top, K, c);
     }
     block_best<T>(top, K, sc, best);
-    if (threadIdx.x != 0) return;
-    Cand b[kMaxK];
+    if (threadIdx.x == 0) {
+        Cand b[kMaxK];
 #pragma unroll
-    for (int i = 0; i < kMaxK; i++) b[i] = i < K ? best[i] : Cand{0, 0};
-    if (ctl->special) push<T>(b, K, Cand{ctl->special, kEmpty});
-    if constexpr (std::is_floating_point<T>::value) {
-        if (ctl->nans)  // every NaN row is a bin of count 1
-            for (uint32_t g = 0; g < nan_blocks; g++)
-                for (uint32_t r = 0; r < nan_n[g]; r++) {
-                    const T v = from_order_key<T>(nan_keys[(size_t)g * kMaxK + r]);
-                    push<T>(b, K, Cand{1ull, ubits(v)});
-                }
+        for (int i = 0; i < kMaxK; i++) b[i] = i < K ? best[i] : Cand{0, 0};
+        if (ctl->special) push<T>(b, K, Cand{ctl->special, kEmpty});
+        if constexpr (std::is_floating_point<T>::value) {
+            if (ctl->nans)  // every NaN row is a bin of count 1
+                for (uint32_t g = 0; g < nan_blocks; g++)
+                    for (uint32_t r = 0; r < nan_n[g]; r++) {
+                        const T v = from_order_key<T>(nan_keys[(size_t)g * kMaxK + r]);
+                        push<T>(b, K, Cand{1ull, ubits(v)});
+                    }
+        }
+        HistResult* out = reinterpret_cast<HistResult*>(host.dst);
+        out->ctl = *ctl;
+#pragma unroll
+        for (int i = 0; i < kMaxK; i++) out->top[i] = b[i];
     }
-#pragma unroll
-    for (int i = 0; i < kMaxK; i++)
-        if (i < K) out[i] = b[i];
-    __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    host_out_done(host);
 }
 
 // The histogram's global table emptied (keys ~0, counts 0) and its control
@@ -448,19 +456,19 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
                                counts.get<unsigned long long>(), cap - 1, ctl.get<HistCtl>(),
                                nan_keys.get<uint64_t>(), nan_n.get<uint32_t>()); }
             HIPC(hipGetLastError());
-            // the top-K runs before the table's state is read back, so that one
-            // read-back brings both (its result is dropped if the table filled)
+            // the top-K runs before the table's state is known, so that one
+            // result brings both (it is dropped if the table filled)
             const unsigned tg = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((cap + kBlock - 1) / kBlock, 128));
-            DevBuf partials(c, sizeof(Cand) * K * tg), out(c, sizeof(Cand) * K);
+            DevBuf partials(c, sizeof(Cand) * K * tg);
+            const HostOut ho = host_out(c);
             { KernelTimer kt_(c, "k_hist_topk"); hipLaunchKernelGGL(k_hist_topk<T>, dim3(tg), dim3(kBlock), 0, c->stream, keys.get<unsigned long long>(),
-                               counts.get<unsigned long long>(), cap, K, partials.get<Cand>(), &c->control->counters[2],
-                               ctl.get<HistCtl>(), nan_keys.get<uint64_t>(), nan_n.get<uint32_t>(), (uint32_t)g,
-                               out.get<Cand>()); }
+                               counts.get<unsigned long long>(), cap, K, partials.get<Cand>(), c->control->tickets,
+                               ctl.get<HistCtl>(), nan_keys.get<uint64_t>(), nan_n.get<uint32_t>(), (uint32_t)g, ho); }
             HIPC(hipGetLastError());
-            HistCtl h;
-            Cand res[kMaxK];
-            const ReadBack rb[2] = {{&h, ctl.get(), sizeof h}, {res, out.get(), sizeof(Cand) * K}};
-            d2h_many(c, rb, 2);
+            HistResult found;
+            memcpy(&found, wait_host_out(c, ho), sizeof found);
+            const HistCtl& h = found.ctl;
+            const Cand* res = found.top;
             if (h.overflow || h.distinct * 10 > cap * 7) {
                 if (attempt == 2 || cap >= all_distinct) fail(DDJ_ENOMEM, "histogram table overflow");
                 const uint64_t seen = h.distinct + (h.overflow ? h.dropped : 0);

@@ -2,9 +2,10 @@
 // and the fused statistics pass the planner reads.
 //
 // Every workgroup reduces a grid-stride share with 16-byte loads and writes a
-// partial.  Min/max partials are folded by a one-workgroup launch
-// (k_minmax_fold); the statistics pass folds its own in the last workgroup
-// to finish (ticket on a control counter that it resets).
+// partial; the last workgroup to finish (tickets that it resets) folds the
+// partials and hands the result to the host itself where the host asked for
+// it.  A launch of its own for the fold and one for the read-back cost 6 us on
+// the device and 7 us of launching for a few kilobytes.
 #include <algorithm>
 #include <cstddef>
 #include <vector>
@@ -102,10 +103,54 @@ template <typename T> __device__ __forceinline__ void fold_fixup(const T* x, uin
     }
 }
 
+// What the last workgroup of a min/max pass does with the partials (STRIDE
+// keys each: min, max, then the first zero and the precision where kept).
+// No tickets: the partials are left to the host.
+struct FoldTail {
+    uint32_t* tickets = nullptr;
+    MinMaxResult* out = nullptr;  // device result, or null
+    HostOut host;                 // {min key, max key, precision}
+};
+
+template <typename T, int STRIDE>
+__device__ __forceinline__ void fold_partials(const FoldTail& ft, const uint64_t* partials, const T* x, uint64_t* sm,
+                                              bool* flag) {
+    if (!ft.tickets || !last_of_grid(ft.tickets, flag)) return;
+    uint64_t mn = ~0ull, mx = 0, zf = ~0ull, pr = 0;
+    for (uint32_t b = threadIdx.x; b < gridDim.x; b += kBlock) {
+        const uint64_t a = rd(partials + STRIDE * b), z = rd(partials + STRIDE * b + 1);
+        const uint64_t q = STRIDE >= 3 ? rd(partials + STRIDE * b + 2) : ~0ull;
+        const uint64_t p = STRIDE == 4 ? rd(partials + STRIDE * b + 3) : 0ull;
+        mn = a < mn ? a : mn;
+        mx = z > mx ? z : mx;
+        zf = q < zf ? q : zf;
+        pr = p > pr ? p : pr;
+    }
+    mn = block_reduce_min(mn, sm);
+    mx = block_reduce_max(mx, sm);
+    if (STRIDE >= 3 && std::is_floating_point<T>::value) zf = block_reduce_min(zf, sm);
+    if (STRIDE == 4) pr = block_reduce_max(pr, sm);
+    if (threadIdx.x == 0) {
+        if (STRIDE >= 3) fold_fixup(x, mn, mx, zf);
+        if (ft.out) {
+            ft.out->min_key = mn;
+            ft.out->max_key = mx;
+        }
+        if (ft.host.dst) {
+            uint64_t* h = reinterpret_cast<uint64_t*>(ft.host.dst);
+            h[0] = mn;
+            h[1] = mx;
+            h[2] = pr;
+        }
+    }
+    if (ft.host.dst) host_out_done(ft.host);
+}
+
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_minmax(const T* __restrict__ x, size_t n, uint64_t* __restrict__ partials,
-                                                   const uint64_t* d_rows) {
+                                                   const uint64_t* d_rows, FoldTail ft) {
     __shared__ uint64_t sm[kBlock / kWave];
+    __shared__ bool last;
     if (d_rows) n = *d_rows < n ? *d_rows : n;  // rows counted on the device (uniform)
     FoldKeys<T> f;
     const size_t tid = (size_t)blockIdx.x * kBlock + threadIdx.x, stride = (size_t)gridDim.x * kBlock;
@@ -143,14 +188,17 @@ __global__ __launch_bounds__(kBlock) void k_minmax(const T* __restrict__ x, size
         st_agent(partials + 3 * blockIdx.x + 1, mx);
         st_agent(partials + 3 * blockIdx.x + 2, zf);
     }
+    fold_partials<T, 3>(ft, partials, x, sm, &last);
 }
 
 // Min/max of the wrapping differences d[i] = x[i+1] - x[i], i < n - 1, read
 // straight from x (the delta encoder's output is never written when an FL
 // node consumes it).  Integer types only.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_minmax_delta(const T* __restrict__ x, size_t n, uint64_t* __restrict__ partials) {
+__global__ __launch_bounds__(kBlock) void k_minmax_delta(const T* __restrict__ x, size_t n, uint64_t* __restrict__ partials,
+                                                         FoldTail ft) {
     __shared__ uint64_t sm[kBlock / kWave];
+    __shared__ bool last;
     using U = typename UnsignedOf<T>::type;
     T dmn = std::numeric_limits<T>::max(), dmx = std::numeric_limits<T>::min();
     bool any = false;
@@ -212,40 +260,7 @@ __global__ __launch_bounds__(kBlock) void k_minmax_delta(const T* __restrict__ x
         st_agent(partials + 2 * blockIdx.x, mn);
         st_agent(partials + 2 * blockIdx.x + 1, mx);
     }
-}
-
-// Folds the per-workgroup partials of k_minmax (STRIDE 3: min, max, first
-// zero) or k_minmax_delta (STRIDE 2) into the result, in a launch of its own:
-// a "last workgroup" ticket would take one device-scope atomic per
-// workgroup on a single address, which costs more than this launch.
-template <typename T, int STRIDE>
-__global__ __launch_bounds__(kBlock) void k_minmax_fold(const uint64_t* __restrict__ partials, int blocks, const T* x,
-                                                        MinMaxResult* out, uint64_t* precision_out) {
-    __shared__ uint64_t sm[kBlock / kWave];
-    uint64_t mn = ~0ull, mx = 0, zf = ~0ull, pr = 0;
-    for (int b = threadIdx.x; b < blocks; b += kBlock) {
-        const uint64_t a = partials[STRIDE * b], z = partials[STRIDE * b + 1];
-        mn = a < mn ? a : mn;
-        mx = z > mx ? z : mx;
-        if (STRIDE >= 3) {
-            const uint64_t q = partials[STRIDE * b + 2];
-            zf = q < zf ? q : zf;
-        }
-        if (STRIDE == 4) {
-            const uint64_t q = partials[STRIDE * b + 3];
-            pr = q > pr ? q : pr;
-        }
-    }
-    mn = block_reduce_min(mn, sm);
-    mx = block_reduce_max(mx, sm);
-    if (STRIDE >= 3) zf = block_reduce_min(zf, sm);
-    if (STRIDE == 4) pr = block_reduce_max(pr, sm);
-    if (threadIdx.x == 0) {
-        if (STRIDE >= 3) fold_fixup(x, mn, mx, zf);
-        out->min_key = mn;
-        out->max_key = mx;
-        if (STRIDE == 4) *precision_out = pr;
-    }
+    fold_partials<T, 2>(ft, partials, x, sm, &last);
 }
 
 // ------------------------------------------------------------------- stats
@@ -269,8 +284,9 @@ __device__ __forceinline__ uint32_t float_precision(float number) {
 // {min, max, first zero, precision} per workgroup.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_minmax_prec(const T* __restrict__ x, size_t n,
-                                                        uint64_t* __restrict__ partials) {
+                                                        uint64_t* __restrict__ partials, FoldTail ft) {
     __shared__ uint64_t sm[kBlock / kWave];
+    __shared__ bool last;
     FoldKeys<T> f;
     uint32_t prec = 0;
     // The precision is a maximum capped at 10: a lane that has seen 10
@@ -320,6 +336,7 @@ __global__ __launch_bounds__(kBlock) void k_minmax_prec(const T* __restrict__ x,
         st_agent(partials + 4 * blockIdx.x + 2, zf);
         st_agent(partials + 4 * blockIdx.x + 3, pr);
     }
+    fold_partials<T, 4>(ft, partials, x, sm, &last);
 }
 
 template <typename T> __device__ __forceinline__ int32_t to_int32_sat(T v) {
@@ -458,7 +475,7 @@ __device__ __forceinline__ StatsAcc block_fold(StatsAcc a, StatsAcc* sm /* kBloc
 // 34 us on 10,000 rows, now 10).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_stats(const T* __restrict__ x, size_t n, DevStats* __restrict__ partials,
-                                                  uint32_t* counter, DevStats* out) {
+                                                  uint32_t* tickets, HostOut host) {
     constexpr int kBins = 65, kRegs = 64;
     __shared__ StatsAcc sm[kBlock / kWave];
     __shared__ uint32_t sm_hist[kBins * kHistCopies];
@@ -519,7 +536,7 @@ __global__ __launch_bounds__(kBlock) void k_stats(const T* __restrict__ x, size_
         }
         st_agent(&p->bit_hist[0] + i, v);
     }
-    if (!last_block_arrives(counter, &last)) return;
+    if (!last_of_grid(tickets, &last)) return;
     StatsAcc f{~0ull, 0, ~0ull, 0, 0, 0, 0, 0.0, 0, 0};
     for (uint32_t b = threadIdx.x; b < gridDim.x; b += kBlock) {
         const DevStats* q = partials + b;
@@ -560,6 +577,7 @@ __global__ __launch_bounds__(kBlock) void k_stats(const T* __restrict__ x, size_
         }
     }
     f = block_fold(f, sm);  // its barriers also complete fin
+    DevStats* out = reinterpret_cast<DevStats*>(host.dst);
     for (int i = threadIdx.x; i < kBins; i += kBlock) out->bit_hist[i] = fin[i];
     for (int i = threadIdx.x; i < kRegs; i += kBlock) out->hll[i] = fin[kBins + i];
     if (threadIdx.x == 0) {
@@ -574,8 +592,8 @@ __global__ __launch_bounds__(kBlock) void k_stats(const T* __restrict__ x, size_
         out->sum_f = f.sum_f;
         out->precision = f.prec;
         out->delta_bits_max = f.dmax;
-        __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    host_out_done(host);
 }
 
 int reduce_grid(Ctx* c, size_t n, int elem) {
@@ -587,40 +605,64 @@ int reduce_grid(Ctx* c, size_t n, int elem) {
 
 }  // namespace
 
-void launch_minmax(Ctx* c, int dtype, const void* x, size_t n, MinMaxResult* d_result, const uint64_t* d_rows) {
-    if (n == 0) fail(DDJ_EINVAL, "minmax of an empty array");
+HostOut launch_minmax(Ctx* c, int dtype, const void* x, size_t n, bool delta, MinMaxResult* d_result) {
+    if (n == 0 || (delta && n < 2)) fail(DDJ_EINVAL, "min/max of too few rows");
+    FoldTail ft;
+    ft.tickets = c->control->tickets;
+    ft.out = d_result;
+    ft.host = host_out(c);
     dispatch_native(dtype, [&](auto tag) {
         using T = decltype(tag);
         const int grid = reduce_grid(c, n, sizeof(T));
         DevBuf partials(c, 24 * (size_t)grid);
-        { KernelTimer kt_(c, "k_minmax"); hipLaunchKernelGGL(k_minmax<T>, dim3(grid), dim3(kBlock), 0, c->stream, static_cast<const T*>(x), n,
-                           partials.get<uint64_t>(), d_rows); }
-        HIPC(hipGetLastError());
-        { KernelTimer kt_(c, "k_minmax_fold"); hipLaunchKernelGGL((k_minmax_fold<T, 3>), dim3(1), dim3(kBlock), 0, c->stream,
-                           partials.get<uint64_t>(), grid, static_cast<const T*>(x), d_result, nullptr); }
+        KernelTimer kt_(c, delta ? "k_minmax_delta" : "k_minmax");
+        if (!delta) {
+            hipLaunchKernelGGL(k_minmax<T>, dim3(grid), dim3(kBlock), 0, c->stream, static_cast<const T*>(x), n,
+                               partials.get<uint64_t>(), nullptr, ft);
+        } else {
+            if constexpr (std::is_floating_point<T>::value)
+                fail(DDJ_EINVAL, "delta min/max: integer columns only");
+            else
+                hipLaunchKernelGGL(k_minmax_delta<T>, dim3(grid), dim3(kBlock), 0, c->stream, static_cast<const T*>(x),
+                                   n, partials.get<uint64_t>(), ft);
+        }
         HIPC(hipGetLastError());
     });
+    return ft.host;
 }
 
-void launch_float_scan(Ctx* c, int dtype, const void* x, size_t n, FloatScanResult* d_result) {
+MinMaxResult wait_minmax(Ctx* c, const HostOut& h) {
+    MinMaxResult r;
+    memcpy(&r, wait_host_out(c, h), sizeof r);
+    return r;
+}
+
+MinMaxResult minmax_to_host(Ctx* c, int dtype, const void* x, size_t n, bool delta) {
+    return wait_minmax(c, launch_minmax(c, dtype, x, n, delta, nullptr));
+}
+
+FloatScanResult float_scan(Ctx* c, int dtype, const void* x, size_t n) {
     if (n == 0) fail(DDJ_EINVAL, "float scan of an empty array");
+    FoldTail ft;
+    ft.tickets = c->control->tickets;
+    ft.host = host_out(c);
     dispatch_native(dtype, [&](auto tag) {
         using T = decltype(tag);
         if constexpr (std::is_floating_point<T>::value) {
             const int grid = reduce_grid(c, n, sizeof(T));
             DevBuf partials(c, 32 * (size_t)grid);
             kernel_bytes(c, "k_minmax_prec", (double)n * sizeof(T));
-            { KernelTimer kt_(c, "k_minmax_prec"); hipLaunchKernelGGL(k_minmax_prec<T>, dim3(grid), dim3(kBlock), 0, c->stream,
-                               static_cast<const T*>(x), n, partials.get<uint64_t>()); }
-            HIPC(hipGetLastError());
-            { KernelTimer kt_(c, "k_minmax_fold"); hipLaunchKernelGGL((k_minmax_fold<T, 4>), dim3(1), dim3(kBlock), 0, c->stream,
-                               partials.get<uint64_t>(), grid, static_cast<const T*>(x), &d_result->mm,
-                               &d_result->precision); }
+            KernelTimer kt_(c, "k_minmax_prec");
+            hipLaunchKernelGGL(k_minmax_prec<T>, dim3(grid), dim3(kBlock), 0, c->stream, static_cast<const T*>(x), n,
+                               partials.get<uint64_t>(), ft);
             HIPC(hipGetLastError());
         } else {
             fail(DDJ_EINVAL, "float scan of an integer column");
         }
     });
+    FloatScanResult r;
+    memcpy(&r, wait_host_out(c, ft.host), sizeof r);
+    return r;
 }
 
 // Workgroups of a reduction whose partials go to the host (6 KB of them):
@@ -642,7 +684,7 @@ int launch_minmax_partials(Ctx* c, int dtype, const void* x, size_t n, const uin
             partials = DevBuf(c, 24 * (size_t)grid);
             KernelTimer kt_(c, "k_minmax");
             hipLaunchKernelGGL(k_minmax<T>, dim3(grid), dim3(kBlock), 0, c->stream, static_cast<const T*>(x), n,
-                               partials.get<uint64_t>(), d_rows);
+                               partials.get<uint64_t>(), d_rows, FoldTail{});
             HIPC(hipGetLastError());
         }
     });
@@ -658,50 +700,6 @@ MinMaxResult fold_minmax_partials(const uint64_t* h, int grid, int stride) {
     return r;
 }
 
-MinMaxResult minmax_to_host(Ctx* c, int dtype, const void* x, size_t n, bool delta) {
-    if (n == 0 || (delta && n < 2)) fail(DDJ_EINVAL, "min/max of too few rows");
-    MinMaxResult r{~0ull, 0ull};
-    dispatch_native(dtype, [&](auto tag) {
-        using T = decltype(tag);
-        if constexpr (std::is_floating_point<T>::value) {
-            fail(DDJ_EINVAL, "host-folded min/max: integer columns only");
-        } else {
-            const int grid = reduce_grid(c, n, sizeof(T));
-            const int stride = delta ? 2 : 3;
-            DevBuf partials(c, 8 * (size_t)stride * (size_t)grid);
-            {
-                KernelTimer kt_(c, delta ? "k_minmax_delta" : "k_minmax");
-                if (delta)
-                    hipLaunchKernelGGL(k_minmax_delta<T>, dim3(grid), dim3(kBlock), 0, c->stream, static_cast<const T*>(x),
-                                       n, partials.get<uint64_t>());
-                else
-                    hipLaunchKernelGGL(k_minmax<T>, dim3(grid), dim3(kBlock), 0, c->stream, static_cast<const T*>(x), n,
-                                       partials.get<uint64_t>(), nullptr);
-            }
-            HIPC(hipGetLastError());
-            std::vector<uint64_t> h((size_t)stride * (size_t)grid);
-            d2h(c, h.data(), partials.get(), 8 * h.size());
-            r = fold_minmax_partials(h.data(), grid, stride);
-        }
-    });
-    return r;
-}
-
-void launch_minmax_delta(Ctx* c, int elem_size, const void* x, size_t n, MinMaxResult* d_result) {
-    if (n < 2) fail(DDJ_EINVAL, "delta min/max needs two rows");
-    dispatch_int(elem_size, [&](auto tag) {
-        using T = decltype(tag);
-        const int grid = reduce_grid(c, n, sizeof(T));
-        DevBuf partials(c, 16 * (size_t)grid);
-        { KernelTimer kt_(c, "k_minmax_delta"); hipLaunchKernelGGL(k_minmax_delta<T>, dim3(grid), dim3(kBlock), 0, c->stream, static_cast<const T*>(x), n,
-                           partials.get<uint64_t>()); }
-        HIPC(hipGetLastError());
-        { KernelTimer kt_(c, "k_minmax_fold"); hipLaunchKernelGGL((k_minmax_fold<T, 2>), dim3(1), dim3(kBlock), 0, c->stream,
-                           partials.get<uint64_t>(), grid, static_cast<const T*>(x), d_result, nullptr); }
-        HIPC(hipGetLastError());
-    });
-}
-
 void decode_minmax(int dtype, const MinMaxResult& r, void* mn, void* mx) {
     dispatch_native(dtype, [&](auto tag) {
         using T = decltype(tag);
@@ -711,16 +709,22 @@ void decode_minmax(int dtype, const MinMaxResult& r, void* mn, void* mx) {
     });
 }
 
-void launch_stats(Ctx* c, int dtype, const void* x, size_t n, DevStats* d_out) {
+DevStats device_stats(Ctx* c, int dtype, const void* x, size_t n) {
     if (n == 0) fail(DDJ_EINVAL, "stats of an empty array");
+    static_assert(sizeof(DevStats) <= kHostOutBytes, "the record fits the result slot");
+    const HostOut h = host_out(c);
     dispatch_native(dtype, [&](auto tag) {
         using T = decltype(tag);
         const int grid = std::min(reduce_grid(c, n, sizeof(T)), 2 * c->cu_count);
         DevBuf partials(c, sizeof(DevStats) * (size_t)grid);
-        { KernelTimer kt_(c, "k_stats"); hipLaunchKernelGGL(k_stats<T>, dim3(grid), dim3(kBlock), 0, c->stream, static_cast<const T*>(x), n,
-                           partials.get<DevStats>(), &c->control->counters[1], d_out); }
+        KernelTimer kt_(c, "k_stats");
+        hipLaunchKernelGGL(k_stats<T>, dim3(grid), dim3(kBlock), 0, c->stream, static_cast<const T*>(x), n,
+                           partials.get<DevStats>(), c->control->tickets, h);
         HIPC(hipGetLastError());
     });
+    DevStats r;
+    memcpy(&r, wait_host_out(c, h), sizeof r);
+    return r;
 }
 
 }  // namespace ddj

@@ -58,16 +58,13 @@ struct FloatScanResult {
     MinMaxResult mm;
     uint64_t precision;
 };
-void launch_float_scan(Ctx* c, int dtype, const void* x, size_t n, FloatScanResult* d_result);
+FloatScanResult float_scan(Ctx* c, int dtype, const void* x, size_t n);
 
-// min/max of n values of `dtype` into d_result (device).  One launch.
-void launch_minmax(Ctx* c, int dtype, const void* x, size_t n, MinMaxResult* d_result,
-                   const uint64_t* d_rows = nullptr /* device row count (<= n) read by the kernel, or null */);
-// min/max of the wrapping differences x[i+1] - x[i] of n integer rows.
-void launch_minmax_delta(Ctx* c, int elem_size, const void* x, size_t n, MinMaxResult* d_result);
-// Integer columns whose min/max the host needs: the reduction's partials
-// are read back and folded on the host (no fold launch).  delta: of the
-// differences x[i+1] - x[i].
+// min/max of n values of `dtype` (delta, integer types: of the wrapping
+// differences x[i+1] - x[i]) in one launch, into d_result (device) when set
+// and into the returned result slot, which wait_minmax reads.
+HostOut launch_minmax(Ctx* c, int dtype, const void* x, size_t n, bool delta, MinMaxResult* d_result);
+MinMaxResult wait_minmax(Ctx* c, const HostOut& h);
 MinMaxResult minmax_to_host(Ctx* c, int dtype, const void* x, size_t n, bool delta);
 // The reduction alone (integer columns, rows from *d_rows when given):
 // `partials` receives 3 order keys per workgroup, of which the returned
@@ -82,7 +79,7 @@ void launch_fl_pack_delta(Ctx* c, int elem_size, const void* x, size_t m, const 
 // Converts order keys back to the typed min/max (host).
 void decode_minmax(int dtype, const MinMaxResult& r, void* mn, void* mx);
 
-// Device statistics record filled by launch_stats.
+// Statistics record filled by device_stats.
 struct DevStats {
     uint64_t min_key, max_key;
     uint64_t first_zero;   // floats: row << 1 | sign of the first zero (~0: none)
@@ -96,7 +93,7 @@ struct DevStats {
     uint32_t bit_hist[65];
     uint32_t hll[64];
 };
-void launch_stats(Ctx* c, int dtype, const void* x, size_t n, DevStats* d_out);
+DevStats device_stats(Ctx* c, int dtype, const void* x, size_t n);
 
 // FL pack: bits from `mm` (device min/max) when mm is set, otherwise `bits`.
 // Writes the ceil(n*b/W)*sizeof(T) stream bytes to out (any byte address),

@@ -131,6 +131,58 @@ void d2h(Ctx* c, void* dst, const void* src, size_t bytes) {
     d2h_many(c, &rb, 1);
 }
 
+namespace {
+// Polls the completion flag for `seq` (a blocking stream wait sleeps once the
+// work outlasts its short spin, and wakes late).  After ~200 us the loop
+// yields between polls, leaving the cores to threads with host work; after
+// ~1 ms it also asks the runtime whether the stream has gone idle, so that a
+// failed launch is reported instead of waited on.
+void poll_flag(Ctx* c, uint32_t seq) {
+    const uint32_t* flag = reinterpret_cast<const uint32_t*>(c->readback + Ctx::kReadbackSize);
+    const auto t0 = std::chrono::steady_clock::now();
+    int phase = 0;  // 0 spin, 1 yield, 2 yield and query the stream
+    for (uint32_t spins = 1;; spins++) {
+        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == seq) return;
+        if (phase) std::this_thread::yield();
+        if ((spins & 255) != 0) continue;
+        if (phase < 2) {
+            const auto us = std::chrono::duration_cast<std::chrono::microseconds>(
+                                std::chrono::steady_clock::now() - t0).count();
+            phase = us > 1000 ? 2 : us > 200 ? 1 : 0;
+            continue;
+        }
+        const hipError_t q = hipStreamQuery(c->stream);
+        if (q == hipErrorNotReady) continue;
+        HIPC(q);  // idle: the flag is set by now
+        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) != seq) fail(DDJ_EHIP, "read-back flag not set");
+        return;
+    }
+}
+}  // namespace
+
+HostOut host_out(Ctx* c) {
+    HostOut h;
+    h.seq = ++c->readback_seq;
+    if (c->readback_dev) {
+        h.dst = c->readback_dev;
+        h.flag = reinterpret_cast<uint32_t*>(c->readback_dev + Ctx::kReadbackSize);
+    } else {
+        h.dst = c->control->host_out;
+        h.flag = reinterpret_cast<uint32_t*>(c->control->host_out + kHostOutBytes);
+    }
+    return h;
+}
+
+const uint8_t* wait_host_out(Ctx* c, const HostOut& h) {
+    if (c->readback_dev) {
+        poll_flag(c, h.seq);
+    } else {
+        HIPC(hipMemcpyAsync(c->readback, h.dst, kHostOutBytes, hipMemcpyDeviceToHost, c->stream));
+        HIPC(hipStreamSynchronize(c->stream));
+    }
+    return c->readback;
+}
+
 void d2h_many(Ctx* c, const ReadBack* rb, size_t count) {
     size_t total = 0;
     for (size_t i = 0; i < count; i++) total += (rb[i].bytes + 63) & ~(size_t)63;
@@ -151,31 +203,8 @@ void d2h_many(Ctx* c, const ReadBack* rb, size_t count) {
             off += (rb[i].bytes + 63) & ~(size_t)63;
         }
         const uint32_t seq = ++c->readback_seq;
-        uint32_t* flag = reinterpret_cast<uint32_t*>(c->readback + Ctx::kReadbackSize);
         launch_to_host(c, t, c->readback_dev, reinterpret_cast<uint32_t*>(c->readback_dev + Ctx::kReadbackSize), seq);
-        // Poll the flag (a blocking stream wait sleeps once the work outlasts
-        // its short spin, and wakes late).  After ~200 us the loop yields
-        // between polls, leaving the cores to threads with host work; after
-        // ~1 ms it also asks the runtime whether the stream has gone idle,
-        // so that a failed launch is reported instead of waited on.
-        const auto t0 = std::chrono::steady_clock::now();
-        int phase = 0;  // 0 spin, 1 yield, 2 yield and query the stream
-        for (uint32_t spins = 1;; spins++) {
-            if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == seq) break;
-            if (phase) std::this_thread::yield();
-            if ((spins & 255) != 0) continue;
-            if (phase < 2) {
-                const auto us = std::chrono::duration_cast<std::chrono::microseconds>(
-                                    std::chrono::steady_clock::now() - t0).count();
-                phase = us > 1000 ? 2 : us > 200 ? 1 : 0;
-                continue;
-            }
-            const hipError_t q = hipStreamQuery(c->stream);
-            if (q == hipErrorNotReady) continue;
-            HIPC(q);  // idle: the flag is set by now
-            if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) != seq) fail(DDJ_EHIP, "read-back flag not set");
-            break;
-        }
+        poll_flag(c, seq);
     } else {
         for (size_t i = 0; i < count; i++) {
             if (rb[i].bytes)

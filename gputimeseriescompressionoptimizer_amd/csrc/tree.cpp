@@ -1,6 +1,7 @@
 // The compression cascade: node records, blob assembly, parse and decode.
 #include "tree.h"
 
+#include <algorithm>
 #include <cstring>
 #include <functional>
 #include <sstream>
@@ -323,25 +324,18 @@ struct ParsedBlob {
 
     ParsedBlob(Ctx* cc, DView b) : c(cc), blob(b) {
         if (blob.n < 8) fail(DDJ_ECORRUPT, "blob shorter than one node header");
-        // status words and node table in one buffer, read back with one copy
-        // (trees have a few nodes; 64 table entries cover every planner tree)
-        constexpr int kHead = 64;  // bytes before the table
-        DevBuf parsed(c, kHead + sizeof(ParsedNode) * kMaxTreeNodes);
-        ParsedNode* table = reinterpret_cast<ParsedNode*>(parsed.bytes_ptr() + kHead);
-        launch_parse_tree(c, blob.p, blob.n, table, kMaxTreeNodes, parsed.get<int>());
-        constexpr int kFirst = 64;
-        std::vector<uint8_t> host(kHead + sizeof(ParsedNode) * kFirst);
-        d2h(c, host.data(), parsed.get(), host.size());
-        int st[3];
-        memcpy(st, host.data(), sizeof st);
+        DevBuf more(c, sizeof(ParsedNode) * kMaxTreeNodes);
+        const uint8_t* host = wait_host_out(c, launch_parse_tree(c, blob.p, blob.n, more.get<ParsedNode>(), kMaxTreeNodes));
+        int st[2];
+        memcpy(st, host, sizeof st);
         if (st[0] != 0) fail(DDJ_ECORRUPT, "malformed tree blob (parse status " + std::to_string(st[0]) + ")");
         const int count = st[1];
         if (count <= 0 || count > kMaxTreeNodes) fail(DDJ_ECORRUPT, "malformed tree blob (node count)");
         nodes.resize((size_t)count);
-        if (count <= kFirst)
-            memcpy(nodes.data(), host.data() + kHead, sizeof(ParsedNode) * count);
-        else
-            d2h(c, nodes.data(), table, sizeof(ParsedNode) * count);
+        memcpy(nodes.data(), host + kParseHostHead, sizeof(ParsedNode) * std::min(count, kParseHostNodes));
+        if (count > kParseHostNodes)
+            d2h(c, nodes.data() + kParseHostNodes, more.get<ParsedNode>() + kParseHostNodes,
+                sizeof(ParsedNode) * (count - kParseHostNodes));
         kids.resize((size_t)count);
         for (int i = 1; i < count; i++) kids[(size_t)nodes[i].parent].push_back(i);
         shadows_before = c->shadows.size();

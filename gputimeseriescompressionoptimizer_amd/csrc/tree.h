@@ -52,7 +52,12 @@ struct ParsedNode {
     uint8_t meta_head[kMetaHead];  // metadata bytes [0, min(meta_len, kMetaHead))
     uint8_t data_head[kMetaHead];  // leaves: data bytes [0, min(data_len, kMetaHead))
 };
-void launch_parse_tree(Ctx* c, const uint8_t* blob, uint64_t bytes, ParsedNode* d_out, int max_nodes, int* d_status);
+// The parse's result slot: {int32 status, int32 nodes}, and from byte
+// kParseHostHead the first kParseHostNodes nodes (trees have a few; 64 cover
+// every planner tree).  Later nodes go to d_more, by their index.
+constexpr int kParseHostHead = 64, kParseHostNodes = 64;
+static_assert(kParseHostHead + kParseHostNodes * sizeof(ParsedNode) <= kHostOutBytes, "the table fits the result slot");
+HostOut launch_parse_tree(Ctx* c, const uint8_t* blob, uint64_t bytes, ParsedNode* d_more, int max_nodes);
 
 // Decompression of none, afl -> none and delta -> afl -> none blobs (integer
 // columns) into caller memory with no device allocation (noalloc.hip).
