@@ -1,8 +1,6 @@
 // The statistics-driven planner.
 #include "planner.h"
 
-#include <deque>
-
 namespace ddj {
 
 namespace {
@@ -54,9 +52,14 @@ std::vector<std::vector<int>> generate_paths() {
     return out;
 }
 
+// Candidates share their subtrees: a node's candidates are every combination
+// of its outputs', 10^4..10^5 trees in all, which differ from each other in a
+// node or two (copying each subtree at each level above it was 45 of the 75
+// ms that planning a 10,000-row int32 sample took).  A chosen tree is copied
+// before anything changes it.
 std::vector<Candidate> full_statistics_update(Ctx* c, const Part& data, int et, int dt, int level) {
     const ddj_stats_t st = stats(c, dt, data.view());
-    std::vector<Candidate> result, part1;
+    std::vector<Candidate> result;
     for (int cont : get_continuations(et, dt, st, level)) {
         std::vector<Part> compr;
         if (cont == DDJ_ENC_NONE) {
@@ -69,39 +72,43 @@ std::vector<Candidate> full_statistics_update(Ctx* c, const Part& data, int et, 
         }
         size_t psize = 8;
         for (auto& p : compr) psize += p.n;
-        NodeP parent = make_node(cont, dt);
-        parent->ratio = ratio_of(data.n, psize);
         int rt[2];
         return_types(cont, dt, rt);
         const int k = n_results(cont);
+        const size_t before = result.size();
         if (k == 1) {
             auto kids = full_statistics_update(c, compr[1], cont, rt[0], level + 1);
-            part1.clear();
+            result.reserve(before + kids.size());
             for (auto& ch : kids) {
                 const size_t out = ch.size + compr[0].n + 8;
                 NodeP t = make_node(cont, dt);
-                t->ch.push_back(copy_tree(ch.tree));
+                t->ch.push_back(std::move(ch.tree));
                 t->ratio = ratio_of(data.n, out);
-                part1.push_back(Candidate{t, out});
+                result.push_back(Candidate{std::move(t), out});
             }
         } else if (k == 2) {
             auto left = full_statistics_update(c, compr[1], cont, rt[0], level + 1);
             auto right = full_statistics_update(c, compr[2], cont, rt[1], level + 1);
-            part1.clear();
+            result.reserve(before + left.size() * right.size());
             for (auto& l : left)
                 for (auto& r : right) {
                     const size_t out = l.size + r.size + compr[0].n + 8;
                     NodeP t = make_node(cont, dt);
-                    t->ch.push_back(copy_tree(l.tree));
-                    t->ch.push_back(copy_tree(r.tree));
+                    t->ch.reserve(2);
+                    t->ch.push_back(l.tree);
+                    t->ch.push_back(r.tree);
                     t->ratio = ratio_of(data.n, out);
-                    part1.push_back(Candidate{t, out});
+                    result.push_back(Candidate{std::move(t), out});
                 }
         }
-        // The reference keeps part1 across iterations (compression_optimizer.cpp:96-137);
-        // `none` comes first, so it only ever sees an empty list here.
-        if (part1.empty()) part1.push_back(Candidate{parent, psize});
-        result.insert(result.end(), part1.begin(), part1.end());
+        // The reference keeps its partial list across iterations
+        // (compression_optimizer.cpp:96-137); `none` comes first, so it only
+        // ever sees an empty list here.
+        if (result.size() == before) {
+            NodeP parent = make_node(cont, dt);
+            parent->ratio = ratio_of(data.n, psize);
+            result.push_back(Candidate{std::move(parent), psize});
+        }
     }
     return result;
 }
@@ -128,7 +135,7 @@ NodeP plan_exhaustive(Ctx* c, DView data, int dt, size_t* best_size, uint64_t* n
         }
     }
     if (best_size) *best_size = bsize;
-    return best;
+    return best ? copy_tree(best) : best;
 }
 
 NodeP optimize_tree(Ctx* c, DView data, int dt) {
@@ -185,26 +192,19 @@ std::pair<std::pair<int, int>, double> EdgeStats::get_best(int no, std::pair<int
 std::vector<Edge> get_edges(const NodeP& root, int max_height) {
     std::vector<Edge> out;
     const int maxno = (1 << (max_height + 1)) - 2;
-    TNode fake;
-    std::deque<TNode*> fifo{root.get()};
+    // breadth-first over the slots of a full binary tree, empty ones included
+    std::vector<TNode*> fifo;
+    fifo.reserve((size_t)maxno + 3);
+    fifo.push_back(root.get());
+    size_t head = 0;
     int no = 0;
-    while (!fifo.empty() && no < maxno) {
-        TNode* el = fifo.front();
-        fifo.pop_front();
-        if (el->ch.size() >= 1) {
-            out.push_back(Edge{el, el->ch[0].get(), no});
-            fifo.push_back(el->ch[0].get());
-        } else {
-            fifo.push_back(&fake);
+    while (head < fifo.size() && no < maxno) {
+        TNode* el = fifo[head++];
+        for (size_t k = 0; k < 2; k++, no++) {
+            TNode* to = el && el->ch.size() > k ? el->ch[k].get() : nullptr;
+            if (to) out.push_back(Edge{el, to, no});
+            fifo.push_back(to);
         }
-        no++;
-        if (el->ch.size() >= 2) {
-            out.push_back(Edge{el, el->ch[1].get(), no});
-            fifo.push_back(el->ch[1].get());
-        } else {
-            fifo.push_back(&fake);
-        }
-        no++;
     }
     return out;
 }
@@ -233,7 +233,7 @@ Part Optimizer::compress_data(DView part, int dt) {
                 best = cd.tree;
             }
         }
-        tree_ = best;
+        tree_ = copy_tree(best);  // compression sets its ratios, repair its children
         old_ratio_ = best->ratio;  // OptimalTree::OptimalTree (optimal_tree.hpp:26-33)
         old_stats_ = stats_;
         aliased_ = false;
