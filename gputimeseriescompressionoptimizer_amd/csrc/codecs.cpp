@@ -421,20 +421,13 @@ std::vector<Part> patch_encode(Ctx* c, int dtype, DView in, bool outside) {
     const bool integral = dtype != DDJ_D_FLOAT && dtype != DDJ_D_DOUBLE;
     auto mm_yes = integral ? std::make_shared<DevBuf>(c, sizeof(MinMaxResult)) : nullptr;
     auto mm_no = integral ? std::make_shared<DevBuf>(c, sizeof(MinMaxResult)) : nullptr;
-    launch_split(c, dtype, x.p, n, p, st.bytes_ptr(), yes.get(), no.get(), nullptr, cnt.get<uint64_t>(),
-                 integral ? mm_yes->get<MinMaxResult>() : nullptr, integral ? mm_no->get<MinMaxResult>() : nullptr);
-    // the count and both outputs' min/max in one read-back: the FL encoders
-    // of the outputs then need no pass and no read-back of their own
-    uint64_t m = 0;
-    auto hy = std::make_shared<MinMaxResult>(), hn = std::make_shared<MinMaxResult>();
-    if (integral) {
-        const ReadBack rb[3] = {{&m, cnt.get(), 8},
-                                {hy.get(), mm_yes->get(), sizeof(MinMaxResult)},
-                                {hn.get(), mm_no->get(), sizeof(MinMaxResult)}};
-        d2h_many(c, rb, 3);
-    } else {
-        d2h(c, &m, cnt.get(), 8);
-    }
+    // the count and both outputs' min/max in one result: the FL encoders of
+    // the outputs then need no pass and no read-back of their own
+    const ScanResult r = launch_split(c, dtype, x.p, n, p, st.bytes_ptr(), yes.get(), no.get(), nullptr,
+                                      cnt.get<uint64_t>(), integral ? mm_yes->get<MinMaxResult>() : nullptr,
+                                      integral ? mm_no->get<MinMaxResult>() : nullptr);
+    const uint64_t m = r.total;
+    auto hy = std::make_shared<MinMaxResult>(r.mm[0]), hn = std::make_shared<MinMaxResult>(r.mm[1]);
     yes.set_size(m * es);
     no.set_size((n - m) * es);
     kernel_bytes(c, "k_split", (double)(2 * n * es + 1 + (n + 7) / 8));
@@ -493,9 +486,8 @@ std::vector<Part> const_encode(Ctx* c, int dtype, DView in) {
     PredArgs p{};
     p.kind = PRED_NOT_EQUAL;
     p.a_bits = key[0];
-    launch_split(c, dtype, x.p, n, p, meta.bytes_ptr() + es, data.get(), nullptr, nullptr, cnt.get<uint64_t>());
-    uint64_t m = 0;
-    d2h(c, &m, cnt.get(), 8);
+    const uint64_t m = launch_split(c, dtype, x.p, n, p, meta.bytes_ptr() + es, data.get(), nullptr, nullptr,
+                                    cnt.get<uint64_t>()).total;
     data.set_size(m * es);
     return {own(std::move(meta)), own(std::move(data))};
 }
@@ -536,8 +528,7 @@ std::vector<Part> dict_encode(Ctx* c, int dtype, DView in, bool defer = false) {
         // rows then go straight to their blob range
         auto job = std::make_shared<SplitJob>();
         job->plan = launch_split_count(c, dtype, x.p, n, p);
-        uint64_t m = 0;
-        d2h(c, &m, job->plan.ts->prefix + job->plan.ts->tiles, 8);
+        const uint64_t m = split_result(c, job->plan).total;
         DevBuf st(c, 1 + (n + 7) / 8), f(c, head + 4 * ((m + 15) / 16));
         kernel_bytes(c, "k_hist_count", (double)(n * es));
         kernel_bytes(c, "k_split", (double)(n * es + 1 + (n + 7) / 8 + (m + 15) / 16 * 4 + (n - m) * es));
@@ -562,10 +553,8 @@ std::vector<Part> dict_encode(Ctx* c, int dtype, DView in, bool defer = false) {
         return {stp, freq, others};
     }
     DevBuf st(c, 1 + (n + 7) / 8), f(c, head + 4 * ((n + 15) / 16)), others(c, n * es), cnt(c, 8);
-    launch_split(c, dtype, x.p, n, p, st.bytes_ptr(), nullptr, others.get(), f.bytes_ptr() + head,
-                 cnt.get<uint64_t>());
-    uint64_t m = 0;
-    d2h(c, &m, cnt.get(), 8);
+    const uint64_t m = launch_split(c, dtype, x.p, n, p, st.bytes_ptr(), nullptr, others.get(), f.bytes_ptr() + head,
+                                    cnt.get<uint64_t>()).total;
     others.set_size((n - m) * es);
     kernel_bytes(c, "k_hist_count", (double)(n * es));
     kernel_bytes(c, "k_split", (double)(n * es + 1 + (n + 7) / 8 + (m + 15) / 16 * 4 + (n - m) * es));
@@ -737,10 +726,9 @@ PatchAflParts patch_afl_encode(Ctx* c, int dtype, DView in, bool outside) {
     job->plan = launch_split_count(c, dtype, x.p, n, p, mmy, mmy + 1);
     job->x = x;
     job->count = std::make_shared<DevBuf>(c, 8);
-    uint64_t m = 0;
-    MinMaxResult h[2];
-    const ReadBack rb[2] = {{&m, job->plan.ts->prefix + job->plan.ts->tiles, 8}, {h, mmb.get(), sizeof h}};
-    d2h_many(c, rb, 2);
+    const ScanResult r = split_result(c, job->plan);
+    const uint64_t m = r.total;
+    const MinMaxResult* h = r.mm;
     const uint64_t sides[2] = {m, n - m};
     PatchAflParts out;
     uint64_t bytes[2];

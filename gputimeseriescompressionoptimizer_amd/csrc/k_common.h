@@ -245,6 +245,82 @@ __device__ __forceinline__ void host_out_done(const HostOut& h) {
     if (threadIdx.x == 0) __hip_atomic_store(h.flag, h.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// A tile's value, where its tail (if any) will find it.
+__device__ __forceinline__ void put_tile(const ScanTail& st, uint64_t* vals, size_t tile, uint64_t v) {
+    if (st.tickets)
+        st_agent(vals + tile, v);
+    else
+        vals[tile] = v;
+}
+
+// The scan of a counting pass by its last workgroup (see ScanTail).  The
+// launch and the device time of a one-workgroup scan (8 us for a handful of
+// tiles) become 3 us of this tail.
+template <int NT = kBlock> __device__ __forceinline__ void scan_tail(const ScanTail& st, const uint64_t* vals) {
+    __shared__ uint64_t red[NT / kWave];
+    __shared__ unsigned long long mm[4];
+    __shared__ bool last;
+    if (!st.tickets || !last_of_grid(st.tickets, &last)) return;
+    auto rd = [](const uint64_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    constexpr int R = 4;  // consecutive values per thread and step
+    uint64_t r[4] = {~0ull, 0, ~0ull, 0};
+    if (st.keys) {
+        if (threadIdx.x < 4) mm[threadIdx.x] = (threadIdx.x & 1) ? 0ull : ~0ull;
+        for (uint64_t i = threadIdx.x; i < st.tiles; i += NT) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint64_t v = rd(st.keys + 4 * i + j);
+                r[j] = (j & 1) ? (v > r[j] ? v : r[j]) : (v < r[j] ? v : r[j]);
+            }
+        }
+    }
+    uint64_t carry = 0;
+    for (uint64_t c0 = 0; c0 < st.tiles; c0 += R * NT) {  // uniform
+        const uint64_t i0 = c0 + (uint64_t)threadIdx.x * R;
+        uint64_t v[R], s = 0, total;
+#pragma unroll
+        for (int k = 0; k < R; k++) v[k] = i0 + k < st.tiles ? rd(vals + i0 + k) : 0;
+#pragma unroll
+        for (int k = 0; k < R; k++) s += v[k];
+        uint64_t run = carry + block_exclusive_scan<uint64_t, NT>(s, &total, red);
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            if (i0 + k < st.tiles) st.prefix[i0 + k] = run;
+            run += v[k];
+        }
+        carry += total;
+    }
+    if (threadIdx.x == 0) st.prefix[st.tiles] = carry;
+    if (st.keys) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const unsigned long long w = (j & 1) ? wave_max(r[j]) : wave_min(r[j]);
+            if ((threadIdx.x & (kWave - 1)) == 0) {
+                if (j & 1)
+                    atomicMax(&mm[j], w);
+                else
+                    atomicMin(&mm[j], w);
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            if (st.mm_a) *st.mm_a = MinMaxResult{mm[0], mm[1]};
+            if (st.mm_b) *st.mm_b = MinMaxResult{mm[2], mm[3]};
+        }
+    }
+    if (!st.host.dst) return;
+    if (threadIdx.x == 0) {
+        ScanResult* h = reinterpret_cast<ScanResult*>(st.host.dst);
+        h->total = carry;
+        h->out_of_range = carry > st.n_yes || (st.n > carry && st.n - carry > st.n_no) ? 1 : 0;
+        if (st.keys) {
+            h->mm[0] = MinMaxResult{mm[0], mm[1]};
+            h->mm[1] = MinMaxResult{mm[2], mm[3]};
+        }
+    }
+    host_out_done(st.host);
+}
+
 // -------------------------------------------------------------- bit helpers
 __device__ __host__ __forceinline__ uint64_t lowmask64(unsigned n) { return n >= 64 ? ~0ull : ((1ull << n) - 1ull); }
 

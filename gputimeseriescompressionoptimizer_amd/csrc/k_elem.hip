@@ -243,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void k_to_host(ToHostPieces t, uint8_t* __r
 
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_delta_sums(const uint8_t* __restrict__ din, size_t m,
-                                                       uint64_t* __restrict__ vals) {
+                                                       uint64_t* __restrict__ vals, ScanTail st) {
     __shared__ uint64_t red[kBlock / kWave];
     const size_t base = (size_t)blockIdx.x * kScanTile;
     const int cnt = (int)((m - base) < (size_t)kScanTile ? (m - base) : (size_t)kScanTile);
@@ -265,7 +265,8 @@ __global__ __launch_bounds__(kBlock) void k_delta_sums(const uint8_t* __restrict
     }
     uint64_t total;
     block_exclusive_scan<uint64_t>(s, &total, red);
-    if (threadIdx.x == 0) vals[blockIdx.x] = total;
+    if (threadIdx.x == 0) put_tile(st, vals, blockIdx.x, total);
+    scan_tail(st, vals);
 }
 
 template <typename T>
@@ -500,6 +501,38 @@ TileScan::TileScan(Ctx* c, size_t n_tiles) : mem(c, 8 * (2 * n_tiles + 1)), tile
     prefix = vals + n_tiles;
 }
 
+// Up to 4M rows.  (Every counting workgroup waits for its store to reach the
+// coherence point before it takes its ticket, which costs a pass of 16K tiles
+// more than the scan's own launch.)
+constexpr size_t kFusedTiles = 1024;
+
+ScanTail TileScan::tail(Ctx* c, bool to_host) {
+    ScanTail t;
+    if (tiles > kFusedTiles) return t;
+    t.tickets = c->control->tickets;
+    t.prefix = prefix;
+    t.tiles = tiles;
+    if (to_host) t.host = host_out(c);
+    return t;
+}
+
+void TileScan::finish(Ctx* c, const ScanTail& t) {
+    if (!t.tickets) scan(c, t.keys, t.mm_a, t.mm_b);
+}
+
+ScanResult TileScan::result(Ctx* c, const ScanTail& t) {
+    ScanResult r{};
+    if (t.host.dst) {
+        memcpy(&r, wait_host_out(c, t.host), sizeof r);
+        return r;
+    }
+    ReadBack rb[3] = {{&r.total, prefix + tiles, 8}, {&r.mm[0], t.mm_a, sizeof(MinMaxResult)},
+                      {&r.mm[1], t.mm_b, sizeof(MinMaxResult)}};
+    d2h_many(c, rb, t.keys ? 3 : 1);
+    r.out_of_range = r.total > t.n_yes || (t.n > r.total && t.n - r.total > t.n_no) ? 1 : 0;
+    return r;
+}
+
 void TileScan::scan(Ctx* c, const uint64_t* keys, MinMaxResult* mm_a, MinMaxResult* mm_b) {
     if (keys && (!mm_a || !mm_b)) fail(DDJ_EINVAL, "tile key fold without outputs");
     if (!keys && tiles > (size_t)kScanRows * kScanThreads) {  // past one step of the one-workgroup scan
@@ -566,9 +599,10 @@ void launch_delta_decode(Ctx* c, int elem_size, const void* first, const uint8_t
         const size_t tiles = (m + kScanTile - 1) / kScanTile;
         TileScan ts(c, tiles);
         kernel_bytes(c, "k_delta_sums", (double)m * sizeof(T));
-        { KernelTimer kt_(c, "k_delta_sums"); hipLaunchKernelGGL(k_delta_sums<T>, dim3((unsigned)tiles), dim3(kBlock), 0, c->stream, d, m, ts.vals); }
+        const ScanTail st = ts.tail(c, false);
+        { KernelTimer kt_(c, "k_delta_sums"); hipLaunchKernelGGL(k_delta_sums<T>, dim3((unsigned)tiles), dim3(kBlock), 0, c->stream, d, m, ts.vals, st); }
         HIPC(hipGetLastError());
-        ts.scan(c);
+        ts.finish(c, st);
         { KernelTimer kt_(c, "k_delta_decode"); hipLaunchKernelGGL(k_delta_decode<T>, dim3((unsigned)tiles), dim3(kBlock), 0, c->stream,
                            static_cast<const uint8_t*>(first), d, m, static_cast<T*>(out), (const uint64_t*)ts.prefix); }
         HIPC(hipGetLastError());

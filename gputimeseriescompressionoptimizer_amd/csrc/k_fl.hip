@@ -76,12 +76,26 @@ __global__ __launch_bounds__(kBlock) void k_fl_unpack(const uint8_t* __restrict_
 // costs far less than writing and re-reading the deltas.  out has m + 1 rows.
 template <int MAXB>
 __global__ __launch_bounds__(kBlock) void k_fl_delta_sums(const uint8_t* __restrict__ in, size_t in_bytes, size_t m,
-                                                          int b, uint64_t* __restrict__ vals, size_t vbase) {
-    // sums of the deltas [vbase, vbase + m), one per tile of 4096
+                                                          int b, uint64_t* __restrict__ vals, size_t split,
+                                                          size_t m2, ScanTail st) {
+    // sums of the deltas [0, m), one per tile of 4096; with split > 0, of
+    // [0, split) in the first ceil(split / 4096) tiles and of [split, split +
+    // m2) in the others (a row range: the deltas before it and its own)
     __shared__ __attribute__((aligned(16))) uint32_t w[fl_stage_words<MAXB>()];
     __shared__ uint64_t red[kBlock / kWave];
-    const size_t v0 = (size_t)blockIdx.x * kFlTile;
-    const int nv = (int)((m - v0) < (size_t)kFlTile ? (m - v0) : (size_t)kFlTile);
+    size_t tile = blockIdx.x, vbase = 0;
+    if (split) {  // uniform
+        const size_t before = (split + kFlTile - 1) / kFlTile;
+        if (tile >= before) {
+            tile -= before;
+            vbase = split;
+            m = m2;
+        } else {
+            m = split;
+        }
+    }
+    const size_t v0 = tile * kFlTile;
+    const int nv = v0 < m ? (int)((m - v0) < (size_t)kFlTile ? (m - v0) : (size_t)kFlTile) : 0;
     const int a = stage_fl_words(in, in_bytes, vbase + v0, nv, b, w);
     __syncthreads();
     const uint64_t mask = lowmask64(b);
@@ -89,7 +103,8 @@ __global__ __launch_bounds__(kBlock) void k_fl_delta_sums(const uint8_t* __restr
     for (int k = threadIdx.x; k < nv; k += kBlock) sum += fl_value(w, k, b, a, mask);
     uint64_t total;
     block_exclusive_scan<uint64_t>(sum, &total, red);
-    if (threadIdx.x == 0) vals[blockIdx.x] = total;
+    if (threadIdx.x == 0) put_tile(st, vals, blockIdx.x, total);
+    scan_tail(st, vals);
 }
 
 template <typename T, int MAXB>
@@ -219,13 +234,19 @@ void launch_fl_unpack_delta(Ctx* c, int elem_size, const uint8_t* first, const u
             vals = own_scan->vals;
         }
         uint64_t* prefix = vals + tiles;
+        // caller's scratch: a scan launch of its own, which touches nothing
+        // that other calls of the context share
+        const ScanTail st = own_scan ? own_scan->tail(c, false) : ScanTail{};
         kernel_bytes(c, "k_fl_delta_sums", (double)((m * (uint64_t)bits + 7) / 8));
         with_maxb(bits, [&](auto mb) {
             constexpr int MAXB = decltype(mb)::value;
             { KernelTimer kt_(c, "k_fl_delta_sums"); hipLaunchKernelGGL(k_fl_delta_sums<MAXB>, dim3((unsigned)tiles), dim3(kBlock), 0, c->stream,
-                               in, in_bytes, m, bits, vals, (size_t)0); }
+                               in, in_bytes, m, bits, vals, (size_t)0, (size_t)0, st); }
             HIPC(hipGetLastError());
-            launch_scan_tiles(c, vals, tiles, prefix);
+            if (own_scan)
+                own_scan->finish(c, st);
+            else
+                launch_scan_tiles(c, vals, tiles, prefix);
             { KernelTimer kt_(c, "k_fl_unpack_delta_scan"); hipLaunchKernelGGL((k_fl_unpack_delta_scan<T, MAXB>), dim3((unsigned)tiles), dim3(kBlock), 0, c->stream,
                                first, in, in_bytes, m, bits, static_cast<T*>(out), (const uint64_t*)prefix, (size_t)0); }
         });
@@ -267,18 +288,14 @@ void launch_fl_unpack_delta_rows(Ctx* c, int elem_size, const uint8_t* first, co
         kernel_bytes(c, "k_fl_delta_sums", (double)(((begin + mb) * (uint64_t)bits + 7) / 8));
         with_maxb(bits, [&](auto mbits) {
             constexpr int MAXB = decltype(mbits)::value;
-            if (ta) {
-                KernelTimer kt_(c, "k_fl_delta_sums");
-                hipLaunchKernelGGL(k_fl_delta_sums<MAXB>, dim3((unsigned)ta), dim3(kBlock), 0, c->stream, in, in_bytes,
-                                   begin, bits, ts.vals, (size_t)0);
-            }
+            const ScanTail st = ts.tail(c, false);
             {
                 KernelTimer kt_(c, "k_fl_delta_sums");
-                hipLaunchKernelGGL(k_fl_delta_sums<MAXB>, dim3((unsigned)tb), dim3(kBlock), 0, c->stream, in, in_bytes,
-                                   mb, bits, ts.vals + ta, begin);
+                hipLaunchKernelGGL(k_fl_delta_sums<MAXB>, dim3((unsigned)(ta + tb)), dim3(kBlock), 0, c->stream, in,
+                                   in_bytes, mb, bits, ts.vals, begin, mb, st);
             }
             HIPC(hipGetLastError());
-            ts.scan(c);
+            ts.finish(c, st);
             KernelTimer kt_(c, "k_fl_unpack_delta_scan");
             hipLaunchKernelGGL((k_fl_unpack_delta_scan<T, MAXB>), dim3((unsigned)tb), dim3(kBlock), 0, c->stream, first, in,
                                in_bytes, mb, bits, static_cast<T*>(out), (const uint64_t*)(ts.prefix + ta), begin);

@@ -74,7 +74,8 @@ template <typename T> T bits_to(uint64_t b) {
 // no max}, so that an FL encoder of either output needs no pass of its own.
 template <typename T, bool MM, int K>
 __global__ __launch_bounds__(kBlock) void k_split_count(const T* __restrict__ x, size_t n, Pred<T> p,
-                                                        uint64_t* __restrict__ vals, uint64_t* __restrict__ keys) {
+                                                        uint64_t* __restrict__ vals, uint64_t* __restrict__ keys,
+                                                        ScanTail st) {
     __shared__ uint64_t red[kBlock / kWave];
     __shared__ unsigned long long mm[4];
     const size_t base = (size_t)blockIdx.x * kTile;
@@ -134,8 +135,9 @@ __global__ __launch_bounds__(kBlock) void k_split_count(const T* __restrict__ x,
     }
     uint64_t total;
     block_exclusive_scan<uint64_t>((uint64_t)c, &total, red);  // a barrier: mm is complete
-    if (threadIdx.x == 0) vals[blockIdx.x] = total;
-    if (MM && threadIdx.x < 4) keys[4 * (size_t)blockIdx.x + threadIdx.x] = mm[threadIdx.x];
+    if (threadIdx.x == 0) put_tile(st, vals, blockIdx.x, total);
+    if (MM && threadIdx.x < 4) put_tile(st, keys, 4 * (size_t)blockIdx.x + threadIdx.x, mm[threadIdx.x]);
+    scan_tail(st, vals);
 }
 
 
@@ -566,9 +568,8 @@ __global__ __launch_bounds__(kBlock) void k_code_edges(const uint64_t* __restric
 // tile, lane l taking the tile's stencil bytes [8l, 8l + 8).  Bits past row
 // n - 1 (the stencil's padding) are not counted.
 __global__ __launch_bounds__(kBlock) void k_stencil_count(const uint8_t* __restrict__ bits, size_t n, size_t tiles,
-                                                          uint64_t* __restrict__ vals) {
-    const size_t tile = (size_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
-    if (tile >= tiles) return;  // uniform per wave
+                                                          uint64_t* __restrict__ vals, ScanTail st) {
+    const size_t tile = (size_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;  // past the last: no rows
     const int lane = threadIdx.x & (kWave - 1);
     const size_t r0 = tile * kTile + (size_t)lane * 64;
     uint32_t c = 0;
@@ -583,7 +584,8 @@ __global__ __launch_bounds__(kBlock) void k_stencil_count(const uint8_t* __restr
         }
     }
     c = wave_sum(c);
-    if (lane == 0) vals[tile] = c;
+    if (lane == 0 && tile < tiles) put_tile(st, vals, tile, c);
+    scan_tail(st, vals);
 }
 
 // The "yes" rows of a merge given as dictionary codes: row j is
@@ -915,7 +917,8 @@ template <typename T> __device__ __forceinline__ T shfl_up_value(T v) {
 
 // Runs starting in each tile (the RLE encoder's counting pass).
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_rle_count(const T* __restrict__ x, size_t n, uint64_t* __restrict__ vals) {
+__global__ __launch_bounds__(kBlock) void k_rle_count(const T* __restrict__ x, size_t n, uint64_t* __restrict__ vals,
+                                                      ScanTail st) {
     __shared__ uint64_t red[kBlock / kWave];
     const size_t base = (size_t)blockIdx.x * kTile;
     const int cnt = (int)((n - base) < (size_t)kTile ? (n - base) : (size_t)kTile);
@@ -953,7 +956,8 @@ __global__ __launch_bounds__(kBlock) void k_rle_count(const T* __restrict__ x, s
     }
     uint64_t total;
     block_exclusive_scan<uint64_t>((uint64_t)c, &total, red);
-    if (threadIdx.x == 0) vals[blockIdx.x] = total;
+    if (threadIdx.x == 0) put_tile(st, vals, blockIdx.x, total);
+    scan_tail(st, vals);
 }
 
 template <typename T>
@@ -1037,7 +1041,7 @@ __device__ __forceinline__ uint64_t run_length(const uint8_t* lens, size_t r, bo
 // Rows covered by each tile of 4096 runs (the decoder's counting pass); a
 // negative length raises the error flag (2: corrupt input).
 __global__ __launch_bounds__(kBlock) void k_length_sums(const uint8_t* __restrict__ lens, size_t R,
-                                                        uint64_t* __restrict__ vals, uint32_t* error) {
+                                                        uint64_t* __restrict__ vals, uint32_t* error, ScanTail st) {
     __shared__ uint64_t red[kBlock / kWave];
     const size_t base = (size_t)blockIdx.x * kTile;
     const int cnt = (int)((R - base) < (size_t)kTile ? (R - base) : (size_t)kTile);
@@ -1048,7 +1052,8 @@ __global__ __launch_bounds__(kBlock) void k_length_sums(const uint8_t* __restric
     if (bad) __hip_atomic_store(error, 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     uint64_t total;
     block_exclusive_scan<uint64_t>(s, &total, red);
-    if (threadIdx.x == 0) vals[blockIdx.x] = total;
+    if (threadIdx.x == 0) put_tile(st, vals, blockIdx.x, total);
+    scan_tail(st, vals);
 }
 
 // Exclusive scan of int32 run lengths into uint64 offsets[R+1].
@@ -1233,6 +1238,11 @@ SplitPlan launch_split_count(Ctx* c, int dtype, const void* x, size_t n, const P
             fail(DDJ_EINVAL, "split min/max outputs need an integer type and both outputs");
         DevBuf keys;
         if (mm) keys = DevBuf(c, 32 * tiles);
+        plan.tail = ts.tail(c, true);
+        plan.tail.keys = mm ? keys.get<uint64_t>() : nullptr;
+        plan.tail.mm_a = mm_yes;
+        plan.tail.mm_b = mm_no;
+        const ScanTail st = plan.tail;
         const dim3 grid((unsigned)tiles), block(kBlock);
         with_kind(p.kind, [&](auto kind) {
             constexpr int K = decltype(kind)::value;
@@ -1240,14 +1250,14 @@ SplitPlan launch_split_count(Ctx* c, int dtype, const void* x, size_t n, const P
             if constexpr (std::is_integral<T>::value) {
                 if (mm) {
                     hipLaunchKernelGGL((k_split_count<T, true, K>), grid, block, 0, c->stream, xs, n, p, ts.vals,
-                                       keys.get<uint64_t>());
+                                       keys.get<uint64_t>(), st);
                     return;
                 }
             }
-            hipLaunchKernelGGL((k_split_count<T, false, K>), grid, block, 0, c->stream, xs, n, p, ts.vals, nullptr);
+            hipLaunchKernelGGL((k_split_count<T, false, K>), grid, block, 0, c->stream, xs, n, p, ts.vals, nullptr, st);
         });
         HIPC(hipGetLastError());
-        ts.scan(c, mm ? keys.get<uint64_t>() : nullptr, mm_yes, mm_no);
+        ts.finish(c, st);
     });
     return plan;
 }
@@ -1294,11 +1304,16 @@ void launch_split_write(Ctx* c, const SplitPlan& plan, uint8_t* stencil, void* y
     });
 }
 
-void launch_split(Ctx* c, int dtype, const void* x, size_t n, const PredArgs& pa, uint8_t* stencil, void* yes,
-                  void* no, uint8_t* codes, uint64_t* d_counts, MinMaxResult* mm_yes, MinMaxResult* mm_no) {
-    if (n == 0) return;
+ScanResult split_result(Ctx* c, const SplitPlan& plan) {
+    return plan.n ? plan.ts->result(c, plan.tail) : ScanResult{};
+}
+
+ScanResult launch_split(Ctx* c, int dtype, const void* x, size_t n, const PredArgs& pa, uint8_t* stencil, void* yes,
+                        void* no, uint8_t* codes, uint64_t* d_counts, MinMaxResult* mm_yes, MinMaxResult* mm_no) {
+    if (n == 0) return ScanResult{};
     const SplitPlan plan = launch_split_count(c, dtype, x, n, pa, mm_yes, mm_no);
     launch_split_write(c, plan, stencil, yes, static_cast<uint8_t*>(no), codes, d_counts);
+    return split_result(c, plan);
 }
 
 void launch_split_fl(Ctx* c, const SplitPlan& plan, uint8_t* stencil, FlSide yes, FlSide no, uint64_t* d_counts) {
@@ -1336,18 +1351,41 @@ void launch_split_fl(Ctx* c, const SplitPlan& plan, uint8_t* stencil, FlSide yes
 
 namespace {
 
+// Stencil counts and their scan.  A stencil that asks for more rows than the
+// outputs hold is corrupt input: with a tail the scan itself finds that, so
+// that the merge is not waited for (check_stencil); otherwise the merge's
+// error flag does.
+ScanTail scan_stencil(Ctx* c, TileScan& ts, const uint8_t* bits, size_t n, uint64_t n_yes, uint64_t n_no) {
+    ScanTail st = ts.tail(c, true);
+    st.n = n;
+    st.n_yes = n_yes;
+    st.n_no = n_no;
+    if (!st.tickets) arm_error_flag(c);
+    const unsigned cg = (unsigned)((ts.tiles + kBlock / kWave - 1) / (kBlock / kWave));
+    kernel_bytes(c, "k_stencil_count", (double)((n + 7) / 8));
+    {
+        KernelTimer kt_(c, "k_stencil_count");
+        hipLaunchKernelGGL(k_stencil_count, dim3(cg), dim3(kBlock), 0, c->stream, bits, n, ts.tiles, ts.vals, st);
+    }
+    HIPC(hipGetLastError());
+    ts.finish(c, st);
+    return st;
+}
+
+void check_stencil(Ctx* c, TileScan& ts, const ScanTail& st) {
+    if (!st.tickets || !ts.result(c, st).out_of_range) return;
+    const uint32_t zero = 0;  // the merge raised the flag too
+    h2d(c, &c->control->error_flag, &zero, 4);
+    fail(DDJ_ECORRUPT, "encoded input failed a device-side check");
+}
+
 // Stencil counts, their scan and the merge; `dc.words` set: yes rows from codes.
 template <typename T>
 void merge_impl(Ctx* c, const uint8_t* bits, size_t n, const uint8_t* yes, size_t n_yes, const DictCodes& dc,
                 const uint8_t* no, size_t n_no, bool const_no, T no_const, T* out) {
     const size_t tiles = (n + kTile - 1) / kTile;
     TileScan ts(c, tiles);
-    arm_error_flag(c);
-    const unsigned cg = (unsigned)((tiles + kBlock / kWave - 1) / (kBlock / kWave));
-    kernel_bytes(c, "k_stencil_count", (double)((n + 7) / 8));
-    { KernelTimer kt_(c, "k_stencil_count"); hipLaunchKernelGGL(k_stencil_count, dim3(cg), dim3(kBlock), 0, c->stream, bits, n, tiles, ts.vals); }
-    HIPC(hipGetLastError());
-    ts.scan(c);
+    const ScanTail st = scan_stencil(c, ts, bits, n, n_yes, const_no ? ~0ull : (uint64_t)n_no);
     const uint64_t* pre = ts.prefix;
     uint32_t* err = &c->control->error_flag;
     const dim3 grid((unsigned)tiles);
@@ -1367,6 +1405,7 @@ void merge_impl(Ctx* c, const uint8_t* bits, size_t n, const uint8_t* yes, size_
                            T(0), out, pre, err, FlSrc{}, FlSrc{});
     }
     HIPC(hipGetLastError());
+    check_stencil(c, ts, st);
 }
 
 // The merge of a patch whose sides are FL streams.
@@ -1375,17 +1414,13 @@ void merge_fl_impl(Ctx* c, const uint8_t* bits, size_t n, const uint8_t* yes, si
                    const uint8_t* no, size_t n_no, FlSrc fn, T* out) {
     const size_t tiles = (n + kTile - 1) / kTile;
     TileScan ts(c, tiles);
-    arm_error_flag(c);
-    const unsigned cg = (unsigned)((tiles + kBlock / kWave - 1) / (kBlock / kWave));
-    kernel_bytes(c, "k_stencil_count", (double)((n + 7) / 8));
-    { KernelTimer kt_(c, "k_stencil_count"); hipLaunchKernelGGL(k_stencil_count, dim3(cg), dim3(kBlock), 0, c->stream, bits, n, tiles, ts.vals); }
-    HIPC(hipGetLastError());
-    ts.scan(c);
+    const ScanTail st = scan_stencil(c, ts, bits, n, n_yes, n_no);
     KernelTimer kt_(c, "k_merge_fl");
     kernel_bytes(c, "k_merge_fl", (double)((n + 7) / 8) + (double)fy.bytes + (double)fn.bytes + (double)n * sizeof(T));
     hipLaunchKernelGGL((k_merge<T, false, false, true>), dim3((unsigned)tiles), dim3(kBlock), 0, c->stream, bits, n, yes,
                        n_yes, DictCodes{}, no, n_no, T(0), out, ts.prefix, &c->control->error_flag, fy, fn);
     HIPC(hipGetLastError());
+    check_stencil(c, ts, st);
 }
 
 }  // namespace
@@ -1442,10 +1477,11 @@ uint64_t launch_rle_encode(Ctx* c, int dtype, const void* x, size_t n, int32_t* 
         const size_t tiles = (n + kTile - 1) / kTile;
         TileScan ts(c, tiles);
         kernel_bytes(c, "k_rle_count", (double)n * sizeof(T));
+        const ScanTail st = ts.tail(c, false);
         { KernelTimer kt_(c, "k_rle_count"); hipLaunchKernelGGL(k_rle_count<T>, dim3((unsigned)tiles), dim3(kBlock), 0, c->stream,
-                           static_cast<const T*>(x), n, ts.vals); }
+                           static_cast<const T*>(x), n, ts.vals, st); }
         HIPC(hipGetLastError());
-        ts.scan(c);
+        ts.finish(c, st);
         DevBuf starts(c, 4 * n);
         { KernelTimer kt_(c, "k_rle_encode"); hipLaunchKernelGGL(k_rle_encode<T>, dim3((unsigned)tiles), dim3(kBlock), 0, c->stream,
                            static_cast<const T*>(x), n, static_cast<T*>(values), starts.get<uint32_t>(),
@@ -1485,10 +1521,11 @@ DevBuf rle_decode_dev(Ctx* c, int dtype, const uint8_t* lengths, const uint8_t* 
         arm_error_flag(c);
         kernel_bytes(c, "k_length_sums", 4.0 * (double)runs);
         kernel_bytes(c, "k_scan_lengths", 4.0 * (double)runs + 8.0 * (double)(runs + 1));
+        const ScanTail st = ts.tail(c, false);
         { KernelTimer kt_(c, "k_length_sums"); hipLaunchKernelGGL(k_length_sums, dim3((unsigned)tiles), dim3(kBlock), 0, c->stream, lengths, runs,
-                           ts.vals, &c->control->error_flag); }
+                           ts.vals, &c->control->error_flag, st); }
         HIPC(hipGetLastError());
-        ts.scan(c);
+        ts.finish(c, st);
         DevBuf offsets(c, 8 * (runs + 1));
         { KernelTimer kt_(c, "k_scan_lengths"); hipLaunchKernelGGL(k_scan_lengths, dim3((unsigned)tiles), dim3(kBlock), 0, c->stream, lengths, runs,
                            offsets.get<uint64_t>(), (const uint64_t*)ts.prefix); }

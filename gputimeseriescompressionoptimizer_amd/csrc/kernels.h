@@ -8,19 +8,50 @@
 
 namespace ddj {
 
+// Minimum and maximum of a column.
+struct MinMaxResult {
+    uint64_t min_key;  // order_key of the minimum
+    uint64_t max_key;  // order_key of the maximum
+};
+
 // Tile offsets of a variable-length output, computed ahead of the output
 // pass: a counting kernel fills vals[0..tiles) (one value per tile), scan()
 // launches k_scan_tiles, which writes prefix[t] = vals[0] + ... + vals[t-1]
 // for t <= tiles (prefix[tiles] is the total).  Sums wrap at 64 bits.
-struct MinMaxResult;
+//
+// Counting passes of up to kFusedTiles tiles take a ScanTail: their last
+// workgroup scans the values itself, and leaves the total (and what else it
+// was asked for) in the host's result slot.  Past that the scan is a launch of
+// its own, k_scan_tiles.
+struct ScanTail {
+    uint32_t* tickets = nullptr;  // null: no tail, the scan is a launch of its own
+    uint64_t* prefix = nullptr;
+    uint64_t tiles = 0;
+    const uint64_t* keys = nullptr;  // per tile {min, max, min, max} order keys, folded into mm_a and mm_b
+    MinMaxResult* mm_a = nullptr;
+    MinMaxResult* mm_b = nullptr;
+    // the total must lie in [n - n_no, n_yes] (a merge's outputs hold its rows)
+    uint64_t n = 0, n_yes = ~0ull, n_no = ~0ull;
+    HostOut host;  // ScanResult
+};
+struct ScanResult {
+    uint64_t total;
+    uint64_t out_of_range;  // 1: the total left [n - n_no, n_yes]
+    MinMaxResult mm[2];
+};
 struct TileScan {
     DevBuf mem;
-    uint64_t* vals = nullptr;
-    uint64_t* prefix = nullptr;
-    size_t tiles = 0;
+    uint64_t* vals;
+    uint64_t* prefix;
+    size_t tiles;
     TileScan(Ctx* c, size_t tiles);
-    // keys (optional): per-tile {min, max, min, max} order keys of two
-    // outputs, folded in the same launch into *mm_a and *mm_b.
+    // The counting launch's tail; to_host: with a result slot, which
+    // result() waits for (one outstanding at a time, as HostOut).
+    ScanTail tail(Ctx* c, bool to_host);
+    // After the counting launch: the scan's own launch where the tail did not
+    // take it.
+    void finish(Ctx* c, const ScanTail& t);
+    ScanResult result(Ctx* c, const ScanTail& t);
     void scan(Ctx* c, const uint64_t* keys = nullptr, MinMaxResult* mm_a = nullptr, MinMaxResult* mm_b = nullptr);
 };
 // k_scan_tiles over caller memory: prefix[t] for t <= tiles.
@@ -46,11 +77,6 @@ template <typename K> K* radix_sort(Ctx* c, K* keys, K* tmp, size_t n, int key_b
 // device-side check) arm it first; the call then reads and clears it.
 void arm_error_flag(Ctx* c);
 
-// Scratch of a single-pass reduction (per-block partials + result).
-struct MinMaxResult {
-    uint64_t min_key;  // order_key of the minimum
-    uint64_t max_key;  // order_key of the maximum
-};
 
 // The floatToInt encoder's inputs for a float / double column: min/max keys
 // and the float precision (maximum over the rows, as DevStats::precision).
@@ -160,18 +186,23 @@ struct PredArgs {
 // little-endian 32-bit word; every word holding a code is written (room for
 // ceil(n / 16) words).
 // `no` may sit at any byte address (rows stored unchanged into a blob).
-void launch_split(Ctx* c, int dtype, const void* x, size_t n, const PredArgs& p, uint8_t* stencil /* 1+ceil(n/8) */,
-                  void* yes, void* no, uint8_t* codes /* packed dict codes or null */, uint64_t* d_counts,
-                  MinMaxResult* mm_yes = nullptr, MinMaxResult* mm_no = nullptr);
-// The same in two steps: the counting pass and scan (the yes count is then
-// prefix[tiles] of the plan's scan, on the device), and the writing pass.
+// Returns the yes count (and the min/max keys where asked for), without
+// waiting for the writing pass.
+ScanResult launch_split(Ctx* c, int dtype, const void* x, size_t n, const PredArgs& p,
+                        uint8_t* stencil /* 1+ceil(n/8) */, void* yes, void* no,
+                        uint8_t* codes /* packed dict codes or null */, uint64_t* d_counts,
+                        MinMaxResult* mm_yes = nullptr, MinMaxResult* mm_no = nullptr);
+// The same in two steps: the counting pass and scan, whose result
+// split_result waits for (before any other read-back), and the writing pass.
 struct SplitPlan {
     int dtype = 0;
     const void* x = nullptr;
     size_t n = 0;
     PredArgs p{};
     std::shared_ptr<TileScan> ts;
+    ScanTail tail;
 };
+ScanResult split_result(Ctx* c, const SplitPlan& plan);
 SplitPlan launch_split_count(Ctx* c, int dtype, const void* x, size_t n, const PredArgs& p,
                              MinMaxResult* mm_yes = nullptr, MinMaxResult* mm_no = nullptr);
 void launch_split_write(Ctx* c, const SplitPlan& plan, uint8_t* stencil, void* yes, uint8_t* no, uint8_t* codes,

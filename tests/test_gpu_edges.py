@@ -90,3 +90,66 @@ def test_most_frequent_all_counts_tie(ctx):
     x = np.random.default_rng(1).permutation(np.arange(-50_000, 50_000, dtype=np.int32))
     meta = g.Encoding(ctx, g.DICT).Encode(ctx.upload(x), g.D_INT)[1].to_bytes()
     assert sorted(np.frombuffer(meta[16:32], np.int32)) == [-50_000, -49_999, -49_998, -49_997]
+
+
+# 4096-row tiles; up to 1024 of them are scanned by the counting pass's last
+# workgroup (its ticket groups begin past 64), more by a launch of their own
+@pytest.mark.parametrize("tiles", [1, 2, 64, 65, 1_023, 1_024, 1_025])
+@pytest.mark.parametrize("path,dtype", [
+    ([g.PATCH, g.AFL, g.NONE, g.AFL, g.NONE], g.D_SHORT),
+    ([g.PATCH, g.NONE, g.NONE], g.D_SHORT),
+    ([g.DICT, g.NONE, g.NONE], g.D_CHAR),
+    ([g.CONST, g.NONE], g.D_SHORT),
+    ([g.RLE, g.NONE, g.NONE], g.D_CHAR),
+    ([g.DELTA, g.AFL, g.NONE], g.D_SHORT),
+    ([g.DELTA, g.NONE], g.D_SHORT),
+], ids=["patch-fl", "patch", "dict", "const", "rle", "delta-fl", "delta"])
+def test_tile_scan(ctx, path, dtype, tiles):
+    npdt = g.NP_DTYPE[dtype]
+    r = np.random.default_rng(tiles)
+    for n in (4096 * tiles - 1, 4096 * tiles, 4096 * tiles + 1):
+        x = (r.integers(0, 100, n) + (r.random(n) < 0.02) * r.integers(0, 27, n)).astype(npdt)
+        x[n // 5: n // 4] = 3
+        tree = g.CompressionTree(ctx, path, dtype)
+        blob = tree.Compress(ctx.upload(x))
+        assert blob.to_bytes() == O.compress(O.tree_from_path(path, dtype), x)
+        assert np.array_equal(tree.Decompress(blob).to_numpy(npdt), x)
+
+
+@pytest.mark.parametrize("n", [5_000, 5_000_000])  # scanned with the count, and by a launch of its own
+def test_merge_outputs_too_short(ctx, n):
+    """A stencil with more set or clear bits than the outputs hold is refused."""
+    x = (np.arange(n) % 5).astype(np.int32)
+    enc = g.Encoding(ctx, g.DICT)
+    stencil, codes, rest = enc.Encode(ctx.upload(x), g.D_INT)
+    flipped = ctx.upload(np.bitwise_xor(np.frombuffer(stencil.to_bytes(), np.uint8),
+                                        np.r_[np.zeros(1, np.uint8), np.full(stencil.nbytes - 1, 255, np.uint8)]))
+    with pytest.raises(g.DdjError) as e:
+        enc.Decode([flipped, codes, rest], g.D_INT)
+    assert e.value.status == 3
+    assert np.array_equal(enc.Decode([stencil, codes, rest], g.D_INT).to_numpy(np.int32), x)
+
+
+@pytest.mark.parametrize("begin,count", [(0, 1), (0, 4097), (1, 1), (4095, 2), (4096, 4096), (4097, 1), (99_999, 1),
+                                         (70_001, 29_999), (0, 100_000)])
+def test_delta_row_ranges(ctx, begin, count):
+    x = np.cumsum(np.random.default_rng(3).integers(0, 60, 100_000)).astype(np.int32)
+    tree = g.CompressionTree(ctx, [g.DELTA, g.AFL, g.NONE], g.D_INT)
+    blob = tree.Compress(ctx.upload(x))
+    assert np.array_equal(tree.DecompressRows(blob, begin, count).to_numpy(np.int32), x[begin:begin + count])
+
+
+def test_parse_deep_and_wide_blobs(ctx):
+    """Node tables up to and past the 64 nodes that come back at once."""
+    x = np.random.default_rng(8).integers(0, 1000, 5_000).astype(np.int32)
+    for depth in (1, 5, 20, 31, 32, 33, 50):
+        path = [g.SCALE] * depth + [g.PATCH, g.DELTA, g.AFL, g.NONE, g.NONE]
+        blob = g.CompressionTree(ctx, path, g.D_INT).Compress(ctx.upload(x))
+        assert blob.to_bytes() == O.compress(O.tree_from_path(path, g.D_INT), x)
+        assert np.array_equal(g.CompressionTree(ctx).Decompress(blob).to_numpy(np.int32), x)
+    def both(d):
+        return [g.PATCH] + both(d - 1) + both(d - 1) if d else [g.NONE]
+    path = both(6)  # 127 nodes
+    blob = g.CompressionTree(ctx, path, g.D_INT).Compress(ctx.upload(x))
+    assert blob.to_bytes() == O.compress(O.tree_from_path(path, g.D_INT), x)
+    assert np.array_equal(g.CompressionTree(ctx).Decompress(blob).to_numpy(np.int32), x)
