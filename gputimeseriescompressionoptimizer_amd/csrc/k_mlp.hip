@@ -4,8 +4,8 @@
 // v_mfma_f32_32x32x8_bf16: BF16 operands, FP32 accumulation.  Master weights,
 // gradients and the Adam state stay in FP32.
 //
-// A wave owns a tile of 32 rows (blocks) and runs a whole pass for it out
-// of LDS.  Register layout of the 32x32x8 instruction, lane l of 64:
+// A workgroup (forward: four waves, backward: one) owns a tile of 32 rows
+// (blocks) and runs a whole pass for it out of LDS.  Register layout of the 32x32x8 instruction, lane l of 64:
 //   A (32 x 8, M x K): lane holds A[l % 32][4 (l / 32) + j], j = 0..3
 //   B (8 x 32, K x N): lane holds B[4 (l / 32) + j][l % 32]
 //   D (32 x 32):       register r holds D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32]
@@ -49,10 +49,29 @@ __device__ __forceinline__ f32x16 mma(const uint16_t* A, int lda, const uint16_t
     return acc;
 }
 
-// Loads W [K][N] (FP32, row-major) as BT [N][K] BF16 into LDS.
-__device__ __forceinline__ void load_wt(const float* __restrict__ W, int K, int N, uint16_t* wt, int ldw) {
-    for (int e = threadIdx.x; e < K * N; e += 64) wt[(e % N) * ldw + e / N] = to_bf16(W[e]);
-}
+// W [K][N] (FP32, row-major) as BT [N][K] BF16 into LDS, in two steps so that
+// every layer's loads are in flight together: fetch() issues a thread's
+// 16-byte loads, put() converts and stores them.
+constexpr int kFwdThreads = 256;
+template <int K, int N> struct WeightTile {
+    static constexpr int L = K * N / 4 / kFwdThreads;  // 16-byte loads per thread
+    static_assert(L * 4 * kFwdThreads == K * N, "whole loads");
+    float4 v[L];
+    __device__ __forceinline__ void fetch(const float* __restrict__ W) {
+#pragma unroll
+        for (int q = 0; q < L; q++) v[q] = reinterpret_cast<const float4*>(W)[threadIdx.x + q * kFwdThreads];
+    }
+    __device__ __forceinline__ void put(uint16_t* wt, int ldw) const {
+#pragma unroll
+        for (int q = 0; q < L; q++) {
+            const int e = 4 * (threadIdx.x + q * kFwdThreads), k = e / N, n = e % N;
+            wt[n * ldw + k] = to_bf16(v[q].x);
+            wt[(n + 1) * ldw + k] = to_bf16(v[q].y);
+            wt[(n + 2) * ldw + k] = to_bf16(v[q].z);
+            wt[(n + 3) * ldw + k] = to_bf16(v[q].w);
+        }
+    }
+};
 // Loads W [K][N] (FP32) as W [K][N] BF16 (row k = B column k of W^T).
 __device__ __forceinline__ void load_w(const float* __restrict__ W, int K, int N, uint16_t* w, int ldw) {
     for (int e = threadIdx.x; e < K * N; e += 64) w[(e / N) * ldw + e % N] = to_bf16(W[e]);
@@ -72,44 +91,56 @@ __device__ __forceinline__ void put_act(const f32x16& acc, uint16_t* Hs, int ldh
 
 }  // namespace
 
-// Forward pass over B rows: Y [B][48] FP32; the hidden activations (BF16)
-// are kept for the backward pass when H1s / H2s are given.
-__global__ __launch_bounds__(64) void k_mlp_forward(const float* __restrict__ X, int B, MlpParams p,
-                                                    float* __restrict__ Y, uint16_t* __restrict__ H1s,
-                                                    uint16_t* __restrict__ H2s) {
+// Forward pass over B rows: Y [B][48] FP32, or with a result slot (one
+// workgroup, B <= 32) straight to the host; the hidden activations (BF16) are
+// kept for the backward pass when H1s / H2s are given.  Planning runs it on a
+// single row, where it is bound by fetching the 115 KB of weights: four waves
+// with all 28 loads a thread in flight, each wave computing its own columns
+// of a layer, take 12 us; one wave loading a float at a time took 78.
+__global__ __launch_bounds__(kFwdThreads) void k_mlp_forward(const float* __restrict__ X, int B, MlpParams p,
+                                                             float* __restrict__ Y, uint16_t* __restrict__ H1s,
+                                                             uint16_t* __restrict__ H2s, HostOut host) {
     __shared__ __attribute__((aligned(16))) uint16_t w1t[kH * LF];
     __shared__ __attribute__((aligned(16))) uint16_t w2t[kH * LH];
     __shared__ __attribute__((aligned(16))) uint16_t w3t[kOP * LH];
     __shared__ __attribute__((aligned(16))) uint16_t xs[32 * LF];
     __shared__ __attribute__((aligned(16))) uint16_t h1[32 * LH];
     __shared__ __attribute__((aligned(16))) uint16_t h2[32 * LH];
-    const int l = threadIdx.x;
-    load_wt(p.W1, kF, kH, w1t, LF);
-    load_wt(p.W2, kH, kH, w2t, LH);
-    load_wt(p.W3, kH, kOP, w3t, LH);
+    const int l = threadIdx.x & 63, wid = threadIdx.x / 64;
+    static_assert(kH / 32 == kFwdThreads / 64, "one wave per 32 columns of a hidden layer");
+    WeightTile<kF, kH> w1;
+    WeightTile<kH, kH> w2;
+    WeightTile<kH, kOP> w3;
+    w1.fetch(p.W1);
+    w2.fetch(p.W2);
+    w3.fetch(p.W3);
     const int r0 = blockIdx.x * 32;
-    for (int e = l; e < 32 * kF; e += 64) {
+    for (int e = threadIdx.x; e < 32 * kF; e += kFwdThreads) {
         const int i = e / kF, k = e % kF;
         xs[i * LF + k] = (r0 + i < B) ? to_bf16(X[(size_t)(r0 + i) * kF + k]) : (uint16_t)0;
     }
+    w1.put(w1t, LF);
+    w2.put(w2t, LH);
+    w3.put(w3t, LH);
     __syncthreads();
-    for (int nt = 0; nt < kH / 32; nt++) put_act(mma(xs, LF, w1t + nt * 32 * LF, LF, kF, f32x16{}), h1, LH, nt * 32, p.b1);
+    put_act(mma(xs, LF, w1t + wid * 32 * LF, LF, kF, f32x16{}), h1, LH, wid * 32, p.b1);
     __syncthreads();
-    for (int nt = 0; nt < kH / 32; nt++) put_act(mma(h1, LH, w2t + nt * 32 * LH, LH, kH, f32x16{}), h2, LH, nt * 32, p.b2);
+    put_act(mma(h1, LH, w2t + wid * 32 * LH, LH, kH, f32x16{}), h2, LH, wid * 32, p.b2);
     __syncthreads();
-    for (int nt = 0; nt < kOP / 32; nt++) {
-        const f32x16 acc = mma(h2, LH, w3t + nt * 32 * LH, LH, kH, f32x16{});
-        const int c = nt * 32 + (l & 31);
+    if (wid < kOP / 32) {
+        float* out = host.dst ? reinterpret_cast<float*>(host.dst) : Y;
+        const f32x16 acc = mma(h2, LH, w3t + wid * 32 * LH, LH, kH, f32x16{});
+        const int c = wid * 32 + (l & 31);
         if (c < kO) {
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int row = r0 + d_row(r, l);
-                if (row < B) Y[(size_t)row * kO + c] = acc[r] + p.b3[c];
+                if (row < B) out[(size_t)row * kO + c] = acc[r] + p.b3[c];
             }
         }
     }
     if (H1s && H2s) {
-        for (int e = l; e < 32 * kH; e += 64) {
+        for (int e = threadIdx.x; e < 32 * kH; e += kFwdThreads) {
             const int i = e / kH, k = e % kH;
             if (r0 + i < B) {
                 H1s[(size_t)(r0 + i) * kH + k] = h1[i * LH + k];
@@ -117,6 +148,7 @@ __global__ __launch_bounds__(64) void k_mlp_forward(const float* __restrict__ X,
             }
         }
     }
+    if (host.dst) host_out_done(host);
 }
 
 namespace {
@@ -241,9 +273,11 @@ __global__ void k_adam(float* __restrict__ w, float* __restrict__ grad, float* _
     grad[i] = 0.f;
 }
 
-void launch_mlp_forward(Ctx* c, const float* X, int B, const MlpParams& p, float* Y, uint16_t* H1s, uint16_t* H2s) {
+void launch_mlp_forward(Ctx* c, const float* X, int B, const MlpParams& p, float* Y, uint16_t* H1s, uint16_t* H2s,
+                        const HostOut& host) {
     if (B <= 0) return;
-    { KernelTimer kt_(c, "k_mlp_forward"); hipLaunchKernelGGL(k_mlp_forward, dim3((B + 31) / 32), dim3(64), 0, c->stream, X, B, p, Y, H1s, H2s); }
+    if (host.dst && B > 32) fail(DDJ_EINVAL, "a result slot takes one tile of predictions");
+    { KernelTimer kt_(c, "k_mlp_forward"); hipLaunchKernelGGL(k_mlp_forward, dim3((B + 31) / 32), dim3(kFwdThreads), 0, c->stream, X, B, p, Y, H1s, H2s, host); }
     HIPC(hipGetLastError());
 }
 

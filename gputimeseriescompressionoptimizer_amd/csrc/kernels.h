@@ -294,7 +294,9 @@ inline MlpParams mlp_params_at(float* base) {
     p.b3 = p.W3 + 128 * 64;
     return p;
 }
-void launch_mlp_forward(Ctx* c, const float* X, int B, const MlpParams& p, float* Y, uint16_t* H1s, uint16_t* H2s);
+// host (B <= 32): the predictions go to the result slot instead of Y.
+void launch_mlp_forward(Ctx* c, const float* X, int B, const MlpParams& p, float* Y, uint16_t* H1s, uint16_t* H2s,
+                        const HostOut& host = HostOut{});
 void launch_mlp_backward(Ctx* c, const float* X, const uint16_t* H1s, const uint16_t* H2s, const float* Y,
                          const float* T, int B, const MlpParams& p, const MlpParams& g);
 void launch_adam(Ctx* c, float* w, float* grad, float* m, float* v, int n, float lr, int step);

@@ -394,6 +394,18 @@ void PlannerNet::predict_dev(const float* dX, int n, float* dY) {
 
 void PlannerNet::predict(const float* X, size_t n, float* Y) {
     if (n == 0) return;
+    static_assert(4 * 32 * kMlpOutputs <= kHostOutBytes, "a tile of predictions fits the result slot");
+    // a tile of rows (planning: one) is read from the pinned staging ring and
+    // predicted straight into the host's result slot
+    const uint8_t* slot = n <= 32 ? staging_slot(c_, 4 * n * kMlpFeatures) : nullptr;
+    if (slot) {
+        memcpy(c_->staging + (slot - c_->staging_dev), X, 4 * n * kMlpFeatures);
+        const HostOut h = host_out(c_);
+        launch_mlp_forward(c_, reinterpret_cast<const float*>(slot), (int)n, mlp_params_at(params_.get<float>()), nullptr,
+                           nullptr, nullptr, h);
+        memcpy(Y, wait_host_out(c_, h), 4 * n * kMlpOutputs);
+        return;
+    }
     DevBuf dX(c_, 4 * n * kMlpFeatures), dY(c_, 4 * n * kMlpOutputs);
     h2d(c_, dX.get(), X, 4 * n * kMlpFeatures);
     predict_dev(dX.get<float>(), (int)n, dY.get<float>());

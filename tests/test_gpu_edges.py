@@ -153,3 +153,14 @@ def test_parse_deep_and_wide_blobs(ctx):
     blob = g.CompressionTree(ctx, path, g.D_INT).Compress(ctx.upload(x))
     assert blob.to_bytes() == O.compress(O.tree_from_path(path, g.D_INT), x)
     assert np.array_equal(g.CompressionTree(ctx).Decompress(blob).to_numpy(np.int32), x)
+
+
+@pytest.mark.parametrize("rows", [1, 31, 32, 33, 100])
+def test_planner_rows_predicted_alone_or_together(ctx, rows):
+    """Up to 32 rows go straight to the host, more through device buffers;
+    a row's prediction does not depend on the rows beside it."""
+    net = g.LearnedPlanner(ctx, seed=5)
+    x = np.random.default_rng(rows).standard_normal((rows, g.MLP_FEATURES)).astype(np.float32)
+    y = net.Predict(x)
+    for i in {0, rows // 2, rows - 1}:
+        assert np.array_equal(net.Predict(x[i:i + 1])[0], y[i])
