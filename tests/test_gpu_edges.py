@@ -164,3 +164,38 @@ def test_planner_rows_predicted_alone_or_together(ctx, rows):
     y = net.Predict(x)
     for i in {0, rows // 2, rows - 1}:
         assert np.array_equal(net.Predict(x[i:i + 1])[0], y[i])
+
+
+# 12,288 rows (10,240 of 8 bytes) are the most that one workgroup counts; past
+# them integer keys within 512 of the first row's are counted by their offset
+@pytest.mark.parametrize("dtype", INT_TYPES + [g.D_FLOAT, g.D_DOUBLE])
+@pytest.mark.parametrize("n", [1, 5, 10_239, 10_240, 10_241, 12_287, 12_288, 12_289, 40_003])
+def test_most_frequent_small_columns_and_windows(ctx, dtype, n):
+    npdt = g.NP_DTYPE[dtype]
+    r = np.random.default_rng(n)
+    if dtype in (g.D_FLOAT, g.D_DOUBLE):
+        x = r.integers(-4, 4, n).astype(npdt) * npdt(-0.25)  # zeros of both signs
+        x[r.random(n) < 0.01] = np.nan
+        every = (r.standard_normal(n) * 1e3).astype(npdt)
+    else:
+        i = np.iinfo(npdt)
+        lo = r.choice([i.min, -1, i.max - 3])  # around the wrap and the all-ones pattern
+        x = (lo + (r.integers(0, 1_200, n) * (r.random(n) < 0.4))).astype(npdt)
+        every = r.permutation(np.arange(n)).astype(npdt)
+    for col in (x, every, np.full(n, x[0], npdt)):
+        outs = [o.to_bytes() for o in g.Encoding(ctx, g.DICT).Encode(ctx.upload(col), dtype)]
+        assert outs == O.encode(g.DICT, dtype, col)
+        outs = [o.to_bytes() for o in g.Encoding(ctx, g.CONST).Encode(ctx.upload(col), dtype)]
+        assert outs == O.encode(g.CONST, dtype, col)
+
+
+@pytest.mark.parametrize("dtype,edge", [(g.D_INT, 512), (g.D_SHORT, 512), (g.D_TIME, 512)])
+def test_most_frequent_at_the_window_edges(ctx, dtype, edge):
+    npdt = g.NP_DTYPE[dtype]
+    for base in (0, np.iinfo(npdt).max, np.iinfo(npdt).min):
+        with np.errstate(over="ignore"):
+            keys = np.array([base], npdt) + np.array([0, -edge - 1, -edge, -edge + 1, edge - 1, edge, edge + 1], npdt)
+        x = np.repeat(keys, [1, 9_001, 9_002, 9_003, 9_004, 9_005, 9_006]).astype(npdt)
+        x[1:] = np.random.default_rng(2).permutation(x[1:])
+        outs = [o.to_bytes() for o in g.Encoding(ctx, g.DICT).Encode(ctx.upload(x), dtype)]
+        assert outs == O.encode(g.DICT, dtype, x)
