@@ -169,8 +169,8 @@ constexpr int kHistThreads = 1024;
 // no two lanes of a wave on one bank but the pairs that share a copy.  Other
 // keys take the hash table.  The count of the 64M-row Zipf(1.2)/50 column was
 // bound by the probe loop's instructions and the LDS atomics' same-address
-// conflicts (92 us); with the window it
-// takes 54, against 42 for a plain pass over the column.
+// conflicts (92 us); with the window it takes 54, against 42 for a plain pass
+// over the column.
 constexpr int kWindow = 1024, kCopies = 32;
 
 template <typename T>
