@@ -264,7 +264,7 @@ class Context:
                "k_delta_sums", "k_fill_zero", "k_fl_delta_sums", "k_fl_edges", "k_fl_fetch", "k_fl_pack",
                "k_fl_pack_lanes", "k_fl_unpack", "k_fl_unpack_delta_scan", "k_fl_unpack_lanes", "k_float_compose",
                "k_float_split", "k_float_to_int", "k_gather_copy", "k_gfc_chunk_bytes", "k_gfc_decode", "k_gfc_encode",
-               "k_gfc_sizes", "k_gfc_walk", "k_hist_count", "k_hist_init", "k_hist_small", "k_hist_topk", "k_int_to_float",
+               "k_gfc_sizes", "k_gfc_walk", "k_hist_count", "k_hist_init", "k_hist_merge", "k_hist_small", "k_hist_topk", "k_int_to_float",
                "k_length_sums", "k_merge", "k_merge_fl", "k_minmax", "k_minmax_delta",
                "k_minmax_prec", "k_mlp_backward", "k_mlp_forward", "k_order_keys", "k_parse_tree", "k_radix_count",
                "k_radix_scatter", "k_rle_count", "k_rle_encode", "k_rle_expand", "k_rle_lengths", "k_rle_tile_runs",

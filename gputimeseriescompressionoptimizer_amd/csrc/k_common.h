@@ -93,7 +93,9 @@ template <bool MAX> __device__ __forceinline__ int32_t wave_extreme_i32(int32_t 
 template <bool MAX> __device__ __forceinline__ uint64_t wave_extreme_u64(uint64_t v) {
     constexpr uint32_t kFlip = 0x80000000u;  // unsigned order as signed order
     const uint32_t hi = (uint32_t)(v >> 32);
-    const uint32_t mh = (uint32_t)wave_extreme_i32<MAX>((int32_t)(hi ^ kFlip)) ^ kFlip;
+    const uint32_t hi0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)hi);
+    const bool same = __ballot(hi != hi0) == 0;  // as for counts: only the low halves differ (uniform)
+    const uint32_t mh = same ? hi0 : (uint32_t)wave_extreme_i32<MAX>((int32_t)(hi ^ kFlip)) ^ kFlip;
     const uint32_t lo = hi == mh ? (uint32_t)v : (MAX ? 0u : ~0u);
     const uint32_t ml = (uint32_t)wave_extreme_i32<MAX>((int32_t)(lo ^ kFlip)) ^ kFlip;
     return ((uint64_t)mh << 32) | ml;
@@ -200,6 +202,12 @@ constexpr int kScanRows = 16;  // rows of kScanThreads values per step of k_scan
 // publishes and another reads within the same launch.
 __device__ __forceinline__ void st_agent(uint64_t* p, uint64_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_agent(unsigned long long* p, unsigned long long v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T> __device__ __forceinline__ T ld_agent(const T* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void st_agent(uint32_t* p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -4,22 +4,27 @@
 // largest counts, equal counts ordered by the smaller value (what the
 // reference's stable sort of key-sorted bins yields).
 //
-// Counting: each workgroup aggregates its rows in an LDS hash table (plain
-// LDS atomics; the 16 rows a thread loads at once keep HBM busy while they
-// wait) and flushes it into a global open-addressing table (64-bit keys,
-// ~0 = empty);
-// rows that find no LDS slot go straight to the global table.  A 64-bit
-// value equal to the empty marker is counted on the side.  Floats count
-// -0.0 with +0.0 (operator==), reporting -0.0 when one was seen (it sorts
-// first in the reference).  A NaN equals nothing, so each NaN row is a bin
-// of count 1: they stay out of the table, and every workgroup keeps the four
-// smallest (radix order) NaN rows, which is all the top-K can ever take from
-// them.  Columns of a few thousand rows are counted whole in one workgroup's
-// LDS (k_hist_small).  The global table starts at 2n slots (at least 1024, at most 64K);
-// if it ends up more than 70% full the host retries once with a table of
-// twice the keys seen (the exact count, or with a full table the keys seen
-// plus the rows it dropped, each possibly a new key), and a second retry,
-// never needed in practice, sizes it for every row distinct.
+// Counting: each workgroup aggregates its rows in LDS (plain LDS atomics; the
+// 16 rows a thread loads at once keep HBM busy while they wait): integers
+// near the first row by offset, other keys in a hash table of kHistParts
+// partitions, each key's partition fixed by its hash.  The workgroups write
+// their keys and counts out; the last of them adds them up in LDS if they are
+// few, else k_hist_merge does, one workgroup per partition, so that no key is
+// counted through device-scope atomics.  A column with more distinct keys than these tables
+// hold is counted again into a global open-addressing table (64-bit keys, ~0 =
+// empty).  A value equal to a table's empty marker is counted on the side.
+// Floats count -0.0 with +0.0 (operator==), reporting -0.0 when one was seen
+// (it sorts first in the reference).  A NaN equals nothing, so each NaN row is
+// a bin of count 1: they stay out of the tables, and every workgroup keeps the
+// four smallest (radix order) NaN rows, which is all the top-K can ever take
+// from them.  Columns of a few thousand rows are counted whole in one
+// workgroup's LDS (k_hist_small).  The global table starts at 2n slots (at
+// least 1024, at most 64K); if it ends up more than 70% full the host retries
+// once with a table of twice the keys seen (the exact count, or with a full
+// table the keys seen plus the rows it dropped, each possibly a new key), and
+// a second retry, never needed in practice, sizes it for every row distinct.
+#include <type_traits>
+
 #include "dispatch.h"
 #include "k_common.h"
 #include "kernels.h"
@@ -29,15 +34,15 @@ namespace ddj {
 namespace {
 
 constexpr uint64_t kEmpty = ~0ull;
-constexpr int kLdsSlots = 2048;
 constexpr int kMaxK = 4;
 
+constexpr uint32_t kTooSmall = 1, kNeedMerge = 2;  // HistCtl::overflow
 struct HistCtl {
     unsigned long long distinct;
-    unsigned long long special;  // rows whose 64-bit pattern equals kEmpty
+    unsigned long long special;  // rows whose bit pattern (4- and 8-byte types) marks an empty slot
     unsigned long long nans;     // NaN rows (floats)
-    unsigned long long dropped;  // rows that found no slot in a full table
-    uint32_t overflow;
+    unsigned long long dropped;  // rows that found no slot in a full global table
+    uint32_t overflow;           // kTooSmall: a table was; kNeedMerge
     uint32_t negzero;
 };
 
@@ -60,32 +65,45 @@ template <typename T> __device__ __forceinline__ uint64_t hist_key(T v, bool& ne
     return ubits(v);
 }
 
-// Adds cnt rows of `key` to the global table; returns 1 when the key is new
-// (the caller sums these: a counter bumped once per new key serializes every
-// workgroup on one address, which for a column of 10^4 distinct rows was most
-// of the count's time).
-__device__ uint32_t global_insert(unsigned long long* keys, unsigned long long* counts, uint64_t cap_mask, uint64_t key,
-                                  unsigned long long cnt, HistCtl* ctl) {
-    uint64_t h = hmix(key) & cap_mask;
-    for (uint64_t p = 0; p <= cap_mask && p < 4096; p++) {
-        const uint64_t s = (h + p) & cap_mask;
-        unsigned long long k = __hip_atomic_load(&keys[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (k == key) {
-            atomicAdd(&counts[s], cnt);
-            return 0;
-        }
-        if (k == kEmpty) {
-            unsigned long long prev = atomicCAS(&keys[s], kEmpty, (unsigned long long)key);
-            if (prev == kEmpty || prev == key) {
-                atomicAdd(&counts[s], cnt);
-                return prev == kEmpty ? 1u : 0u;
-            }
-        }
+// The global table.  New keys are counted per thread and summed (a counter
+// bumped once per new key serializes every workgroup on one address, which for
+// a column of 10^4 distinct rows was most of the count's time).  A table that fills is dropped and counted again in a larger one, so a thread that
+// once found no slot (no free one within kProbes: far past what a table
+// 70% full needs) only counts the rows it drops.
+constexpr uint64_t kProbes = 512;
+struct GlobalTable {
+    unsigned long long* keys = nullptr;
+    unsigned long long* counts = nullptr;
+    uint64_t mask = 0;
+    HistCtl* ctl = nullptr;
+    uint32_t fresh = 0;               // keys this thread brought in
+    unsigned long long dropped = 0;   // rows it found no slot for
+    __device__ __forceinline__ uint64_t home(uint64_t key) const { return hmix(key) & mask; }
+    __device__ __forceinline__ unsigned long long peek(uint64_t s) const {
+        return __hip_atomic_load(&keys[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    atomicOr(&ctl->overflow, 1u);
-    atomicAdd(&ctl->dropped, cnt);
-    return 0;
-}
+    __device__ __forceinline__ void add(uint64_t key, unsigned long long cnt) {
+        if (dropped) {
+            dropped += cnt;
+            return;
+        }
+        uint64_t s = home(key);
+        for (uint64_t p = 0; p <= mask && p < kProbes; p++) {
+            unsigned long long seen = peek(s);
+            if (seen == kEmpty) {
+                const unsigned long long prev = atomicCAS(&keys[s], kEmpty, (unsigned long long)key);
+                if (prev == kEmpty) fresh++;
+                seen = prev == kEmpty ? key : prev;
+            }
+            if (seen == key) {
+                atomicAdd(&counts[s], cnt);
+                return;
+            }
+            s = (s + 1) & mask;
+        }
+        dropped += cnt;
+    }
+};
 
 // Ascending list of the (up to) four smallest keys seen, with multiplicity.
 struct Small4 {
@@ -144,177 +162,44 @@ __device__ void block_small4(Small4& s, uint64_t* sm_keys /* NT/kWave * kMaxK */
     }
 }
 
-// LDS slot of a key: a multiplicative hash of its folded halves (cheaper
-// than hmix's 64-bit multiplies, which the global table keeps).
-__device__ __forceinline__ uint32_t lds_slot(uint64_t key) {
+// The counting workgroup's hash table: kHistParts partitions of 192 slots of
+// 4-byte keys (narrower types widened) or 128 of 8-byte keys.  A multiplicative
+// hash of the key's folded halves (cheaper than hmix's 64-bit multiplies, which
+// the other tables keep) gives the partition and the slot to start from;
+// probing stays inside the partition.
+template <typename T> using HistKey = typename std::conditional<sizeof(T) == 8, unsigned long long, uint32_t>::type;
+constexpr int kHistParts = 64;
+template <typename T> constexpr int part_slots() { return sizeof(T) == 8 ? 128 : 192; }
+// A partition written out: the keys in use with their counts, in any order.
+template <typename KT> struct HistEntry {
+    KT key;
+    uint32_t count;
+};
+__device__ __forceinline__ uint32_t lds_hash(uint64_t key) {
     const uint32_t a = (uint32_t)key ^ ((uint32_t)(key >> 32) * 0x85ebca6bu);
-    return (a * 0x9E3779B1u) >> (32 - 11);
+    return a * 0x9E3779B1u;
 }
-static_assert(kLdsSlots == 1 << 11, "lds_slot yields 11 bits");
 
-// The LDS table has 2048 slots.  (8192, a quarter of the CU's LDS, was
-// slower on a long-tailed column of 10^5 distinct values: 420 against 310
-// us for 16M rows, as every workgroup then flushes more keys into the
-// global table, whose device-scope atomics are the cost.)
+// What a counting workgroup saw outside its tables.
+struct HistInfo {
+    unsigned long long special, nans;
+    uint32_t negzero, overflow;
+    uint32_t nan_n, pad;
+    uint64_t nan_keys[kMaxK];
+};
+
 // Workgroups of 1024 threads, one per CU, stride over tiles of 16384 rows,
-// each thread taking 16 rows with 16-byte loads issued together.  Few, big
-// workgroups keep the final flush short: every workgroup adds each of its
-// distinct keys to the global table with a device-scope atomic, and those
-// serialize per key.
+// each thread taking 16 rows with their loads issued together.
 constexpr int kHistThreads = 1024;
 
-// Integer columns: keys within kWindow of the first row's (dictionary codes,
-// categories, most small integers) are counted by their offset, in kCopies
-// copies of the window, lane l in copy l % 32: no key compare, no probing, and
-// no two lanes of a wave on one bank but the pairs that share a copy.  Other
-// keys take the hash table.  The count of the 64M-row Zipf(1.2)/50 column was
-// bound by the probe loop's instructions and the LDS atomics' same-address
-// conflicts (92 us); with the window it takes 54, against 42 for a plain pass
-// over the column.
-constexpr int kWindow = 1024, kCopies = 32;
-
-template <typename T>
-__global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict__ x, size_t n, unsigned long long* keys,
-                                                       unsigned long long* counts, uint64_t cap_mask, HistCtl* ctl,
-                                                       uint64_t* nan_keys /* [grid * 4] */,
-                                                       uint32_t* nan_n /* [grid] */) {
-    __shared__ unsigned long long skey[kLdsSlots];
-    __shared__ uint32_t scnt[kLdsSlots];
-    __shared__ uint64_t s_nk[kHistThreads / kWave * kMaxK];
-    __shared__ int s_nc[kHistThreads / kWave];
-    __shared__ uint32_t s_new;  // keys this workgroup brought into the global table
-    constexpr bool kInt = !std::is_floating_point<T>::value;
-    using U = typename UnsignedOf<T>::type;
-    __shared__ __attribute__((aligned(16))) uint32_t win[kInt ? kWindow * kCopies : 1];
-    const U wbase = kInt ? (U)(ubits(x[0]) - kWindow / 2) : U(0);  // wraps in the type
-    if constexpr (kInt) {
-        u32x4* w4 = reinterpret_cast<u32x4*>(win);
-        for (int i = threadIdx.x; i < kWindow * kCopies / 4; i += kHistThreads) w4[i] = u32x4{0u, 0u, 0u, 0u};
-    }
-    uint32_t fresh = 0;
-    Small4 nan4;
-    unsigned long long nans = 0;
-    for (int i = threadIdx.x; i < kLdsSlots; i += kHistThreads) {
-        skey[i] = kEmpty;
-        scnt[i] = 0;
-    }
-    if (threadIdx.x == 0) s_new = 0;
-    __syncthreads();
-    bool negzero = false;
-    unsigned long long special = 0;
-    // Adds `add` rows of `key` to the LDS table (or, when its probe run is
-    // full, to the global table).
-    auto lds_add = [&](uint64_t key, uint32_t add) {
-        const uint32_t h = lds_slot(key);
-        for (int p = 0; p < 16; p++) {
-            const uint32_t s = (h + p) & (kLdsSlots - 1);
-            unsigned long long k = skey[s];
-            if (k == kEmpty) k = atomicCAS(&skey[s], kEmpty, (unsigned long long)key);
-            if (k == kEmpty || k == key) {
-                atomicAdd(&scnt[s], add);
-                return;
-            }
-        }
-        fresh += global_insert(keys, counts, cap_mask, key, (unsigned long long)add, ctl);
-    };
-    // Two keys per thread counted in registers (the first two distinct keys
-    // the thread meets): on skewed columns most rows hit them and skip the
-    // LDS atomics, whose same-address conflicts are the cost.
-    uint64_t rk0 = kEmpty, rk1 = kEmpty;
-    uint32_t rc0 = 0, rc1 = 0;
-    auto count = [&](T v) {
-        if constexpr (std::is_floating_point<T>::value) {
-            if (v != v) {
-                nan4.insert(order_key(v));
-                nans++;
-                return;
-            }
-        }
-        if constexpr (kInt) {
-            const U off = (U)((U)ubits(v) - wbase);
-            if (sizeof(U) == 1 || (uint64_t)off < (uint64_t)kWindow) {
-                atomicAdd(&win[(uint32_t)off * kCopies + (threadIdx.x & (kCopies - 1))], 1u);
-                return;
-            }
-        }
-        const uint64_t key = hist_key(v, negzero);
-        if (key == kEmpty) {
-            special++;
-            return;
-        }
-        if (key == rk0) {
-            rc0++;
-        } else if (key == rk1) {
-            rc1++;
-        } else if (rk0 == kEmpty) {
-            rk0 = key;
-            rc0 = 1;
-        } else if (rk1 == kEmpty) {
-            rk1 = key;
-            rc1 = 1;
-        } else {
-            lds_add(key, 1u);
-        }
-    };
-    constexpr int kRows = 16 * kHistThreads;
-    constexpr int V = 16 / sizeof(T);
-    constexpr int Q = kRows / V / kHistThreads;  // 16-byte loads per thread and tile
-    const size_t tiles = (n + kRows - 1) / kRows;
-    const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
-    for (size_t t = blockIdx.x; t < tiles; t += gridDim.x) {  // uniform per workgroup
-        const size_t base = t * kRows;
-        if (aligned && base + kRows <= n) {
-            const u32x4* s4 = reinterpret_cast<const u32x4*>(x + base);
-            u32x4 w[Q];
-#pragma unroll
-            for (int q = 0; q < Q; q++) w[q] = s4[threadIdx.x + kHistThreads * q];
-#pragma unroll
-            for (int q = 0; q < Q; q++) {
-                T v[V];
-                __builtin_memcpy(v, &w[q], 16);
-#pragma unroll
-                for (int k = 0; k < V; k++) count(v[k]);
-            }
-        } else {
-            const int cnt = (int)((n - base) < (size_t)kRows ? (n - base) : (size_t)kRows);
-            for (int i = threadIdx.x; i < cnt; i += kHistThreads) count(x[base + i]);
-        }
-    }
-    if (rk0 != kEmpty) lds_add(rk0, rc0);
-    if (rk1 != kEmpty) lds_add(rk1, rc1);
-    __syncthreads();
-    if constexpr (kInt) {
-        // a thread sums one offset's copies, rotated so that the lanes' reads
-        // spread over the banks, and adds the key to the global table
-        static_assert(kWindow == kHistThreads, "one offset a thread");
-        uint32_t c = 0;
-#pragma unroll
-        for (int k = 0; k < kCopies; k++) c += win[threadIdx.x * kCopies + ((threadIdx.x + k) & (kCopies - 1))];
-        if (c) {
-            const uint64_t key = (uint64_t)(U)(wbase + (U)threadIdx.x);
-            if (key == kEmpty)
-                special += c;
-            else
-                fresh += global_insert(keys, counts, cap_mask, key, (unsigned long long)c, ctl);
-        }
-    }
-    for (int s = threadIdx.x; s < kLdsSlots; s += kHistThreads)
-        if (skey[s] != kEmpty) fresh += global_insert(keys, counts, cap_mask, skey[s], scnt[s], ctl);
-    fresh = wave_sum(fresh);
-    if ((threadIdx.x & (kWave - 1)) == 0 && fresh) atomicAdd(&s_new, fresh);
-    __syncthreads();
-    if (threadIdx.x == 0 && s_new) atomicAdd(&ctl->distinct, (unsigned long long)s_new);
-    const uint64_t nz = wave_or((uint64_t)negzero);
-    const unsigned long long sp = wave_sum(special);
-    const unsigned long long nn = wave_sum(nans);
-    if ((threadIdx.x & (kWave - 1)) == 0) {
-        if (nz) atomicOr(&ctl->negzero, 1u);
-        if (sp) atomicAdd(&ctl->special, sp);
-        if (nn) atomicAdd(&ctl->nans, nn);
-    }
-    if constexpr (std::is_floating_point<T>::value)
-        block_small4<kHistThreads>(nan4, s_nk, s_nc, nan_keys + (size_t)blockIdx.x * kMaxK, nan_n + blockIdx.x);
-}
+// Integer columns: keys within kWindow / 2 of the first row's (dictionary
+// codes, categories, most small integers) are counted by their offset, in
+// kCopies copies of the window, lane l in copy l % kCopies: no key compare, no
+// probing, and few lanes of a wave on one bank.  The count of the 64M-row
+// Zipf(1.2)/50 column was bound by the probe loop's instructions and the LDS
+// atomics' same-address conflicts (92 us); with the window it takes 45, against
+// 42 for a plain pass over the column.
+constexpr int kWindow = 1024, kCopies = 8;
 
 struct Cand {
     unsigned long long count;
@@ -402,57 +287,498 @@ template <typename T, int NT = kBlock> __device__ void block_best(Cand* top, int
     __syncthreads();
 }
 
+// The host's result from the best K of the tables (thread 0 of the last
+// workgroup) and the counting workgroups' records: rows of the empty markers'
+// bit pattern (all ones), and every NaN row as a bin of count 1.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_hist_topk(const unsigned long long* keys, const unsigned long long* counts,
-                                                      uint64_t cap, int K, Cand* partials, uint32_t* tickets,
-                                                      const HistCtl* ctl, const uint64_t* nan_keys,
-                                                      const uint32_t* nan_n, uint32_t nan_blocks, HostOut host) {
-    __shared__ Cand sc[kBlock / kWave * kMaxK];
-    __shared__ Cand best[kMaxK];
-    __shared__ bool last;
-    Cand top[kMaxK];
+__device__ void finish_topk(const Cand* best, int K, HistCtl ctl, const HistInfo* info, uint32_t blocks, HistResult* out) {
+    Cand b[kMaxK];
+#pragma unroll
+    for (int i = 0; i < kMaxK; i++) b[i] = i < K ? best[i] : Cand{0, 0};
+    if (ctl.special) push<T>(b, K, Cand{ctl.special, (uint64_t)(HistKey<T>)~(HistKey<T>)0});
+    if (std::is_floating_point<T>::value && ctl.nans)
+        for (uint32_t g = 0; g < blocks; g++)
+            for (uint32_t r = 0, nr = ld_agent(&info[g].nan_n); r < nr; r++)
+                push<T>(b, K, Cand{1ull, ubits(from_order_key<T>(ld_agent(&info[g].nan_keys[r])))});
+    out->ctl = ctl;
+#pragma unroll
+    for (int i = 0; i < kMaxK; i++) out->top[i] = b[i];
+}
+
+// The counting workgroups' records summed into ctl (LDS), by one workgroup.
+template <int NT> __device__ __forceinline__ void fold_info(const HistInfo* info, uint32_t blocks, HistCtl* ctl) {
+    for (uint32_t g = threadIdx.x; g < blocks; g += NT) {
+        const unsigned long long special = ld_agent(&info[g].special), nans = ld_agent(&info[g].nans);
+        const uint32_t negzero = ld_agent(&info[g].negzero), over = ld_agent(&info[g].overflow);
+        if (special) atomicAdd(&ctl->special, special);
+        if (nans) atomicAdd(&ctl->nans, nans);
+        if (negzero) atomicOr(&ctl->negzero, 1u);
+        if (over) atomicOr(&ctl->overflow, kTooSmall);
+    }
+}
+
+// A table's entries into sorted lists of K, a list a thread, and the keys
+// counted into *distinct.
+template <typename T, int SLOTS, int NT, typename KT, typename CT>
+__device__ __forceinline__ void take_table(const KT* skey, const CT* scnt, Cand* top, int K, uint32_t* distinct) {
 #pragma unroll
     for (int i = 0; i < kMaxK; i++) top[i] = Cand{0, 0};
-    const size_t stride = (size_t)gridDim.x * kBlock;
-    for (size_t s = (size_t)blockIdx.x * kBlock + threadIdx.x; s < cap; s += stride) {
-        const uint64_t k = keys[s];
-        if (k != kEmpty) push<T>(top, K, Cand{counts[s], k});
+    uint32_t d = 0;
+    for (int s = threadIdx.x; s < SLOTS; s += NT)
+        if (scnt[s]) {
+            d++;
+            push<T>(top, K, Cand{scnt[s], (uint64_t)skey[s]});
+        }
+    d = wave_sum(d);
+    if ((threadIdx.x & (kWave - 1)) == 0 && d) atomicAdd(distinct, d);
+}
+
+// The segment that entry e lies in: first[s] <= e < first[s + 1].
+__device__ __forceinline__ uint32_t segment_of(const uint32_t* first, uint32_t segments, uint32_t e) {
+    uint32_t lo = 0, hi = segments;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (first[mid] <= e)
+            lo = mid;
+        else
+            hi = mid;
     }
-    block_best<T>(top, K, sc, best);
+    return lo;
+}
+
+// GLOBAL: the tables are flushed into, and keys without a slot added to, the
+// global table, which k_hist_topk searches.  Else the workgroup's used slots
+// go to segs (its kHistParts * part_slots entries from blockIdx.x on, partition
+// by partition, partition p from off[p * grid + workgroup] on), and a key
+// without a slot ends the count (info[].overflow: the host counts again with
+// GLOBAL).  With a tail, if all workgroups' entries are few (columns of few
+// distinct values), the last workgroup adds them up itself and hands the best K
+// to the host; else (kNeedMerge) k_hist_merge does.
+constexpr uint32_t kTailEntries = 8192;
+struct HistTail {
+    uint32_t* tickets = nullptr;
+    int K = 0;
+    HostOut host;
+};
+template <typename T, bool GLOBAL>
+__global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict__ x, size_t n, GlobalTable table,
+                                                             HistEntry<HistKey<T>>* __restrict__ segs,
+                                                             uint32_t* __restrict__ off, HistInfo* __restrict__ info,
+                                                             HistTail tail) {
+    using KT = HistKey<T>;
+    constexpr KT kFree = (KT)~(KT)0;  // an empty slot; rows of that bit pattern are counted on the side
+    constexpr int PS = part_slots<T>(), kLdsSlots = kHistParts * PS;
+    __shared__ __attribute__((aligned(16))) KT skey[kLdsSlots];
+    __shared__ __attribute__((aligned(16))) uint32_t scnt[kLdsSlots];
+    __shared__ uint64_t s_nk[kHistThreads / kWave * kMaxK];
+    __shared__ int s_nc[kHistThreads / kWave];
+    __shared__ uint32_t s_new;   // keys this workgroup brought into the global table
+    __shared__ uint32_t s_over;  // a key found no slot
+    __shared__ unsigned long long s_special, s_nans;
+    __shared__ uint32_t s_negzero;
+    constexpr bool kInt = !std::is_floating_point<T>::value;
+    using U = typename UnsignedOf<T>::type;
+    __shared__ __attribute__((aligned(16))) uint32_t win[kInt ? kWindow * kCopies : 4];
+    const U wbase = kInt ? (U)(ubits(x[0]) - kWindow / 2) : U(0);  // wraps in the type
+    auto fill = [](void* p, int bytes, uint32_t v) {
+        u32x4* q = reinterpret_cast<u32x4*>(p);
+        for (int i = threadIdx.x; i < bytes / 16; i += kHistThreads) q[i] = u32x4{v, v, v, v};
+    };
+    if (kInt) fill(win, sizeof win, 0u);
+    fill(skey, sizeof skey, ~0u);
+    fill(scnt, sizeof scnt, 0u);
+    if (threadIdx.x == 0) {
+        s_new = s_over = s_negzero = 0;
+        s_special = s_nans = 0;
+    }
+    __syncthreads();
+    Small4 nan4;
+    unsigned long long special = 0, nans = 0;
+    bool negzero = false;
+    // Adds `add` rows of `key` to its partition; a key without a slot goes to
+    // the global table, or ends the count.
+    auto lds_add = [&](KT key, uint32_t add) {
+        const uint64_t at = (uint64_t)lds_hash((uint64_t)key) * kHistParts;
+        const uint32_t base = (uint32_t)(at >> 32) * PS;
+        uint32_t h = (uint32_t)(((uint64_t)(uint32_t)at * PS) >> 32);
+        for (int p = 0; p < 24; p++) {
+            const uint32_t s = base + h;
+            h = h + 1 < (uint32_t)PS ? h + 1 : 0;
+            KT k = skey[s];
+            if (k == kFree) k = atomicCAS(&skey[s], kFree, key);
+            if (k == kFree || k == key) {
+                atomicAdd(&scnt[s], add);
+                return;
+            }
+        }
+        if (GLOBAL)
+            table.add((uint64_t)key, add);
+        else
+            s_over = 1;
+    };
+    // Two keys per thread counted in registers (the first two distinct keys
+    // the thread meets): on skewed columns most rows hit them and skip the
+    // LDS atomics, whose same-address conflicts are the cost.
+    KT rk0 = kFree, rk1 = kFree;
+    uint32_t rc0 = 0, rc1 = 0;
+    auto count = [&](T v) {
+        if constexpr (std::is_floating_point<T>::value) {
+            if (v != v) {
+                nan4.insert(order_key(v));
+                nans++;
+                return;
+            }
+        }
+        if constexpr (kInt) {
+            const U off = (U)((U)ubits(v) - wbase);
+            if (sizeof(U) == 1 || (uint64_t)off < (uint64_t)kWindow) {
+                atomicAdd(&win[(uint32_t)off * kCopies + (threadIdx.x & (kCopies - 1))], 1u);
+                return;
+            }
+        }
+        const KT key = (KT)hist_key(v, negzero);
+        if (key == kFree) {
+            special++;
+            return;
+        }
+        if (key == rk0) {
+            rc0++;
+        } else if (key == rk1) {
+            rc1++;
+        } else if (rk0 == kFree) {
+            rk0 = key;
+            rc0 = 1;
+        } else if (rk1 == kFree) {
+            rk1 = key;
+            rc1 = 1;
+        } else {
+            lds_add(key, 1u);
+        }
+    };
+    constexpr int kPer = 16, kRows = kPer * kHistThreads;
+    constexpr int V = 16 / sizeof(T);
+    constexpr int Q = kRows / V / kHistThreads;  // 16-byte loads per thread and tile
+    const size_t tiles = (n + kRows - 1) / kRows;
+    const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+    for (size_t t = blockIdx.x; t < tiles; t += gridDim.x) {  // uniform per workgroup
+        if (!GLOBAL && *(volatile uint32_t*)&s_over) break;  // (each wave by itself: the count is dropped)
+        const size_t base = t * kRows;
+        if (aligned && base + kRows <= n) {
+            const u32x4* s4 = reinterpret_cast<const u32x4*>(x + base);
+            u32x4 w[Q];
+#pragma unroll
+            for (int q = 0; q < Q; q++) w[q] = s4[threadIdx.x + kHistThreads * q];
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                T v[V];
+                __builtin_memcpy(v, &w[q], 16);
+#pragma unroll
+                for (int k = 0; k < V; k++) count(v[k]);
+            }
+        } else {
+            const int cnt = (int)((n - base) < (size_t)kRows ? (n - base) : (size_t)kRows);
+            T v[kPer];
+#pragma unroll
+            for (int k = 0; k < kPer; k++) {
+                const int i = threadIdx.x + k * kHistThreads;
+                if (i < cnt) v[k] = x[base + i];
+            }
+#pragma unroll
+            for (int k = 0; k < kPer; k++)
+                if ((int)threadIdx.x + k * kHistThreads < cnt) count(v[k]);
+        }
+    }
+    if (rk0 != kFree) lds_add(rk0, rc0);
+    if (rk1 != kFree) lds_add(rk1, rc1);
+    __syncthreads();
+    if constexpr (kInt) {
+        // a thread sums one offset's copies and adds its key to the table
+        static_assert(kWindow == kHistThreads, "one offset a thread");
+        uint32_t c = 0;
+#pragma unroll
+        for (int k = 0; k < kCopies; k++) c += win[threadIdx.x * kCopies + ((threadIdx.x + k) & (kCopies - 1))];
+        if (c) {
+            const KT key = (KT)(U)(wbase + (U)threadIdx.x);
+            if (key == kFree)
+                special += c;
+            else
+                lds_add(key, c);
+        }
+        __syncthreads();
+    }
+    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    if (GLOBAL) {
+        for (int s = threadIdx.x; s < kLdsSlots; s += kHistThreads)
+            if (skey[s] != kFree) table.add((uint64_t)skey[s], scnt[s]);
+        const uint32_t fresh = wave_sum(table.fresh);
+        const unsigned long long dropped = wave_sum(table.dropped);
+        if (lane == 0) {
+            if (fresh) atomicAdd(&s_new, fresh);
+            if (dropped) {
+                atomicOr(&table.ctl->overflow, 1u);
+                atomicAdd(&table.ctl->dropped, dropped);
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x == 0 && s_new) atomicAdd(&table.ctl->distinct, (unsigned long long)s_new);
+    } else {
+        // partitions' used slots, where each begins, then the entries
+        __shared__ uint32_t s_off[kHistParts + 1];
+        static_assert(kHistParts == kWave && PS % kWave == 0, "a partition a lane, whole waves of slots");
+        constexpr int C = PS / kWave;  // slots a lane
+        for (int p = wid; p < kHistParts; p += kHistThreads / kWave) {
+            uint32_t used = 0;
+#pragma unroll
+            for (int q = 0; q < C; q++) used += __popcll(__ballot(scnt[p * PS + lane + q * kWave] != 0));
+            if (lane == 0) s_off[p] = used;
+        }
+        __syncthreads();
+        if (wid == 0) {
+            const uint32_t used = s_off[lane], upto = wave_inclusive_scan(used);
+            s_off[lane] = upto - used;
+            if (lane == kWave - 1) s_off[kHistParts] = upto;
+        }
+        __syncthreads();
+        HistEntry<KT>* mine = segs + (size_t)blockIdx.x * kLdsSlots;
+        for (int p = wid; p < kHistParts; p += kHistThreads / kWave) {
+            uint32_t at = s_off[p];
+#pragma unroll
+            for (int q = 0; q < C; q++) {
+                const KT k = skey[p * PS + lane + q * kWave];
+                const uint32_t c = scnt[p * PS + lane + q * kWave];
+                const uint64_t has = __ballot(c != 0);
+                if (c) {
+                    HistEntry<KT>* e = mine + at + __popcll(has & ((1ull << lane) - 1));
+                    st_agent(&e->key, k);
+                    st_agent(&e->count, c);
+                }
+                at += __popcll(has);
+            }
+        }
+        for (int p = threadIdx.x; p <= kHistParts; p += kHistThreads) st_agent(&off[(size_t)p * gridDim.x + blockIdx.x], s_off[p]);
+    }
+    const bool nz = __ballot(negzero) != 0;
+    special = wave_sum(special);
+    nans = wave_sum(nans);
+    if (lane == 0) {
+        if (nz) atomicOr(&s_negzero, 1u);
+        if (special) atomicAdd(&s_special, special);
+        if (nans) atomicAdd(&s_nans, nans);
+    }
+    HistInfo* me = info + blockIdx.x;
+    __shared__ uint64_t nan_keys[kMaxK];
+    __shared__ uint32_t nan_n;
+    if (threadIdx.x == 0) nan_n = 0;
+    __syncthreads();
+    if constexpr (std::is_floating_point<T>::value) block_small4<kHistThreads>(nan4, s_nk, s_nc, nan_keys, &nan_n);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        st_agent(&me->special, s_special);
+        st_agent(&me->nans, s_nans);
+        st_agent(&me->negzero, s_negzero);
+        st_agent(&me->overflow, s_over);
+        st_agent(&me->nan_n, nan_n);
+        for (uint32_t r = 0; r < nan_n; r++) st_agent(&me->nan_keys[r], nan_keys[r]);
+    }
+    if constexpr (!GLOBAL) {
+        __shared__ bool last;
+        if (!tail.tickets || !last_of_grid(tail.tickets, &last)) return;
+        // every workgroup's entries: how many, and where they begin
+        __shared__ uint32_t first[kHistThreads + 1];
+        __shared__ uint32_t red[kHistThreads / kWave];
+        __shared__ HistCtl ctl;
+        __shared__ uint32_t s_distinct;
+        __shared__ Cand sc[kHistThreads / kWave * kMaxK];
+        __shared__ Cand best[kMaxK];
+        const uint32_t blocks = gridDim.x;  // <= kHistThreads
+        const uint32_t have = threadIdx.x < blocks ? ld_agent(&off[(size_t)kHistParts * blocks + threadIdx.x]) : 0u;
+        if (threadIdx.x == 0) {
+            ctl = HistCtl{};
+            s_distinct = 0;
+        }
+        fill(skey, sizeof skey, ~0u);
+        fill(scnt, sizeof scnt, 0u);
+        uint32_t total;
+        first[threadIdx.x] = block_exclusive_scan<uint32_t, kHistThreads>(have, &total, red);
+        __syncthreads();
+        fold_info<kHistThreads>(info, blocks, &ctl);
+        HistResult* out = reinterpret_cast<HistResult*>(tail.host.dst);
+        const bool few = total <= kTailEntries && n < (1ull << 32);
+        if (few)
+            for (uint32_t e = threadIdx.x; e < total; e += kHistThreads) {
+                const uint32_t w = segment_of(first, blocks, e);
+                const HistEntry<KT>* en = segs + (size_t)w * kLdsSlots + (e - first[w]);
+                const KT key = ld_agent(&en->key);
+                const uint32_t c = ld_agent(&en->count);
+                uint32_t s = (uint32_t)(((uint64_t)lds_hash((uint64_t)key) * kLdsSlots) >> 32);
+                int left = 256;
+                for (; left > 0; left--) {
+                    KT k = skey[s];
+                    if (k == kFree) k = atomicCAS(&skey[s], kFree, key);
+                    if (k == kFree || k == key) {
+                        atomicAdd(&scnt[s], c);
+                        break;
+                    }
+                    s = s + 1 < (uint32_t)kLdsSlots ? s + 1 : 0;
+                }
+                if (left == 0) atomicOr(&ctl.overflow, kNeedMerge);
+            }
+        else if (threadIdx.x == 0)
+            atomicOr(&ctl.overflow, kNeedMerge);
+        __syncthreads();
+        if (ctl.overflow) {  // uniform
+            if (threadIdx.x == 0) out->ctl = ctl;
+        } else {
+            Cand top[kMaxK];
+            take_table<T, kLdsSlots, kHistThreads>(skey, scnt, top, tail.K, &s_distinct);
+            block_best<T, kHistThreads>(top, tail.K, sc, best);  // its barriers complete s_distinct
+            if (threadIdx.x == 0) {
+                ctl.distinct = s_distinct;
+                finish_topk<T>(best, tail.K, ctl, info, blocks, out);
+            }
+        }
+        host_out_done(tail.host);
+    }
+}
+
+// The best K over all workgroups, from the K each has in best: partials by
+// tickets, and the last workgroup takes the best of them into best.  Whether
+// this is that workgroup.
+template <typename T, int NT>
+__device__ __forceinline__ bool best_of_grid(Cand* top, int K, Cand* sc, Cand* best, Cand* partials, uint32_t* tickets,
+                                             bool* last) {
     if (threadIdx.x < K) {
         st_agent(reinterpret_cast<uint64_t*>(&partials[blockIdx.x * K + threadIdx.x].count),
                  (uint64_t)best[threadIdx.x].count);
         st_agent(&partials[blockIdx.x * K + threadIdx.x].key, best[threadIdx.x].key);
     }
-    if (!last_of_grid(tickets, &last)) return;
-    // the last workgroup takes the best of every workgroup's list
+    if (!last_of_grid(tickets, last)) return false;
 #pragma unroll
     for (int i = 0; i < kMaxK; i++) top[i] = Cand{0, 0};
-    for (uint32_t i = threadIdx.x; i < gridDim.x * (uint32_t)K; i += kBlock) {
+    for (uint32_t i = threadIdx.x; i < gridDim.x * (uint32_t)K; i += NT) {
         Cand c;
         c.count = __hip_atomic_load(&partials[i].count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         c.key = __hip_atomic_load(&partials[i].key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         push<T>(top, K, c);
     }
-    block_best<T>(top, K, sc, best);
-    if (threadIdx.x == 0) {
-        Cand b[kMaxK];
-#pragma unroll
-        for (int i = 0; i < kMaxK; i++) b[i] = i < K ? best[i] : Cand{0, 0};
-        if (ctl->special) push<T>(b, K, Cand{ctl->special, kEmpty});
-        if constexpr (std::is_floating_point<T>::value) {
-            if (ctl->nans)  // every NaN row is a bin of count 1
-                for (uint32_t g = 0; g < nan_blocks; g++)
-                    for (uint32_t r = 0; r < nan_n[g]; r++) {
-                        const T v = from_order_key<T>(nan_keys[(size_t)g * kMaxK + r]);
-                        push<T>(b, K, Cand{1ull, ubits(v)});
-                    }
-        }
-        HistResult* out = reinterpret_cast<HistResult*>(host.dst);
-        out->ctl = *ctl;
-#pragma unroll
-        for (int i = 0; i < kMaxK; i++) out->top[i] = b[i];
+    block_best<T, NT>(top, K, sc, best);
+    return true;
+}
+
+// One workgroup per partition: the counting workgroups' entries added up in an
+// LDS table (an entry a thread, several in flight), then the best K.  Replaces
+// a global table that every workgroup flushed its keys into with device-scope
+// atomics, the launch that cleared it and the one that searched its 64K slots:
+// 5M rows of long-tailed volumes 2 + 72 + 11 us, now 20 + 22; 16M rows, whose
+// table overflowed and was counted again, 2.5 ms, now 38 + 32 us.
+constexpr int kMergeThreads = 1024, kMergeSlots = 4096;
+template <typename T>
+__global__ __launch_bounds__(kMergeThreads) void k_hist_merge(const HistEntry<HistKey<T>>* __restrict__ segs,
+                                                              const uint32_t* __restrict__ off,
+                                                              const HistInfo* __restrict__ info, uint32_t blocks, int K,
+                                                              Cand* partials, uint32_t* part_ctl, uint32_t* tickets,
+                                                              HostOut host) {
+    using KT = HistKey<T>;
+    constexpr KT kFree = (KT)~(KT)0;
+    constexpr int kSegSlots = kHistParts * part_slots<T>(), W = kMergeThreads / kWave;
+    __shared__ __attribute__((aligned(16))) KT skey[kMergeSlots];
+    __shared__ unsigned long long scnt[kMergeSlots];
+    __shared__ Cand sc[W * kMaxK];
+    __shared__ Cand best[kMaxK];
+    __shared__ HistCtl ctl;
+    __shared__ uint32_t s_distinct, s_over;
+    __shared__ uint32_t first[kMergeThreads];  // of the partition's entries, where each workgroup's begin
+    __shared__ uint32_t begin[kMergeThreads];  // and where they are among the workgroup's
+    __shared__ uint32_t red[W];
+    __shared__ bool last;
+    const uint32_t* row = off + (size_t)blockIdx.x * blocks;  // blocks <= kMergeThreads
+    const uint32_t at = threadIdx.x < blocks ? row[threadIdx.x] : 0u;
+    const uint32_t mine = threadIdx.x < blocks ? row[blocks + threadIdx.x] - at : 0u;
+    for (int i = threadIdx.x; i < kMergeSlots; i += kMergeThreads) {
+        skey[i] = kFree;
+        scnt[i] = 0;
     }
+    if (threadIdx.x == 0) {
+        s_distinct = s_over = 0;
+        ctl = HistCtl{};
+    }
+    uint32_t total;
+    first[threadIdx.x] = block_exclusive_scan<uint32_t, kMergeThreads>(mine, &total, red);
+    begin[threadIdx.x] = at;
+    __syncthreads();
+    const int lane = threadIdx.x & (kWave - 1);
+    constexpr int F = 4;  // entries in flight a thread
+    for (uint32_t e0 = threadIdx.x; e0 < total; e0 += F * kMergeThreads) {
+        HistEntry<KT> en[F];
+#pragma unroll
+        for (int f = 0; f < F; f++) {
+            const uint32_t e = e0 + f * kMergeThreads;
+            en[f].count = 0;
+            if (e < total) {
+                const uint32_t w = segment_of(first, blocks, e);
+                en[f] = segs[(size_t)w * kSegSlots + begin[w] + (e - first[w])];
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < F; f++) {
+            if (!en[f].count) continue;
+            uint32_t s = (uint32_t)hmix((uint64_t)en[f].key) & (kMergeSlots - 1);
+            int left = 256;  // past 90% full the count runs again with the global table
+            for (; left > 0; left--) {
+                KT have = skey[s];
+                if (have == kFree) have = atomicCAS(&skey[s], kFree, en[f].key);
+                if (have == kFree || have == en[f].key) {
+                    atomicAdd(&scnt[s], (unsigned long long)en[f].count);
+                    break;
+                }
+                s = (s + 1) & (kMergeSlots - 1);
+            }
+            if (left == 0) s_over = 1;
+        }
+        if (*(volatile uint32_t*)&s_over) break;  // the count is dropped
+    }
+    __syncthreads();
+    Cand top[kMaxK];
+    take_table<T, kMergeSlots, kMergeThreads>(skey, scnt, top, K, &s_distinct);
+    block_best<T, kMergeThreads>(top, K, sc, best);  // its barriers complete s_distinct
+    if (threadIdx.x == 0) {
+        st_agent(&part_ctl[2 * blockIdx.x], s_distinct);
+        st_agent(&part_ctl[2 * blockIdx.x + 1], s_over);
+    }
+    if (!best_of_grid<T, kMergeThreads>(top, K, sc, best, partials, tickets, &last)) return;
+    for (uint32_t i = threadIdx.x; i < gridDim.x; i += kMergeThreads) {
+        atomicAdd(&ctl.distinct, (unsigned long long)ld_agent(&part_ctl[2 * i]));
+        if (ld_agent(&part_ctl[2 * i + 1])) atomicOr(&ctl.overflow, kTooSmall);
+    }
+    fold_info<kMergeThreads>(info, blocks, &ctl);
+    __syncthreads();
+    if (threadIdx.x == 0) finish_topk<T>(best, K, ctl, info, blocks, reinterpret_cast<HistResult*>(host.dst));
+    host_out_done(host);
+}
+
+// The best K of the global table.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_hist_topk(GlobalTable table, int K, Cand* partials, uint32_t* tickets,
+                                                      const HistInfo* info, uint32_t blocks, HostOut host) {
+    __shared__ Cand sc[kBlock / kWave * kMaxK];
+    __shared__ Cand best[kMaxK];
+    __shared__ HistCtl ctl;
+    __shared__ bool last;
+    Cand top[kMaxK];
+#pragma unroll
+    for (int i = 0; i < kMaxK; i++) top[i] = Cand{0, 0};
+    const size_t stride = (size_t)gridDim.x * kBlock;
+    for (size_t s = (size_t)blockIdx.x * kBlock + threadIdx.x; s <= table.mask; s += stride) {
+        const uint64_t k = table.keys[s];
+        if (k != kEmpty) push<T>(top, K, Cand{table.counts[s], k});
+    }
+    block_best<T>(top, K, sc, best);
+    if (!best_of_grid<T, kBlock>(top, K, sc, best, partials, tickets, &last)) return;
+    if (threadIdx.x == 0) ctl = *table.ctl;
+    __syncthreads();
+    fold_info<kBlock>(info, blocks, &ctl);
+    __syncthreads();
+    if (threadIdx.x == 0) finish_topk<T>(best, K, ctl, info, blocks, reinterpret_cast<HistResult*>(host.dst));
     host_out_done(host);
 }
 
@@ -468,7 +794,7 @@ template <typename T> constexpr size_t small_rows() { return sizeof(T) == 8 ? 10
 
 template <typename T>
 __global__ __launch_bounds__(kHistThreads) void k_hist_small(const T* __restrict__ x, uint32_t n, int K, HostOut host) {
-    using KT = typename std::conditional<sizeof(T) == 8, unsigned long long, uint32_t>::type;
+    using KT = HistKey<T>;
     constexpr KT kFree = (KT)~(KT)0;  // an empty slot; rows of that bit pattern are counted on the side
     constexpr int S = small_slots<T>(), W = kHistThreads / kWave;
     __shared__ KT skey[S];
@@ -505,12 +831,11 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_small(const T* __restrict
             }
         }
         const KT key = (KT)hist_key(v[r], negzero);
-        if (key == kFree && sizeof(T) >= 4) {
+        if (key == kFree) {
             special++;
             continue;
         }
-        const uint32_t a = (uint32_t)key ^ ((uint32_t)((uint64_t)key >> 32) * 0x85ebca6bu);
-        uint32_t s = (uint32_t)(((uint64_t)(a * 0x9E3779B1u) * S) >> 32);
+        uint32_t s = (uint32_t)(((uint64_t)lds_hash((uint64_t)key) * S) >> 32);
         // at most n < S keys: a free slot or the key itself is always found
         for (;;) {
             KT k = skey[s];
@@ -611,32 +936,68 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
             memcpy(&found, wait_host_out(c, ho), sizeof found);
             return take(found);
         }
+        size_t g = (n + 16 * kHistThreads - 1) / (16 * kHistThreads);  // at most one workgroup per tile and per CU
+        g = std::max<size_t>(1, std::min<size_t>(g, (size_t)c->cu_count));
+        DevBuf info(c, sizeof(HistInfo) * g);
+        auto xs = static_cast<const T*>(x);
+        {
+            using Entry = HistEntry<HistKey<T>>;
+            DevBuf segs(c, sizeof(Entry) * part_slots<T>() * kHistParts * g), off(c, 4 * (kHistParts + 1) * g);
+            // up to 64 workgroups (1M rows) the last of them merges (50 codes:
+            // one launch of 22 us for two of 9 + 16); more of them have too many
+            // entries for one workgroup (64M rows 70 us, two launches 45 + 19)
+            HistTail tail;
+            if (g <= 64) tail = HistTail{c->control->tickets, K, host_out(c)};
+            {
+                KernelTimer kt_(c, "k_hist_count");
+                hipLaunchKernelGGL((k_hist_count<T, false>), dim3((unsigned)g), dim3(kHistThreads), 0, c->stream, xs, n,
+                                   GlobalTable{}, segs.get<Entry>(), off.get<uint32_t>(), info.get<HistInfo>(), tail);
+            }
+            HIPC(hipGetLastError());
+            if (tail.tickets) memcpy(&found, wait_host_out(c, tail.host), sizeof found);
+            if (!tail.tickets || found.ctl.overflow == kNeedMerge) {
+                DevBuf partials(c, sizeof(Cand) * K * kHistParts), part_ctl(c, 8 * kHistParts);
+                const HostOut ho = host_out(c);
+                {
+                    KernelTimer kt_(c, "k_hist_merge");
+                    hipLaunchKernelGGL(k_hist_merge<T>, dim3(kHistParts), dim3(kMergeThreads), 0, c->stream,
+                                       segs.get<Entry>(), off.get<uint32_t>(), info.get<HistInfo>(), (uint32_t)g, K,
+                                       partials.get<Cand>(), part_ctl.get<uint32_t>(), c->control->tickets, ho);
+                }
+                HIPC(hipGetLastError());
+                memcpy(&found, wait_host_out(c, ho), sizeof found);
+            }
+            if (!found.ctl.overflow) return take(found);
+        }
+        // more distinct keys than the LDS tables hold
         const uint64_t all_distinct = pow2_at_least(2 * (uint64_t)n + 2);
         uint64_t cap = std::min<uint64_t>(std::max<uint64_t>(1024, all_distinct), 1u << 16);
         for (int attempt = 0; attempt < 3; attempt++) {
             DevBuf keys(c, 8 * cap), counts(c, 8 * cap), ctl(c, sizeof(HistCtl));
+            const GlobalTable table{keys.get<unsigned long long>(), counts.get<unsigned long long>(), cap - 1,
+                                    ctl.get<HistCtl>()};
             const unsigned fg = (unsigned)std::min<uint64_t>((cap + kBlock - 1) / kBlock, (uint64_t)c->cu_count * 16);
             {
                 KernelTimer kt_(c, "k_hist_init");
-                hipLaunchKernelGGL(k_hist_init, dim3(fg), dim3(kBlock), 0, c->stream, keys.get<unsigned long long>(),
-                                   counts.get<unsigned long long>(), cap, ctl.get<HistCtl>());
+                hipLaunchKernelGGL(k_hist_init, dim3(fg), dim3(kBlock), 0, c->stream, table.keys, table.counts, cap,
+                                   table.ctl);
             }
-            size_t g = (n + 16 * kHistThreads - 1) / (16 * kHistThreads);  // at most one workgroup per tile and per CU
-            g = std::max<size_t>(1, std::min<size_t>(g, (size_t)c->cu_count));
-            DevBuf nan_keys(c, 8 * kMaxK * g), nan_n(c, 4 * g);
-            { KernelTimer kt_(c, "k_hist_count"); hipLaunchKernelGGL(k_hist_count<T>, dim3((unsigned)g), dim3(kHistThreads), 0, c->stream,
-                               static_cast<const T*>(x), n, keys.get<unsigned long long>(),
-                               counts.get<unsigned long long>(), cap - 1, ctl.get<HistCtl>(),
-                               nan_keys.get<uint64_t>(), nan_n.get<uint32_t>()); }
+            {
+                KernelTimer kt_(c, "k_hist_count");
+                hipLaunchKernelGGL((k_hist_count<T, true>), dim3((unsigned)g), dim3(kHistThreads), 0, c->stream, xs, n,
+                                   table, nullptr, nullptr, info.get<HistInfo>(), HistTail{});
+            }
             HIPC(hipGetLastError());
             // the top-K runs before the table's state is known, so that one
             // result brings both (it is dropped if the table filled)
             const unsigned tg = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((cap + kBlock - 1) / kBlock, 128));
             DevBuf partials(c, sizeof(Cand) * K * tg);
             const HostOut ho = host_out(c);
-            { KernelTimer kt_(c, "k_hist_topk"); hipLaunchKernelGGL(k_hist_topk<T>, dim3(tg), dim3(kBlock), 0, c->stream, keys.get<unsigned long long>(),
-                               counts.get<unsigned long long>(), cap, K, partials.get<Cand>(), c->control->tickets,
-                               ctl.get<HistCtl>(), nan_keys.get<uint64_t>(), nan_n.get<uint32_t>(), (uint32_t)g, ho); }
+            {
+                KernelTimer kt_(c, "k_hist_topk");
+                hipLaunchKernelGGL(k_hist_topk<T>, dim3(tg), dim3(kBlock), 0, c->stream, table, K, partials.get<Cand>(),
+                                   c->control->tickets, info.get<HistInfo>(), (uint32_t)g, ho);
+            }
             HIPC(hipGetLastError());
             memcpy(&found, wait_host_out(c, ho), sizeof found);
             const HistCtl& h = found.ctl;

@@ -69,9 +69,9 @@ def _top(x, k):
     return [int(v[i]) for i in np.lexsort((v, -c))[:k]]
 
 
-# 2048 LDS slots a workgroup, 16384 rows a workgroup, 64K slots in the first
-# global table (70% of it full makes the count run again)
-@pytest.mark.parametrize("distinct", [1, 3, 4, 63, 2_047, 2_048, 2_049, 45_875, 45_876, 70_000, 300_000])
+# 16384 rows a workgroup, 12288 LDS slots (6144 of 8 bytes), 64K slots in the
+# first global table (70% of it full makes the count run again)
+@pytest.mark.parametrize("distinct", [1, 3, 4, 63, 2_049, 6_144, 12_289, 45_875, 45_876, 70_000, 300_000])
 @pytest.mark.parametrize("dtype", [g.D_INT, g.D_TIME])
 def test_most_frequent(ctx, dtype, distinct):
     npdt = g.NP_DTYPE[dtype]
@@ -199,3 +199,18 @@ def test_most_frequent_at_the_window_edges(ctx, dtype, edge):
         x[1:] = np.random.default_rng(2).permutation(x[1:])
         outs = [o.to_bytes() for o in g.Encoding(ctx, g.DICT).Encode(ctx.upload(x), dtype)]
         assert outs == O.encode(g.DICT, dtype, x)
+
+
+@pytest.mark.parametrize("dtype,per_tile", [(g.D_INT, 5_000), (g.D_TIME, 2_500)])
+@pytest.mark.parametrize("tiles", [40, 257])
+def test_most_frequent_many_keys_in_few_rows(ctx, dtype, per_tile, tiles):
+    """Every 16384-row tile has keys of its own: they fit the workgroups' tables,
+    and with 257 tiles (the last one a second tile of the first workgroup)
+    not the partitions' sums."""
+    npdt = g.NP_DTYPE[dtype]
+    row = np.arange(tiles * 16_384)
+    x = ((row // 16_384) * per_tile + row % per_tile).astype(npdt) * npdt(1_003)
+    x[::97] = -5
+    x[1::1_009] = 77
+    meta = g.Encoding(ctx, g.DICT).Encode(ctx.upload(x), dtype)[1].to_bytes()
+    assert sorted(np.frombuffer(meta[16:16 + 4 * npdt().itemsize], npdt)) == sorted(_top(x, 4))
