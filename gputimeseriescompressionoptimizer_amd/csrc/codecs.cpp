@@ -765,7 +765,15 @@ PatchAflParts patch_afl_encode(Ctx* c, int dtype, DView in, bool outside) {
     return out;
 }
 
-Part delta_afl_decode(Ctx* c, int dtype, DView dmeta, DView ameta, DView data) {
+int float_to_int_precision(Ctx* c, DView meta) {
+    if (meta.n < 4) fail(DDJ_ECORRUPT, "floatToInt metadata shorter than 4 bytes");
+    const int32_t p = read_dev<int32_t>(c, meta.p);
+    if (p < 0) fail(DDJ_ECORRUPT, "negative precision");
+    return p;
+}
+
+Part delta_afl_decode(Ctx* c, int dtype, DView dmeta, DView ameta, DView data, DView scale_meta, int float_dtype,
+                      int precision) {
     const size_t es = dtype_size(dtype);
     if (dmeta.n < es) fail(DDJ_ECORRUPT, "delta metadata shorter than one value");
     if (ameta.n < 2) fail(DDJ_ECORRUPT, "AFL metadata shorter than 2 bytes");
@@ -777,9 +785,22 @@ Part delta_afl_decode(Ctx* c, int dtype, DView dmeta, DView ameta, DView data) {
     const long long bits = (long long)data.n * 8 - rest;
     if (bits < 0) fail(DDJ_ECORRUPT, "AFL rest larger than the data");
     const size_t m = (size_t)(bits / b);
-    DevBuf out(c, (m + 1) * es);
-    launch_fl_unpack_delta(c, (int)es, dmeta.p, data.p, data.n, m, b, out.get());
-    kernel_bytes(c, "k_fl_unpack_delta_scan", (double)((m * b + 7) / 8 + (m + 1) * es));
+    FlDeltaOut o;
+    if (scale_meta.n) {
+        if (scale_meta.n < es) fail(DDJ_ECORRUPT, "scale metadata shorter than one value");
+        read_small(c, &o.bias, scale_meta.p, es);
+    }
+    size_t out_es = es;
+    if (float_dtype >= 0) {
+        static const double pw[10] = {1e0, 1e1, 1e2, 1e3, 1e4, 1e5, 1e6, 1e7, 1e8, 1e9};
+        if (precision < 0 || precision > 9) fail(DDJ_EINVAL, "converted rows need a precision below 10");
+        o.dtype = float_dtype;
+        o.pow10 = pw[precision];
+        out_es = dtype_size(float_dtype);
+    }
+    DevBuf out(c, (m + 1) * out_es);
+    launch_fl_unpack_delta(c, (int)es, dmeta.p, data.p, data.n, m, b, out.get(), nullptr, o);
+    kernel_bytes(c, "k_fl_unpack_delta_scan", (double)((m * b + 7) / 8 + (m + 1) * out_es));
     return own(std::move(out));
 }
 

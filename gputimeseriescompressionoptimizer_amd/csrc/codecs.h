@@ -91,7 +91,13 @@ ddj_stats_t stats(Ctx* c, int dtype, DView in);
 // delta_encode followed by the AFL encoder on its output.
 std::vector<Part> delta_afl_encode(Ctx* c, int dtype, DView in, bool defer_fl = false);
 // The inverse: AFL data (non-empty) decoded and prefix-summed in one pass.
-Part delta_afl_decode(Ctx* c, int dtype, DView delta_meta, DView afl_meta, DView afl_data);
+// scale_meta (may be empty): the metadata of a scale node above, whose value is
+// added to every row; float_dtype >= 0 (int32 deltas): a floatToInt node of that
+// type and precision (0..9) above those, whose rows are written.
+Part delta_afl_decode(Ctx* c, int dtype, DView dmeta, DView ameta, DView data, DView scale_meta = DView{},
+                      int float_dtype = -1, int precision = 0);
+// The precision a floatToInt node's metadata holds.
+int float_to_int_precision(Ctx* c, DView meta);
 
 // Patch (lower, or outside with `outside`) whose two outputs each go to an
 // AFL node stored unchanged, on an integer column of >= 1 row: the patch

@@ -134,8 +134,16 @@ void launch_fl_pack(Ctx* c, int dtype, const void* x, size_t n, const MinMaxResu
 // 64-bit words, every one written before it is read) or, when it is null,
 // to memory from the context's allocator.
 size_t fl_unpack_delta_scratch_words(size_t m);
+// Its rows may pass through the nodes above on the way out: `bias` is added
+// (scale), and with `dtype` a float type int32 rows are written as row / pow10
+// in that type (floatToInt).
+struct FlDeltaOut {
+    uint64_t bias = 0;
+    int dtype = -1;
+    double pow10 = 1.0;
+};
 void launch_fl_unpack_delta(Ctx* c, int elem_size, const uint8_t* first, const uint8_t* in, size_t in_bytes, size_t m,
-                           int bits, void* out, uint64_t* tile_scratch = nullptr);
+                           int bits, void* out, uint64_t* tile_scratch = nullptr, const FlDeltaOut& o = FlDeltaOut{});
 // FL unpack of the n values [first_row, first_row + n) of a b-bit stream at
 // an arbitrary byte address.
 void launch_fl_unpack(Ctx* c, int dtype, const uint8_t* in, size_t in_bytes, size_t n, int bits, void* out,

@@ -368,6 +368,22 @@ struct ParsedBlob {
         return is_leaf(kids[(size_t)a][0]) ? a : -1;
     }
 
+    // Node i is DELTA over AFL (delta_afl_child), or SCALE over that, or
+    // FLOAT_TO_INT (of a float type) over either with int32 rows: the DELTA
+    // node, else -1.
+    int delta_chain(int i) const {
+        const ParsedNode& nd = nodes[(size_t)i];
+        if (delta_afl_child(i) >= 0) return i;
+        if (nd.nchild != 1 || kids[(size_t)i].size() != 1) return -1;
+        const int k = kids[(size_t)i][0];
+        if (nd.enc == DDJ_ENC_SCALE && is_int_type(nd.dtype) && nodes[(size_t)k].dtype == nd.dtype)
+            return delta_afl_child(k) >= 0 ? k : -1;
+        if (nd.enc == DDJ_ENC_FLOAT_TO_INT && (nd.dtype == DDJ_D_FLOAT || nd.dtype == DDJ_D_DOUBLE) &&
+            nodes[(size_t)k].dtype == DDJ_D_INT && nodes[(size_t)k].enc != DDJ_ENC_FLOAT_TO_INT)
+            return delta_chain(k);
+        return -1;
+    }
+
     // The integer node i is a patch whose two children are AFL over a none
     // leaf: whether it is.
     bool patch_afl_kids(int i) const {
@@ -396,12 +412,26 @@ struct ParsedBlob {
             return patch_afl_decode(c, nd.dtype, m, meta(y), leaf_data(kids[(size_t)y][0]), meta(z),
                                     leaf_data(kids[(size_t)z][0]));
         }
-        // DELTA over AFL over none (integer): unpack and prefix-sum in one pass
-        const int a = delta_afl_child(i);
-        if (a >= 0) {
-            const int leaf = kids[(size_t)a][0];
-            if (nodes[(size_t)leaf].data_len > 0 && m.n >= dtype_size(nd.dtype))
-                return delta_afl_decode(c, nd.dtype, m, meta(a), leaf_data(leaf));
+        // DELTA over AFL over none (integer): unpack and prefix-sum in one
+        // pass, which the SCALE and FLOAT_TO_INT nodes right above it ride on
+        if (const int d = delta_chain(i); d >= 0) {
+            const int a = delta_afl_child(d), leaf = kids[(size_t)a][0];
+            const ParsedNode& dn = nodes[(size_t)d];
+            DView scale{};
+            int fdt = -1, precision = 0;
+            bool fits = nodes[(size_t)leaf].data_len > 0 && meta(d).n >= dtype_size(dn.dtype);
+            for (int k = i; fits && k != d; k = kids[(size_t)k][0]) {
+                if (nodes[(size_t)k].enc == DDJ_ENC_SCALE) {
+                    scale = meta(k);
+                    fits = scale.n >= dtype_size(dn.dtype);
+                } else {
+                    fdt = nodes[(size_t)k].dtype;
+                    fits = meta(k).n >= 4;
+                    if (fits) precision = float_to_int_precision(c, meta(k));
+                    fits = fits && precision < 10;  // else its rows are stored unconverted
+                }
+            }
+            if (fits) return delta_afl_decode(c, dn.dtype, meta(d), meta(a), leaf_data(leaf), scale, fdt, precision);
         }
         std::vector<Part> parts;
         std::vector<DView> in{m};

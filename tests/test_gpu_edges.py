@@ -214,3 +214,45 @@ def test_most_frequent_many_keys_in_few_rows(ctx, dtype, per_tile, tiles):
     x[1::1_009] = 77
     meta = g.Encoding(ctx, g.DICT).Encode(ctx.upload(x), dtype)[1].to_bytes()
     assert sorted(np.frombuffer(meta[16:16 + 4 * npdt().itemsize], npdt)) == sorted(_top(x, 4))
+
+
+@pytest.mark.parametrize("dtype", [g.D_FLOAT, g.D_DOUBLE])
+@pytest.mark.parametrize("path", [
+    [g.FLOAT_TO_INT, g.DELTA, g.AFL, g.NONE],
+    [g.FLOAT_TO_INT, g.SCALE, g.DELTA, g.AFL, g.NONE],
+    [g.FLOAT_TO_INT, g.SCALE, g.SCALE, g.DELTA, g.AFL, g.NONE],
+    [g.FLOAT_TO_INT, g.FLOAT_TO_INT, g.DELTA, g.AFL, g.NONE],
+], ids=["f2i-delta", "f2i-scale-delta", "f2i-scale-scale-delta", "f2i-f2i-delta"])
+@pytest.mark.parametrize("n", [1, 2, 3, 4_096, 4_097, 4_098, 8_193, 20_001])
+def test_float_rows_written_by_the_delta_decode(ctx, dtype, path, n):
+    npdt = g.NP_DTYPE[dtype]
+    r = np.random.default_rng(n)
+    for scale, step in ((1.0, 1), (4.0, 1), (100.0, 40), (0.0, 0)):  # 0, 2 and 2-3 decimals; not decimal at all
+        if scale:
+            x = (np.cumsum(r.integers(-step if step > 1 else 0, step + 1, n)) / scale - 5.0).astype(npdt)
+        else:
+            x = r.standard_normal(n).astype(npdt)
+        tree = g.CompressionTree(ctx, path, dtype)
+        blob = tree.Compress(ctx.upload(x)).to_bytes()
+        assert blob == O.compress(O.tree_from_path(path, dtype), x)
+        want = O.decompress(blob)
+        for shift in (0, 1, 2, 3):  # the 32-bit deltas at any byte address
+            moved = ctx.upload(b"\0" * shift + blob)
+            assert tree.Decompress(moved.view(shift, len(blob))).to_bytes() == want, (scale, shift)
+
+
+@pytest.mark.parametrize("dtype", [g.D_INT, g.D_TIME, g.D_SHORT, g.D_CHAR])
+@pytest.mark.parametrize("n", [1, 2, 4_097, 12_290])
+def test_scaled_deltas(ctx, dtype, n):
+    """scale over delta over FL at the full width (wrapping steps) and a narrow one."""
+    npdt = g.NP_DTYPE[dtype]
+    r = np.random.default_rng(n)
+    i = np.iinfo(npdt)
+    path = [g.SCALE, g.DELTA, g.AFL, g.NONE]
+    for x in (r.integers(i.min, i.max, n, dtype=npdt, endpoint=True), (50 + np.arange(n) % 60).astype(npdt)):
+        tree = g.CompressionTree(ctx, path, dtype)
+        blob = tree.Compress(ctx.upload(x)).to_bytes()
+        assert blob == O.compress(O.tree_from_path(path, dtype), x)
+        for shift in (0, 1, 3):
+            moved = ctx.upload(b"\0" * shift + blob)
+            assert np.array_equal(tree.Decompress(moved.view(shift, len(blob))).to_numpy(npdt), x)
