@@ -275,6 +275,22 @@ __device__ __forceinline__ uint32_t float_precision(float number) {
     }
     return k;
 }
+// The maximum of float_precision over the rows seen: a row that k = prec
+// decimals represent has a precision of at most prec, so only a row that fails
+// that one test (whose power of ten, exact in float up to 10^10, is kept with
+// prec) runs the loop.  One division a row in place of one per decimal.
+struct MaxPrecision {
+    uint32_t prec = 0;
+    float e = 1.0f;
+    __device__ __forceinline__ void add(float number) {
+        if (prec >= 10 || __fdiv_rn(roundf(number * e), e) == number) return;
+        const uint32_t p = float_precision(number);
+        while (prec < p) {
+            prec++;
+            e *= 10.0f;
+        }
+    }
+};
 
 // Min/max keys and the float precision (the maximum of float_precision
 // over the rows, as the statistics pass computes it) in one pass: the two
@@ -286,16 +302,10 @@ __global__ __launch_bounds__(kBlock) void k_minmax_prec(const T* __restrict__ x,
     __shared__ uint64_t sm[kBlock / kWave];
     __shared__ bool last;
     FoldKeys<T> f;
-    uint32_t prec = 0;
-    // The precision is a maximum capped at 10: a lane that has seen 10
-    // (noisy or NaN data) only folds min/max from then on, and once every
-    // lane of the wave has, the precision loop is skipped by the whole wave.
+    MaxPrecision pm;
     auto add = [&](T v, size_t row) {
         f.add(v, row);
-        if (prec < 10) {
-            const uint32_t p = float_precision((float)v);
-            prec = p > prec ? p : prec;
-        }
+        pm.add((float)v);
     };
     const size_t tid = (size_t)blockIdx.x * kBlock + threadIdx.x, stride = (size_t)gridDim.x * kBlock;
     constexpr int V = 16 / sizeof(T);
@@ -327,7 +337,7 @@ __global__ __launch_bounds__(kBlock) void k_minmax_prec(const T* __restrict__ x,
     const uint64_t mn = block_reduce_min(f.min_key(), sm);
     const uint64_t mx = block_reduce_max(f.max_key(), sm);
     const uint64_t zf = block_reduce_min(f.zf, sm);
-    const uint64_t pr = block_reduce_max((uint64_t)prec, sm);
+    const uint64_t pr = block_reduce_max((uint64_t)pm.prec, sm);
     if (threadIdx.x == 0) {
         st_agent(partials + 4 * blockIdx.x, mn);
         st_agent(partials + 4 * blockIdx.x + 1, mx);
@@ -594,10 +604,10 @@ __global__ __launch_bounds__(kBlock) void k_stats(const T* __restrict__ x, size_
     host_out_done(host);
 }
 
-int reduce_grid(Ctx* c, size_t n, int elem) {
+int reduce_grid(Ctx* c, size_t n, int elem, int per_cu = 2) {
     const size_t per_block = (size_t)kBlock * (16 / elem) * 4;
     const size_t g = (n + per_block - 1) / per_block;
-    const size_t cap = (size_t)c->cu_count * 2;  // 4 a CU: min/max of 64M int32 rows 48.2 us, of their deltas 50.3; 2: 47.2, 47.5
+    const size_t cap = (size_t)c->cu_count * per_cu;  // 4 a CU: min/max of 64M int32 rows 48.2 us, of their deltas 50.3; 2: 47.2, 47.5
     return (int)std::max<size_t>(1, std::min(g, cap));
 }
 
@@ -647,7 +657,8 @@ FloatScanResult float_scan(Ctx* c, int dtype, const void* x, size_t n) {
     dispatch_native(dtype, [&](auto tag) {
         using T = decltype(tag);
         if constexpr (std::is_floating_point<T>::value) {
-            const int grid = reduce_grid(c, n, sizeof(T));
+            // the precision's divisions need more waves than a plain pass
+            const int grid = reduce_grid(c, n, sizeof(T), 8);
             DevBuf partials(c, 32 * (size_t)grid);
             kernel_bytes(c, "k_minmax_prec", (double)n * sizeof(T));
             KernelTimer kt_(c, "k_minmax_prec");

@@ -256,3 +256,19 @@ def test_scaled_deltas(ctx, dtype, n):
         for shift in (0, 1, 3):
             moved = ctx.upload(b"\0" * shift + blob)
             assert np.array_equal(tree.Decompress(moved.view(shift, len(blob))).to_numpy(npdt), x)
+
+
+@pytest.mark.parametrize("dtype", [g.D_FLOAT, g.D_DOUBLE])
+@pytest.mark.parametrize("n", [1, 63, 5_000, 300_001])
+def test_precision_of_late_rows(ctx, dtype, n):
+    """Rows whose decimals grow along the column, one row deciding."""
+    npdt = g.NP_DTYPE[dtype]
+    x = np.full(n, 2.0, npdt)
+    for decimals in (0, 1, 2, 3, 4):
+        x[n - 1 - n // 7] = npdt(1.0) + npdt(3) / npdt(10.0 ** decimals)
+        outs = [o.to_bytes() for o in g.Encoding(ctx, g.FLOAT_TO_INT).Encode(ctx.upload(x), dtype)]
+        assert outs == O.encode(g.FLOAT_TO_INT, dtype, x)
+        assert ctx.stats(ctx.upload(x), dtype).precision == O.stats(dtype, x).precision
+    x[n // 2] = np.nan
+    outs = [o.to_bytes() for o in g.Encoding(ctx, g.FLOAT_TO_INT).Encode(ctx.upload(x), dtype)]
+    assert outs == O.encode(g.FLOAT_TO_INT, dtype, x)
