@@ -465,11 +465,13 @@ struct PatchFlJob {
     uint8_t* dst[3] = {nullptr, nullptr, nullptr};  // stencil, yes stream, no stream
     int expected = 0, seen = 0;
     std::shared_ptr<DevBuf> count;
-    void place(Ctx* c, int which, uint8_t* p) {
+    void place(Ctx* c, int which, uint8_t* p, SmallPieces* sp) {
         dst[which] = p;
         if (++seen < expected) return;
+        SmallPieces pieces = sp ? *sp : SmallPieces{};
+        if (sp) sp->count = 0;  // taken
         launch_split_fl(c, plan, dst[0], FlSide{dst[1], ybytes, by, nullptr}, FlSide{dst[2], nbytes, bn, nullptr},
-                        count->get<uint64_t>());
+                        count->get<uint64_t>(), pieces);
     }
 };
 
@@ -698,7 +700,7 @@ std::vector<Part> gfc_encode_any(Ctx* c, int dtype, DView in, bool defer) {
     job->dtype = dtype;
     job->n = n;
     job->x = x;
-    job->write = [plan](Ctx* c, uint8_t* out, size_t bytes) {
+    job->write = [plan](Ctx* c, uint8_t* out, size_t bytes, SmallPieces*) {
         if (bytes != plan.payload_bytes) fail(DDJ_EHIP, "GFC payload size mismatch");
         gfc_write(c, plan, out);
     };
@@ -755,7 +757,7 @@ PatchAflParts patch_afl_encode(Ctx* c, int dtype, DView in, bool outside) {
         if (!nb) return part;
         auto fj = std::make_shared<FlJob>();
         fj->dtype = dtype;
-        fj->write = [job, which](Ctx* cc, uint8_t* dst, size_t) { job->place(cc, which, dst); };
+        fj->write = [job, which](Ctx* cc, uint8_t* dst, size_t, SmallPieces* sp) { job->place(cc, which, dst, sp); };
         part.fl = std::move(fj);
         return part;
     };
@@ -937,18 +939,19 @@ void run_split_job(Ctx* c, const SplitJob& j, void* no_rows) {
                        j.count->get<uint64_t>());
 }
 
-void run_fl_job(Ctx* c, const FlJob& j, void* out, size_t bytes) {
+void run_fl_job(Ctx* c, const FlJob& j, void* out, size_t bytes, SmallPieces* sp) {
     if (j.write) {
-        if (bytes) j.write(c, static_cast<uint8_t*>(out), bytes);
+        if (bytes) j.write(c, static_cast<uint8_t*>(out), bytes, sp);
         return;
     }
     const size_t es = dtype_size(j.dtype);
     if (j.n == 0 || bytes == 0) return;
     if (bytes != fl_bytes(es, j.bits, j.n)) fail(DDJ_EHIP, "FL job size mismatch");
     if (j.delta)
-        launch_fl_pack_delta(c, (int)es, j.x.p, j.n, nullptr, out, j.bits, bytes);
+        launch_fl_pack_delta(c, (int)es, j.x.p, j.n, nullptr, out, j.bits, bytes, sp ? *sp : SmallPieces{});
     else
-        launch_fl_pack(c, j.dtype, j.x.p, j.n, nullptr, j.bits, out, bytes);
+        launch_fl_pack(c, j.dtype, j.x.p, j.n, nullptr, j.bits, out, bytes, sp ? *sp : SmallPieces{});
+    if (sp) sp->count = 0;  // taken
     kernel_bytes(c, "k_fl_pack", (double)((j.n + (j.delta ? 1 : 0)) * es + fl_bytes(es, j.bits, j.n)));
 }
 

@@ -47,10 +47,12 @@ struct FlJob {
     size_t n = 0;  // values packed
     Part x;        // the rows, kept alive until the pack runs
     // set: writes the stream itself (a GFC payload) instead of an FL pack
-    std::function<void(Ctx*, uint8_t*, size_t)> write;
+    std::function<void(Ctx*, uint8_t*, size_t, SmallPieces*)> write;
 };
 // Runs the pack into the `bytes` stream bytes at out (any byte address).
-void run_fl_job(Ctx* c, const FlJob& j, void* out, size_t bytes);
+// sp (optional): the blob's small pieces, which the first job that can takes
+// along (its count is then 0).
+void run_fl_job(Ctx* c, const FlJob& j, void* out, size_t bytes, SmallPieces* sp = nullptr);
 
 // A dictionary split whose counting pass ran (the yes count is known): its
 // writing pass fills the stencil and code buffers (parts of its encoder's

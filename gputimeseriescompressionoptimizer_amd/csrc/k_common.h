@@ -253,6 +253,15 @@ __device__ __forceinline__ void host_out_done(const HostOut& h) {
     if (threadIdx.x == 0) __hip_atomic_store(h.flag, h.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Writes the small pieces of a blob (one workgroup).
+__device__ __forceinline__ void write_small(const SmallPieces& sp) {
+    for (int p = 0; p < sp.count; p++) {  // uniform
+        const auto& r = sp.piece[p];
+        for (uint32_t i = threadIdx.x; i < r.bytes; i += blockDim.x)
+            sp.blob[r.dst_off + i] = r.src ? r.src[i] : sp.inl[r.at + i];
+    }
+}
+
 // A tile's value, where its tail (if any) will find it.
 __device__ __forceinline__ void put_tile(const ScanTail& st, uint64_t* vals, size_t tile, uint64_t v) {
     if (st.tickets)

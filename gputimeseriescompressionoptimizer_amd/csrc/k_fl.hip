@@ -31,8 +31,13 @@ namespace {
 
 template <typename T, bool DELTA = false>
 __global__ __launch_bounds__(kBlock) void k_fl_pack(const T* __restrict__ x, size_t n, const MinMaxResult* mm,
-                                                    int fixed_bits, uint8_t* __restrict__ out, size_t out_bytes) {
+                                                    int fixed_bits, uint8_t* __restrict__ out, size_t out_bytes,
+                                                    SmallPieces sp) {
     __shared__ __attribute__((aligned(16))) T vals[kFlLdsVals];
+    if ((size_t)blockIdx.x * kFlTile >= n) {  // one past the tiles
+        write_small(sp);
+        return;
+    }
     int b = fixed_bits;
     if (mm) b = bitlen_of<T>(from_order_key<T>(mm->min_key), from_order_key<T>(mm->max_key));
     fl_pack_tile<T, DELTA>(x, n, b, out, out_bytes, blockIdx.x, vals);
@@ -227,7 +232,7 @@ template <typename F> void with_maxb(int b, F&& f) {
 }  // namespace
 
 void launch_fl_pack(Ctx* c, int dtype, const void* x, size_t n, const MinMaxResult* mm, int bits, void* out,
-                    size_t out_bytes) {
+                    size_t out_bytes, const SmallPieces& sp) {
     if (n == 0) return;
     const int esize = (int)dtype_size(dtype);
     dispatch_int(esize, [&](auto tag) {
@@ -238,14 +243,14 @@ void launch_fl_pack(Ctx* c, int dtype, const void* x, size_t n, const MinMaxResu
             out_bytes = ((size_t)((maxb * (uint64_t)n + W - 1) / W) * sizeof(T) + 3) & ~size_t(3);
         }
         const size_t tiles = (n + kFlTile - 1) / kFlTile;
-        { KernelTimer kt_(c, "k_fl_pack"); hipLaunchKernelGGL(k_fl_pack<T>, dim3((unsigned)tiles), dim3(kBlock), 0, c->stream, static_cast<const T*>(x),
-                           n, mm, bits, static_cast<uint8_t*>(out), out_bytes); }
+        { KernelTimer kt_(c, "k_fl_pack"); hipLaunchKernelGGL(k_fl_pack<T>, dim3((unsigned)(tiles + (sp.count ? 1 : 0))), dim3(kBlock), 0, c->stream,
+                           static_cast<const T*>(x), n, mm, bits, static_cast<uint8_t*>(out), out_bytes, sp); }
         HIPC(hipGetLastError());
     });
 }
 
 void launch_fl_pack_delta(Ctx* c, int elem_size, const void* x, size_t m, const MinMaxResult* mm, void* out, int bits,
-                          size_t out_bytes) {
+                          size_t out_bytes, const SmallPieces& sp) {
     if (m == 0) return;
     dispatch_int(elem_size, [&](auto tag) {
         using T = decltype(tag);
@@ -254,8 +259,8 @@ void launch_fl_pack_delta(Ctx* c, int elem_size, const void* x, size_t m, const 
             out_bytes = ((size_t)((W * m + W - 1) / W) * sizeof(T) + 3) & ~size_t(3);
         }
         const size_t tiles = (m + kFlTile - 1) / kFlTile;
-        { KernelTimer kt_(c, "k_fl_pack"); hipLaunchKernelGGL((k_fl_pack<T, true>), dim3((unsigned)tiles), dim3(kBlock), 0, c->stream,
-                           static_cast<const T*>(x), m, mm, bits, static_cast<uint8_t*>(out), out_bytes); }
+        { KernelTimer kt_(c, "k_fl_pack"); hipLaunchKernelGGL((k_fl_pack<T, true>), dim3((unsigned)(tiles + (sp.count ? 1 : 0))), dim3(kBlock), 0, c->stream,
+                           static_cast<const T*>(x), m, mm, bits, static_cast<uint8_t*>(out), out_bytes, sp); }
         HIPC(hipGetLastError());
     });
 }

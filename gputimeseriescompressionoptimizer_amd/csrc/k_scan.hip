@@ -309,7 +309,12 @@ __global__ __launch_bounds__(kBlock) void k_split(const T* __restrict__ x, size_
 template <typename T, int K>
 __global__ __launch_bounds__(kBlock) void k_split_fl(const T* __restrict__ x, size_t n, Pred<T> p,
                                                      uint8_t* __restrict__ stencil, FlSide yside, FlSide nside,
-                                                     const uint64_t* __restrict__ prefix, uint64_t* d_count) {
+                                                     const uint64_t* __restrict__ prefix, uint64_t* d_count,
+                                                     SmallPieces sp) {
+    if ((size_t)blockIdx.x * kTile >= n) {  // one past the tiles
+        write_small(sp);
+        return;
+    }
     using U = typename UnsignedOf<T>::type;
     static_assert(sizeof(T) * kTilePad >= 4 * (kTile / 32 + 2) * 8 * sizeof(T), "packed words fit the tile buffer");
     __shared__ __attribute__((aligned(16))) T buf[kTilePad];
@@ -1316,7 +1321,8 @@ ScanResult launch_split(Ctx* c, int dtype, const void* x, size_t n, const PredAr
     return split_result(c, plan);
 }
 
-void launch_split_fl(Ctx* c, const SplitPlan& plan, uint8_t* stencil, FlSide yes, FlSide no, uint64_t* d_counts) {
+void launch_split_fl(Ctx* c, const SplitPlan& plan, uint8_t* stencil, FlSide yes, FlSide no, uint64_t* d_counts,
+                     const SmallPieces& sp) {
     if (plan.n == 0) return;
     if (plan.p.kind != PRED_LOWER && plan.p.kind != PRED_INSIDE) fail(DDJ_EINVAL, "FL split: patch predicates only");
     const size_t tiles = plan.ts->tiles;
@@ -1337,8 +1343,9 @@ void launch_split_fl(Ctx* c, const SplitPlan& plan, uint8_t* stencil, FlSide yes
             with_kind(p.kind, [&](auto kind) {
                 constexpr int K = decltype(kind)::value;
                 if constexpr (K == PRED_LOWER || K == PRED_INSIDE)
-                    hipLaunchKernelGGL((k_split_fl<T, K>), dim3((unsigned)tiles), dim3(kBlock), 0, c->stream,
-                                       static_cast<const T*>(plan.x), plan.n, p, stencil, yes, no, pre, d_counts);
+                    hipLaunchKernelGGL((k_split_fl<T, K>), dim3((unsigned)(tiles + (sp.count ? 1 : 0))), dim3(kBlock), 0,
+                                       c->stream, static_cast<const T*>(plan.x), plan.n, p, stencil, yes, no, pre,
+                                       d_counts, sp);
             });
         }
         HIPC(hipGetLastError());

@@ -97,11 +97,30 @@ MinMaxResult minmax_to_host(Ctx* c, int dtype, const void* x, size_t n, bool del
 // count; fold_minmax_partials folds them (stride 3; 2 for delta) on the host.
 int launch_minmax_partials(Ctx* c, int dtype, const void* x, size_t n, const uint64_t* d_rows, DevBuf& partials);
 MinMaxResult fold_minmax_partials(const uint64_t* h, int grid, int stride);
+// The few bytes of a blob around its streams (node headers, metadata), written
+// by one more workgroup of the kernel that writes a stream, from the kernel's
+// arguments: a gather launch of their own, its table read over PCIe, was 4.7
+// us on the device and 3.4 us of launching.
+struct SmallPieces {
+    static constexpr int kMax = 12, kInline = 192;
+    static constexpr size_t kMaxBytes = 1024;  // of all of them
+    uint8_t* blob = nullptr;
+    int count = 0;
+    struct {
+        const uint8_t* src;  // null: bytes of `inl`
+        uint32_t at;         // first of them
+        uint32_t bytes;
+        uint64_t dst_off;
+    } piece[kMax];
+    uint8_t inl[kInline];
+};
+
 // FL pack of the m = n - 1 differences of n integer rows (bits from mm).
 // With mm null the width is `bits`; no byte at or past out + out_bytes is
 // written (0: room for the widest b, rounded up to whole words).
 void launch_fl_pack_delta(Ctx* c, int elem_size, const void* x, size_t m, const MinMaxResult* mm, void* out,
-                          int bits = 0, size_t out_bytes = 0);
+                          int bits = 0, size_t out_bytes = 0,
+                          const SmallPieces& sp = SmallPieces{});
 // Converts order keys back to the typed min/max (host).
 void decode_minmax(int dtype, const MinMaxResult& r, void* mn, void* mx);
 
@@ -127,7 +146,7 @@ DevStats device_stats(Ctx* c, int dtype, const void* x, size_t n);
 // or past out + out_bytes (0: room for the widest b, rounded up to whole
 // words).
 void launch_fl_pack(Ctx* c, int dtype, const void* x, size_t n, const MinMaxResult* mm, int bits, void* out,
-                    size_t out_bytes = 0);
+                    size_t out_bytes = 0, const SmallPieces& sp = SmallPieces{});
 // FL unpack of m b-bit deltas fused with the delta decode: out[0] = first
 // (device, one value), out[i+1] = out[i] + d[i] (wrapping).  The per-tile
 // sums and prefixes go to tile_scratch (fl_unpack_delta_scratch_words(m)
@@ -231,7 +250,8 @@ struct FlSide {
 // The writing pass of a patch split whose two outputs are FL leaves: the
 // stencil, and both sides packed into their streams (k_split_fl, then
 // k_fl_edges for the words neighbouring tiles share).
-void launch_split_fl(Ctx* c, const SplitPlan& plan, uint8_t* stencil, FlSide yes, FlSide no, uint64_t* d_counts);
+void launch_split_fl(Ctx* c, const SplitPlan& plan, uint8_t* stencil, FlSide yes, FlSide no, uint64_t* d_counts,
+                     const SmallPieces& sp = SmallPieces{});
 // Merge: out[i] = bit i ? yes[k++] : no[j++] (const_no: `no_const` for every
 // clear bit).  yes / no may sit at any byte address (outputs stored
 // unchanged in a blob); n_yes / n_no rows are available; a stencil asking

@@ -223,8 +223,8 @@ Part compress_tree(Ctx* c, const NodeP& root, DView data) {
     std::vector<Piece> pieces;
     size_t total = compress_node(c, *root, borrow(data), pieces);
     // Concatenate (util/copy/cuda_array_copy.cu:14-33): deferred FL packs
-    // write straight into their blob ranges, everything else moves in one
-    // gather kernel.  The copy table, the node headers and the host-resident
+    // write straight into their blob ranges and take a few small pieces along,
+    // everything else moves in one gather kernel.  The copy table, the node headers and the host-resident
     // metadata form one table, read by the kernel from the pinned staging
     // ring (or, without a device address for it, uploaded in one copy):
     // their ranges point into the table itself.
@@ -287,25 +287,54 @@ Part compress_tree(Ctx* c, const NodeP& root, DView data) {
     if (off != total || ri != n_ranges) fail(DDJ_EHIP, "blob size mismatch");
     // deferred splits first: they also fill outputs that the gather copies
     for (const auto& sj : splits) run_split_job(c, *sj.first, blob.bytes_ptr() + sj.second);
-    // the table's device address: a slot of the staging ring, taken now (no
-    // staged copy may follow before the launch), else a device buffer
-    DevBuf rdev;
-    const uint8_t* tdev = staging_slot(c, table_bytes);
-    if (!tdev) {
-        rdev = DevBuf(c, table_bytes);
-        tdev = rdev.bytes_ptr();
+    // a few small pieces ride along with a job's kernel
+    SmallPieces sp;
+    if (!jobs.empty() && copied <= SmallPieces::kMaxBytes && inline_bytes <= SmallPieces::kInline) {
+        sp.blob = blob.bytes_ptr();
+        size_t next_inline = 0;  // index into inline_ranges
+        bool fits = true;
+        for (size_t k = 0; k < n_ranges && fits; k++) {
+            const bool in = next_inline < inline_ranges.size() && inline_ranges[next_inline] == k;
+            if (in) next_inline++;
+            const uint32_t at = in ? (uint32_t)reinterpret_cast<uintptr_t>(ranges[k].src) : 0u;
+            auto* last = sp.count ? &sp.piece[sp.count - 1] : nullptr;
+            if (in && last && !last->src && last->at + last->bytes == at &&
+                last->dst_off + last->bytes == ranges[k].dst_off) {
+                last->bytes += (uint32_t)ranges[k].bytes;  // headers and host metadata run on
+            } else if ((fits = sp.count < SmallPieces::kMax)) {
+                auto& q = sp.piece[sp.count++];
+                q.src = in ? nullptr : ranges[k].src;
+                q.at = at;
+                q.bytes = (uint32_t)ranges[k].bytes;
+                q.dst_off = ranges[k].dst_off;
+            }
+        }
+        if (!fits) sp.count = 0;
+        memcpy(sp.inl, inl, inline_bytes);
     }
-    for (size_t k : inline_ranges)
-        ranges[k].src = tdev + sizeof(CopyRange) * n_ranges + reinterpret_cast<uintptr_t>(ranges[k].src);
-    if (rdev.get())
-        h2d(c, rdev.get(), table.data(), table.size());
-    else
-        memcpy(c->staging + (tdev - c->staging_dev), table.data(), table.size());
-    kernel_bytes(c, "k_gather_copy", 2.0 * (double)copied);
-    launch_gather_copy(c, reinterpret_cast<const CopyRange*>(tdev), (int)n_ranges, blob.bytes_ptr(),
-                       std::max<uint64_t>(max_bytes, 8));
+    const bool riding = sp.count > 0;
     // the FL streams go straight to their blob ranges (any byte offset)
-    for (const JobAt& j : jobs) run_fl_job(c, *j.job, blob.bytes_ptr() + j.off, j.bytes);
+    for (const JobAt& j : jobs)
+        run_fl_job(c, *j.job, blob.bytes_ptr() + j.off, j.bytes, sp.count > 0 ? &sp : nullptr);
+    if (!(riding && sp.count == 0) && n_ranges) {
+        // the table's device address: a slot of the staging ring, taken now (no
+        // staged copy may follow before the launch), else a device buffer
+        DevBuf rdev;
+        const uint8_t* tdev = staging_slot(c, table_bytes);
+        if (!tdev) {
+            rdev = DevBuf(c, table_bytes);
+            tdev = rdev.bytes_ptr();
+        }
+        for (size_t k : inline_ranges)
+            ranges[k].src = tdev + sizeof(CopyRange) * n_ranges + reinterpret_cast<uintptr_t>(ranges[k].src);
+        if (rdev.get())
+            h2d(c, rdev.get(), table.data(), table.size());
+        else
+            memcpy(c->staging + (tdev - c->staging_dev), table.data(), table.size());
+        kernel_bytes(c, "k_gather_copy", 2.0 * (double)copied);
+        launch_gather_copy(c, reinterpret_cast<const CopyRange*>(tdev), (int)n_ranges, blob.bytes_ptr(),
+                           std::max<uint64_t>(max_bytes, 8));
+    }
     return own(std::move(blob));
 }
 
