@@ -344,12 +344,12 @@ std::vector<Part> rle_encode(Ctx* c, int dtype, DView in) {
     int32_t R = 0;
     if (n == 0) return {host_part(&R, 4), empty(), empty()};
     Part x = aligned_view(c, in, es);
-    DevBuf lens(c, 4 * n), vals(c, es * n), runs(c, 8);
+    DevBuf lens(c, 4 * n), vals(c, es * n);
     // the run count comes back with both outputs' min/max (integer values):
     // FL encoders of the outputs then need no pass or read-back of their own
     const bool integral = dtype != DDJ_D_FLOAT && dtype != DDJ_D_DOUBLE;
     auto hl = std::make_shared<MinMaxResult>(), hv = std::make_shared<MinMaxResult>();
-    const uint64_t r = launch_rle_encode(c, dtype, x.p, n, lens.get<int32_t>(), vals.get(), runs.get<uint64_t>(),
+    const uint64_t r = launch_rle_encode(c, dtype, x.p, n, lens.get<int32_t>(), vals.get(),
                                          integral ? hv.get() : nullptr, hl.get());
     R = (int32_t)r;
     kernel_bytes(c, "k_rle_encode", (double)(n * es + r * (4 + es)));

@@ -103,7 +103,6 @@ template <typename T> __device__ __forceinline__ void fold_fixup(const T* x, uin
 
 // What the last workgroup of a min/max pass does with the partials (STRIDE
 // keys each: min, max, then the first zero and the precision where kept).
-// No tickets: the partials are left to the host.
 struct FoldTail {
     uint32_t* tickets = nullptr;
     MinMaxResult* out = nullptr;  // device result, or null
@@ -113,7 +112,7 @@ struct FoldTail {
 template <typename T, int STRIDE>
 __device__ __forceinline__ void fold_partials(const FoldTail& ft, const uint64_t* partials, const T* x, uint64_t* sm,
                                               bool* flag) {
-    if (!ft.tickets || !last_of_grid(ft.tickets, flag)) return;
+    if (!last_of_grid(ft.tickets, flag)) return;
     uint64_t mn = ~0ull, mx = 0, zf = ~0ull, pr = 0;
     for (uint32_t b = threadIdx.x; b < gridDim.x; b += kBlock) {
         const uint64_t a = rd(partials + STRIDE * b), z = rd(partials + STRIDE * b + 1);
@@ -146,10 +145,9 @@ __device__ __forceinline__ void fold_partials(const FoldTail& ft, const uint64_t
 
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_minmax(const T* __restrict__ x, size_t n, uint64_t* __restrict__ partials,
-                                                   const uint64_t* d_rows, FoldTail ft) {
+                                                   FoldTail ft) {
     __shared__ uint64_t sm[kBlock / kWave];
     __shared__ bool last;
-    if (d_rows) n = *d_rows < n ? *d_rows : n;  // rows counted on the device (uniform)
     FoldKeys<T> f;
     const size_t tid = (size_t)blockIdx.x * kBlock + threadIdx.x, stride = (size_t)gridDim.x * kBlock;
     constexpr int V = 16 / sizeof(T);
@@ -626,7 +624,7 @@ HostOut launch_minmax(Ctx* c, int dtype, const void* x, size_t n, bool delta, Mi
         KernelTimer kt_(c, delta ? "k_minmax_delta" : "k_minmax");
         if (!delta) {
             hipLaunchKernelGGL(k_minmax<T>, dim3(grid), dim3(kBlock), 0, c->stream, static_cast<const T*>(x), n,
-                               partials.get<uint64_t>(), nullptr, ft);
+                               partials.get<uint64_t>(), ft);
         } else {
             if constexpr (std::is_floating_point<T>::value)
                 fail(DDJ_EINVAL, "delta min/max: integer columns only");
@@ -671,41 +669,6 @@ FloatScanResult float_scan(Ctx* c, int dtype, const void* x, size_t n) {
     });
     FloatScanResult r;
     memcpy(&r, wait_host_out(c, ft.host), sizeof r);
-    return r;
-}
-
-// Workgroups of a reduction whose partials go to the host (6 KB of them):
-// RLE's values and lengths, whose row count (the run count) is only known
-// on the device and usually far below the bound the grid is sized for.
-// Against a full column's 1024 workgroups and a device fold, the 64M-row
-// step-function tree compresses in 0.145 instead of 0.158 ms.
-constexpr int kPartialsGrid = 256;
-
-int launch_minmax_partials(Ctx* c, int dtype, const void* x, size_t n, const uint64_t* d_rows, DevBuf& partials) {
-    if (n == 0) fail(DDJ_EINVAL, "minmax of an empty array");
-    int grid = 0;
-    dispatch_native(dtype, [&](auto tag) {
-        using T = decltype(tag);
-        if constexpr (std::is_floating_point<T>::value) {
-            fail(DDJ_EINVAL, "host-folded min/max: integer columns only");
-        } else {
-            grid = std::min(reduce_grid(c, n, sizeof(T)), kPartialsGrid);
-            partials = DevBuf(c, 24 * (size_t)grid);
-            KernelTimer kt_(c, "k_minmax");
-            hipLaunchKernelGGL(k_minmax<T>, dim3(grid), dim3(kBlock), 0, c->stream, static_cast<const T*>(x), n,
-                               partials.get<uint64_t>(), d_rows, FoldTail{});
-            HIPC(hipGetLastError());
-        }
-    });
-    return grid;
-}
-
-MinMaxResult fold_minmax_partials(const uint64_t* h, int grid, int stride) {
-    MinMaxResult r{~0ull, 0ull};
-    for (int b = 0; b < grid; b++) {  // order keys: the min of the minima, the max of the maxima
-        r.min_key = std::min(r.min_key, h[(size_t)stride * b]);
-        r.max_key = std::max(r.max_key, h[(size_t)stride * b + 1]);
-    }
     return r;
 }
 

@@ -920,11 +920,26 @@ template <typename T> __device__ __forceinline__ T shfl_up_value(T v) {
     return out;
 }
 
-// Runs starting in each tile (the RLE encoder's counting pass).
+// What an RLE encoder hands to the host: the min/max keys of its two outputs
+// are folded from {values min, max, lengths min, max} of each tile.
+struct RleResult {
+    uint64_t runs;
+    MinMaxResult values, lengths;
+};
+
+// Runs starting in each tile (the RLE encoder's counting pass), and the first
+// row that starts one (~0: none).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_rle_count(const T* __restrict__ x, size_t n, uint64_t* __restrict__ vals,
-                                                      ScanTail st) {
+                                                      uint32_t* __restrict__ firsts, ScanTail st) {
     __shared__ uint64_t red[kBlock / kWave];
+    __shared__ uint32_t s_first;
+    if (threadIdx.x == 0) s_first = ~0u;
+    uint32_t first = ~0u;
+    auto starts = [&](uint32_t mask, size_t row) {  // a thread's rows ascend, and fit 32 bits (n < 2^31)
+        if (mask && first == ~0u) first = (uint32_t)row + __builtin_ctz(mask);
+        return (uint32_t)__popc(mask);
+    };
     const size_t base = (size_t)blockIdx.x * kTile;
     const int cnt = (int)((n - base) < (size_t)kTile ? (n - base) : (size_t)kTile);
     uint32_t c = 0;
@@ -949,32 +964,93 @@ __global__ __launch_bounds__(kBlock) void k_rle_count(const T* __restrict__ x, s
             // the row before this chunk ends the previous lane's chunk
             T prev = shfl_up_value(v[V - 1]);
             if (lane0) prev = g > 0 ? before[q] : v[0];
-            c += (g == 0 || !(v[0] == prev)) ? 1u : 0u;
+            uint32_t mask = (g == 0 || !(v[0] == prev)) ? 1u : 0u;
 #pragma unroll
-            for (int k = 1; k < V; k++) c += !(v[k] == v[k - 1]) ? 1u : 0u;
+            for (int k = 1; k < V; k++) mask |= (uint32_t)!(v[k] == v[k - 1]) << k;
+            c += starts(mask, g);
         }
     } else {
         for (int i = threadIdx.x; i < cnt; i += kBlock) {
             const size_t g = base + i;
-            c += (g == 0 || !(x[g] == x[g - 1])) ? 1u : 0u;
+            c += starts((g == 0 || !(x[g] == x[g - 1])) ? 1u : 0u, g);
         }
     }
+    const uint32_t wf = wave_min(first);
     uint64_t total;
-    block_exclusive_scan<uint64_t>((uint64_t)c, &total, red);
-    if (threadIdx.x == 0) put_tile(st, vals, blockIdx.x, total);
+    block_exclusive_scan<uint64_t>((uint64_t)c, &total, red);  // barriers: s_first is set
+    if ((threadIdx.x & (kWave - 1)) == 0 && wf != ~0u) atomicMin(&s_first, wf);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        put_tile(st, vals, blockIdx.x, total);
+        firsts[blockIdx.x] = s_first;
+    }
     scan_tail(st, vals);
 }
 
+// Adds a thread's {min, max, min, max} to a workgroup's mm; whole waves.
+__device__ __forceinline__ void fold4(unsigned long long* mm, const uint64_t (&k)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const unsigned long long w = (j & 1) ? wave_max(k[j]) : wave_min(k[j]);
+        if ((threadIdx.x & (kWave - 1)) != 0) continue;
+        if (j & 1)
+            atomicMax(&mm[j], w);
+        else
+            atomicMin(&mm[j], w);
+    }
+}
+
+// Folds `count` entries of keys (begin, begin + step, ...) into mm: by the
+// whole workgroup, which has to pass a barrier before it reads mm.
+__device__ __forceinline__ void fold_keys(unsigned long long* mm, const uint64_t* keys, size_t count, size_t begin,
+                                          size_t step) {
+    if (threadIdx.x < 4) mm[threadIdx.x] = (threadIdx.x & 1) ? 0ull : ~0ull;
+    uint64_t r[4] = {~0ull, 0, ~0ull, 0};
+    for (size_t i = begin; i < count; i += step) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint64_t v = ld_agent(keys + 4 * i + j);
+            r[j] = (j & 1) ? (v > r[j] ? v : r[j]) : (v < r[j] ? v : r[j]);
+        }
+    }
+    __syncthreads();
+    fold4(mm, r);
+}
+
+// The fold and the run count to the host, by one workgroup.
+__device__ __forceinline__ void rle_to_host(unsigned long long* mm, const uint64_t* keys, size_t count, uint64_t runs,
+                                            const HostOut& host) {
+    fold_keys(mm, keys, count, threadIdx.x, kBlock);
+    __syncthreads();
+    if (threadIdx.x == 0) *reinterpret_cast<RleResult*>(host.dst) = RleResult{runs, {mm[0], mm[1]}, {mm[2], mm[3]}};
+    host_out_done(host);
+}
+
+// Values and lengths of each tile's runs.  A thread's last run ends where the
+// next thread that holds a start has its first (its wave's ballot, then the
+// waves' firsts), a tile's last run where the next tile that starts one does
+// (firsts, found through the prefixes when the very next tile starts none).
+// The outputs' min/max keys come along: with a tail the last workgroup folds
+// them and hands them to the host with the run count.  Bound by the tile's
+// chain of latencies at 8 workgroups per CU (LDS: compacting the starts there
+// first left 6, 62 us for 64M int32 rows).
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_rle_encode(const T* __restrict__ x, size_t n, T* __restrict__ values,
-                                                       uint32_t* __restrict__ starts,
-                                                       const uint64_t* __restrict__ prefix, uint64_t* d_runs) {
+__global__ __launch_bounds__(kBlock) void k_rle_encode(const T* __restrict__ x, size_t n, size_t tiles,
+                                                       T* __restrict__ values, int32_t* __restrict__ lengths,
+                                                       const uint64_t* __restrict__ prefix,
+                                                       const uint32_t* __restrict__ firsts, uint64_t* __restrict__ keys,
+                                                       uint32_t* tickets, HostOut host) {
     __shared__ T buf[kTilePad + 1];
     __shared__ uint64_t red[kBlock / kWave];
+    __shared__ uint32_t wave_first[kBlock / kWave];  // the first row of each wave that starts a run
+    __shared__ unsigned long long mm[4];
+    __shared__ bool last;
     const uint32_t tile = blockIdx.x;
     const size_t base = (size_t)tile * kTile;
     const int cnt = (int)((n - base) < (size_t)kTile ? (n - base) : (size_t)kTile);
     const uint64_t s_prefix = prefix[tile];  // loaded with the tile
+    if (threadIdx.x < 4) mm[threadIdx.x] = (threadIdx.x & 1) ? 0ull : ~0ull;
+    uint32_t next = tile + 1 < tiles ? firsts[tile + 1] : (uint32_t)n;  // loaded with the tile too
     if (cnt == kTile && (reinterpret_cast<uintptr_t>(x + base) & 15) == 0) {
         // buf[i + 1] = x[base + i]; buf[0] = the row before the tile
         constexpr int V = 16 / sizeof(T);
@@ -1003,29 +1079,80 @@ __global__ __launch_bounds__(kBlock) void k_rle_encode(const T* __restrict__ x, 
             mask |= (uint32_t)f << k;
         }
     }
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const uint32_t row0 = (uint32_t)base + threadIdx.x * kItems;  // rows fit 32 bits (n < 2^31)
+    const uint32_t first = mask ? row0 + __builtin_ctz(mask) : ~0u;
+    const uint64_t holders = __ballot(mask != 0);
+    if (holders && lane == __builtin_ctzll(holders)) wave_first[wave] = first;
+    if (!holders && lane == 0) wave_first[wave] = ~0u;
     uint64_t total;
-    const uint64_t excl = block_exclusive_scan<uint64_t>((uint64_t)__popc(mask), &total, red);
-    uint64_t r = s_prefix + excl;
-#pragma unroll
-    for (int k = 0; k < kItems; k++) {
-        if ((mask >> k) & 1) {
-            const int idx = threadIdx.x * kItems + k;
-            values[r] = buf[P(idx + 1)];
-            starts[r] = (uint32_t)(base + idx);
-            r++;
+    uint64_t r = s_prefix + block_exclusive_scan<uint64_t>((uint64_t)__popc(mask), &total, red);  // has barriers
+    if (next == ~0u) {  // uniform: the first later tile with a run has prefix[u + 1] > upto
+        const uint64_t upto = prefix[tile + 1];
+        size_t lo = tile + 1, hi = tiles;
+        while (lo < hi) {
+            const size_t mid = (lo + hi) / 2;
+            if (prefix[mid + 1] > upto)
+                hi = mid;
+            else
+                lo = mid + 1;
+        }
+        next = lo < tiles ? firsts[lo] : (uint32_t)n;
+    }
+    // the row that ends the thread's last run: the next thread's first start
+    for (int w = kBlock / kWave - 1; w > wave; w--) next = wave_first[w] != ~0u ? wave_first[w] : next;
+    const uint64_t later = holders & ~((2ull << lane) - 1);
+    const uint32_t in_wave = (uint32_t)__shfl((int)first, later ? __builtin_ctzll(later) : lane);
+    if (later) next = in_wave;
+    T vlo = std::numeric_limits<T>::max(), vhi = std::numeric_limits<T>::lowest();
+    int32_t llo = std::numeric_limits<int32_t>::max(), lhi = 0;
+    for (uint32_t m = mask; m; r++) {
+        const int k = __builtin_ctz(m);
+        m &= m - 1;
+        const T v = buf[P(threadIdx.x * kItems + k + 1)];
+        const int32_t l = (int32_t)((m ? row0 + __builtin_ctz(m) : next) - (row0 + k));
+        values[r] = v;
+        lengths[r] = l;
+        vlo = v < vlo ? v : vlo;
+        vhi = v > vhi ? v : vhi;
+        llo = l < llo ? l : llo;
+        lhi = l > lhi ? l : lhi;
+    }
+    if (holders) {
+        // in the types' own width: keys of 64 bits take several times the steps
+        llo = wave_min(llo);
+        lhi = wave_max(lhi);
+        uint64_t vk[2] = {0, 0};
+        if constexpr (std::is_integral<T>::value) {
+            using W = std::conditional_t<sizeof(T) == 8, int64_t, int32_t>;
+            vk[0] = order_key((T)wave_min((W)vlo));
+            vk[1] = order_key((T)wave_max((W)vhi));
+        }
+        if (lane == 0) {
+            atomicMin(&mm[0], (unsigned long long)vk[0]);
+            atomicMax(&mm[1], (unsigned long long)vk[1]);
+            atomicMin(&mm[2], (unsigned long long)order_key(llo));
+            atomicMax(&mm[3], (unsigned long long)order_key(lhi));
         }
     }
-    if (threadIdx.x == 0 && base + cnt == n) d_runs[0] = s_prefix + total;
+    __syncthreads();
+    if (threadIdx.x < 4) st_agent(keys + 4 * (size_t)tile + threadIdx.x, (uint64_t)mm[threadIdx.x]);
+    if (!tickets || !last_of_grid(tickets, &last)) return;
+    rle_to_host(mm, keys, tiles, prefix[tiles], host);
 }
 
-__global__ __launch_bounds__(kBlock) void k_rle_lengths(const uint32_t* __restrict__ starts, const uint64_t* d_runs,
-                                                        size_t n, int32_t* __restrict__ lengths) {
-    const size_t runs = *d_runs;
-    const size_t stride = (size_t)gridDim.x * kBlock;
-    for (size_t r = (size_t)blockIdx.x * kBlock + threadIdx.x; r < runs; r += stride) {
-        const uint64_t e = r + 1 < runs ? starts[r + 1] : n;
-        lengths[r] = (int32_t)(e - starts[r]);
-    }
+// The fold of more tiles than a tail pays for: up to 64 workgroups, the last
+// of which folds theirs.
+__global__ __launch_bounds__(kBlock) void k_rle_fold(const uint64_t* __restrict__ keys, size_t tiles,
+                                                     const uint64_t* __restrict__ runs, uint64_t* partials,
+                                                     uint32_t* tickets, HostOut host) {
+    __shared__ unsigned long long mm[4];
+    __shared__ bool last;
+    fold_keys(mm, keys, tiles, (size_t)blockIdx.x * kBlock + threadIdx.x, (size_t)gridDim.x * kBlock);
+    __syncthreads();
+    if (threadIdx.x < 4) st_agent(partials + 4 * blockIdx.x + threadIdx.x, (uint64_t)mm[threadIdx.x]);
+    if (!last_of_grid(tickets, &last)) return;
+    rle_to_host(mm, partials, gridDim.x, *runs, host);
 }
 
 // Run length r of an RLE stream at any byte address; a negative length is
@@ -1475,7 +1602,7 @@ void launch_merge_codes(Ctx* c, int dtype, const uint8_t* bits, size_t n, const 
 
 
 
-uint64_t launch_rle_encode(Ctx* c, int dtype, const void* x, size_t n, int32_t* lengths, void* values, uint64_t* d_runs,
+uint64_t launch_rle_encode(Ctx* c, int dtype, const void* x, size_t n, int32_t* lengths, void* values,
                            MinMaxResult* h_values, MinMaxResult* h_lengths) {
     if (n == 0) return 0;
     if (n >= (1ull << 31)) fail(DDJ_EUNSUPPORTED, "RLE run lengths are int32 (reference rle_encoding.hpp:35)");
@@ -1483,38 +1610,31 @@ uint64_t launch_rle_encode(Ctx* c, int dtype, const void* x, size_t n, int32_t* 
         using T = decltype(tag);
         const size_t tiles = (n + kTile - 1) / kTile;
         TileScan ts(c, tiles);
+        DevBuf firsts(c, 4 * tiles), keys(c, 32 * tiles);
         kernel_bytes(c, "k_rle_count", (double)n * sizeof(T));
         const ScanTail st = ts.tail(c, false);
         { KernelTimer kt_(c, "k_rle_count"); hipLaunchKernelGGL(k_rle_count<T>, dim3((unsigned)tiles), dim3(kBlock), 0, c->stream,
-                           static_cast<const T*>(x), n, ts.vals, st); }
+                           static_cast<const T*>(x), n, ts.vals, firsts.get<uint32_t>(), st); }
         HIPC(hipGetLastError());
         ts.finish(c, st);
-        DevBuf starts(c, 4 * n);
+        const HostOut ho = host_out(c);
         { KernelTimer kt_(c, "k_rle_encode"); hipLaunchKernelGGL(k_rle_encode<T>, dim3((unsigned)tiles), dim3(kBlock), 0, c->stream,
-                           static_cast<const T*>(x), n, static_cast<T*>(values), starts.get<uint32_t>(),
-                           (const uint64_t*)ts.prefix, d_runs); }
+                           static_cast<const T*>(x), n, tiles, static_cast<T*>(values), lengths,
+                           (const uint64_t*)ts.prefix, firsts.get<uint32_t>(), keys.get<uint64_t>(), st.tickets, ho); }
         HIPC(hipGetLastError());
-        // lengths (and the outputs' min/max) over the run count the device
-        // holds, so that one read-back brings everything the next nodes need
-        { KernelTimer kt_(c, "k_rle_lengths"); hipLaunchKernelGGL(k_rle_lengths, dim3(grid_for(c, n)), dim3(kBlock), 0, c->stream,
-                           starts.get<uint32_t>(), (const uint64_t*)d_runs, n, lengths); }
-        HIPC(hipGetLastError());
-        // the two min/max reductions' partials come back with the run count
-        // and are folded on the host
-        const bool mv = h_values && std::is_integral<T>::value;
-        DevBuf pv, pl;
-        const int gv = mv ? launch_minmax_partials(c, dtype, values, n, d_runs, pv) : 0;
-        const int gl = h_lengths ? launch_minmax_partials(c, DDJ_D_INT, lengths, n, d_runs, pl) : 0;
-        std::vector<uint64_t> hv(3 * (size_t)gv), hl(3 * (size_t)gl);
-        uint64_t runs = 0;
-        ReadBack rb[3] = {{&runs, d_runs, 8}, {nullptr, nullptr, 0}, {nullptr, nullptr, 0}};
-        size_t k = 1;
-        if (mv) rb[k++] = ReadBack{hv.data(), pv.get(), 8 * hv.size()};
-        if (h_lengths) rb[k++] = ReadBack{hl.data(), pl.get(), 8 * hl.size()};
-        d2h_many(c, rb, k);
-        if (mv) *h_values = fold_minmax_partials(hv.data(), gv, 3);
-        if (h_lengths) *h_lengths = fold_minmax_partials(hl.data(), gl, 3);
-        return runs;
+        if (!st.tickets) {
+            const unsigned grid = (unsigned)std::min<size_t>(64, (tiles + kBlock - 1) / kBlock);
+            DevBuf partials(c, 32 * grid);
+            { KernelTimer kt_(c, "k_rle_fold"); hipLaunchKernelGGL(k_rle_fold, dim3(grid), dim3(kBlock), 0, c->stream,
+                               keys.get<uint64_t>(), tiles, (const uint64_t*)(ts.prefix + tiles), partials.get<uint64_t>(),
+                               c->control->tickets, ho); }
+            HIPC(hipGetLastError());
+        }
+        RleResult r;
+        memcpy(&r, wait_host_out(c, ho), sizeof r);
+        if (h_values) *h_values = r.values;
+        if (h_lengths) *h_lengths = r.lengths;
+        return r.runs;
     });
 }
 

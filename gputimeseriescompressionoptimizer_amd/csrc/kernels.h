@@ -92,11 +92,6 @@ FloatScanResult float_scan(Ctx* c, int dtype, const void* x, size_t n);
 HostOut launch_minmax(Ctx* c, int dtype, const void* x, size_t n, bool delta, MinMaxResult* d_result);
 MinMaxResult wait_minmax(Ctx* c, const HostOut& h);
 MinMaxResult minmax_to_host(Ctx* c, int dtype, const void* x, size_t n, bool delta);
-// The reduction alone (integer columns, rows from *d_rows when given):
-// `partials` receives 3 order keys per workgroup, of which the returned
-// count; fold_minmax_partials folds them (stride 3; 2 for delta) on the host.
-int launch_minmax_partials(Ctx* c, int dtype, const void* x, size_t n, const uint64_t* d_rows, DevBuf& partials);
-MinMaxResult fold_minmax_partials(const uint64_t* h, int grid, int stride);
 // The few bytes of a blob around its streams (node headers, metadata), written
 // by one more workgroup of the kernel that writes a stream, from the kernel's
 // arguments: a gather launch of their own, its table read over PCIe, was 4.7
@@ -273,7 +268,7 @@ void launch_merge_codes(Ctx* c, int dtype, const uint8_t* stencil_bits, size_t n
 // Returns the run count (one read-back, which also brings the min/max of the
 // values and of the lengths into *h_values / *h_lengths when those are set;
 // values: integer types only).
-uint64_t launch_rle_encode(Ctx* c, int dtype, const void* x, size_t n, int32_t* lengths, void* values, uint64_t* d_runs,
+uint64_t launch_rle_encode(Ctx* c, int dtype, const void* x, size_t n, int32_t* lengths, void* values,
                            MinMaxResult* h_values = nullptr, MinMaxResult* h_lengths = nullptr);
 DevBuf rle_decode_dev(Ctx* c, int dtype, const uint8_t* lengths, const uint8_t* values, size_t runs);
 

@@ -272,3 +272,21 @@ def test_precision_of_late_rows(ctx, dtype, n):
     x[n // 2] = np.nan
     outs = [o.to_bytes() for o in g.Encoding(ctx, g.FLOAT_TO_INT).Encode(ctx.upload(x), dtype)]
     assert outs == O.encode(g.FLOAT_TO_INT, dtype, x)
+
+
+# 4096 rows a tile: runs that start, end and stretch at and over the tiles'
+# edges, tiles without a run's start, and more tiles than a tail folds (4096)
+@pytest.mark.parametrize("dtype", INT_TYPES + [g.D_FLOAT, g.D_DOUBLE])
+@pytest.mark.parametrize("n", [1, 4_096, 4_097, 40_961, 2_000_001, 4_096 * 4_097 + 5])
+def test_runs_over_tiles(ctx, dtype, n):
+    npdt = g.NP_DTYPE[dtype]
+    starts = {0, 4_095, 4_096, 8_193, 12_288, 12_289, 32_768, 40_960, 1_048_576, 4_096 * 4_096, n - 1}
+    starts |= set(range(49_152, 53_248, 3))  # one tile of short runs
+    starts = np.array(sorted(s for s in starts if 0 <= s < n))
+    keys = (np.arange(starts.size) * 37 % 101 - 50).astype(npdt)
+    x = np.repeat(keys, np.diff(np.append(starts, n)))
+    path = [g.RLE, g.AFL, g.NONE, g.AFL, g.NONE] if dtype in INT_TYPES else [g.RLE, g.AFL, g.NONE, g.NONE]
+    tree = g.CompressionTree(ctx, path, dtype)
+    blob = tree.Compress(ctx.upload(x))
+    assert blob.to_bytes() == O.compress(O.tree_from_path(path, dtype), x)
+    assert np.array_equal(tree.Decompress(blob).to_numpy(npdt), x)
