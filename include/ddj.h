@@ -6,7 +6,10 @@
  * src/).  Every entry point takes plain pointers and sizes; device buffers
  * are ddj_buf handles allocated from the context's caching allocator.  All
  * GPU work of a context runs on its own HIP stream; calls on one context
- * are serialised by the caller, separate contexts are independent.
+ * are serialised by the caller, separate contexts are independent.  A call
+ * may return with its last kernels still queued on that stream: copies to the
+ * host through this interface come after them, and a caller's own stream waits
+ * on ddj_ctx_stream.
  *
  * Status codes replace the reference's exit(1) / print-and-continue error
  * handling (core/macros.h:8-17).
