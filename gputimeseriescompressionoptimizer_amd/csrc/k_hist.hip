@@ -197,7 +197,7 @@ constexpr int kHistThreads = 1024;
 // kCopies copies of the window, lane l in copy l % kCopies: no key compare, no
 // probing, and few lanes of a wave on one bank.  The count of the 64M-row
 // Zipf(1.2)/50 column was bound by the probe loop's instructions and the LDS
-// atomics' same-address conflicts (92 us); with the window it takes 45, against
+// atomics' same-address conflicts (92 us); with the window it takes 53, against
 // 42 for a plain pass over the column.
 constexpr int kWindow = 1024, kCopies = 8;
 
@@ -945,7 +945,7 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
             DevBuf segs(c, sizeof(Entry) * part_slots<T>() * kHistParts * g), off(c, 4 * (kHistParts + 1) * g);
             // up to 64 workgroups (1M rows) the last of them merges (50 codes:
             // one launch of 22 us for two of 9 + 16); more of them have too many
-            // entries for one workgroup (64M rows 70 us, two launches 45 + 19)
+            // entries for one workgroup (64M rows 70 us, two launches 53 + 17)
             HistTail tail;
             if (g <= 64) tail = HistTail{c->control->tickets, K, host_out(c)};
             {

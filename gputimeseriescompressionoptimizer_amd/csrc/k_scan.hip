@@ -1031,9 +1031,10 @@ __device__ __forceinline__ void rle_to_host(unsigned long long* mm, const uint64
 // waves' firsts), a tile's last run where the next tile that starts one does
 // (firsts, found through the prefixes when the very next tile starts none).
 // The outputs' min/max keys come along: with a tail the last workgroup folds
-// them and hands them to the host with the run count.  Bound by the tile's
-// chain of latencies at 8 workgroups per CU (LDS: compacting the starts there
-// first left 6, 62 us for 64M int32 rows).
+// them and hands them to the host with the run count.  Bound by vector
+// instructions (43 us of issue of its 52 us for 64M int32 rows); 45 us without
+// lengths and keys, which then took four launches and 18 us.  Compacting the
+// starts in LDS first leaves 6 instead of 8 workgroups per CU: 62 us.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_rle_encode(const T* __restrict__ x, size_t n, size_t tiles,
                                                        T* __restrict__ values, int32_t* __restrict__ lengths,
