@@ -163,10 +163,17 @@ __device__ void block_small4(Small4& s, uint64_t* sm_keys /* NT/kWave * kMaxK */
 }
 
 // The counting workgroup's hash table: kHistParts partitions of 192 slots of
-// 4-byte keys (narrower types widened) or 128 of 8-byte keys.  A multiplicative
-// hash of the key's folded halves (cheaper than hmix's 64-bit multiplies, which
-// the other tables keep) gives the partition and the slot to start from;
-// probing stays inside the partition.
+// 4-byte keys (narrower types widened) or 128 of 8-byte keys.  A hash of the
+// key's folded halves in 32 bits (cheaper than hmix's 64-bit multiplies, which
+// the other tables keep) gives the partition and the slot to start from; probing
+// stays inside the partition.
+//
+// SPREAD: one multiplication, which lays whole numbers in a row (codes, ids)
+// out evenly, so that 10,000 of them fill the table without long probes (16M
+// rows of them 57 us, with the mix 332).  But it packs the rows of some arithmetic
+// progressions (strides 10946, 50549, ...; sampled times are such columns) into
+// one end of a table: 10,000 of them took 3000-4700 probes a row.  Where nothing
+// comes after it that would count such columns, the hash is a mix.
 template <typename T> using HistKey = typename std::conditional<sizeof(T) == 8, unsigned long long, uint32_t>::type;
 constexpr int kHistParts = 64;
 template <typename T> constexpr int part_slots() { return sizeof(T) == 8 ? 128 : 192; }
@@ -175,9 +182,12 @@ template <typename KT> struct HistEntry {
     KT key;
     uint32_t count;
 };
-__device__ __forceinline__ uint32_t lds_hash(uint64_t key) {
-    const uint32_t a = (uint32_t)key ^ ((uint32_t)(key >> 32) * 0x85ebca6bu);
-    return a * 0x9E3779B1u;
+template <bool SPREAD> __device__ __forceinline__ uint32_t lds_hash(uint64_t key) {
+    uint32_t a = (uint32_t)key ^ ((uint32_t)(key >> 32) * 0x85ebca6bu);
+    if (SPREAD) return a * 0x9E3779B1u;
+    a = (a ^ (a >> 16)) * 0x85ebca6bu;
+    a = (a ^ (a >> 13)) * 0xc2b2ae35u;
+    return a ^ (a >> 16);
 }
 
 // What a counting workgroup saw outside its tables.
@@ -398,7 +408,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
     // Adds `add` rows of `key` to its partition; a key without a slot goes to
     // the global table, or ends the count.
     auto lds_add = [&](KT key, uint32_t add) {
-        const uint64_t at = (uint64_t)lds_hash((uint64_t)key) * kHistParts;
+        const uint64_t at = (uint64_t)lds_hash<true>((uint64_t)key) * kHistParts;
         const uint32_t base = (uint32_t)(at >> 32) * PS;
         uint32_t h = (uint32_t)(((uint64_t)(uint32_t)at * PS) >> 32);
         for (int p = 0; p < 24; p++) {
@@ -610,7 +620,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
                 const HistEntry<KT>* en = segs + (size_t)w * kLdsSlots + (e - first[w]);
                 const KT key = ld_agent(&en->key);
                 const uint32_t c = ld_agent(&en->count);
-                uint32_t s = (uint32_t)(((uint64_t)lds_hash((uint64_t)key) * kLdsSlots) >> 32);
+                uint32_t s = (uint32_t)(((uint64_t)lds_hash<true>((uint64_t)key) * kLdsSlots) >> 32);
                 int left = 256;
                 for (; left > 0; left--) {
                     KT k = skey[s];
@@ -785,10 +795,14 @@ __global__ __launch_bounds__(kBlock) void k_hist_topk(GlobalTable table, int K, 
 // Columns of a few thousand rows (the planner's samples): one workgroup
 // counts every row in an LDS table that can hold them all distinct, takes the
 // best K and hands them to the host: one launch for four (table fill, count,
-// top-K, read-back), and no device-scope atomics (10,000 distinct int32 rows:
-// 2 + 45 + 9 us and three launches, now 21 us).  The limits keep the table at
+// top-K, read-back), and no device-scope atomics (10,000 distinct int32 rows by
+// HIP events: 7 + 90 + 24 us in three launches, now 34).  The limits keep the table at
 // most 2/3 full (8-byte keys 5/6, which is what LDS allows a 10,000-row
-// sample).
+// sample).  The probes' step is the key's own (6 k + 1, which has no factor in
+// common with the 2^a 3^b slots, so that it visits all of them); a key without a
+// slot after kSmallProbes of them, which takes keys made for it, has the
+// column counted by the other kernels.
+constexpr int kSmallProbes = 512;
 template <typename T> constexpr int small_slots() { return sizeof(T) == 8 ? 12288 : 18432; }
 template <typename T> constexpr size_t small_rows() { return sizeof(T) == 8 ? 10240 : 12288; }
 
@@ -797,18 +811,19 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_small(const T* __restrict
     using KT = HistKey<T>;
     constexpr KT kFree = (KT)~(KT)0;  // an empty slot; rows of that bit pattern are counted on the side
     constexpr int S = small_slots<T>(), W = kHistThreads / kWave;
+    static_assert(S == 12288 || S == 18432, "no prime factors but 2 and 3; steps are shorter");
     __shared__ KT skey[S];
     __shared__ uint32_t scnt[S];
     __shared__ Cand sc[W * kMaxK];
     __shared__ Cand best[kMaxK];
     __shared__ uint64_t s_nk[W * kMaxK], nan_keys[kMaxK];
     __shared__ int s_nc[W];
-    __shared__ uint32_t nan_n, s_distinct, s_special, s_nans, s_negzero;
+    __shared__ uint32_t nan_n, s_distinct, s_special, s_nans, s_negzero, s_over;
     for (int i = threadIdx.x; i < S; i += kHistThreads) {
         skey[i] = kFree;
         scnt[i] = 0;
     }
-    if (threadIdx.x == 0) s_distinct = s_special = s_nans = s_negzero = nan_n = 0;
+    if (threadIdx.x == 0) s_distinct = s_special = s_nans = s_negzero = s_over = nan_n = 0;
     __syncthreads();
     bool negzero = false;
     uint32_t special = 0, nans = 0, distinct = 0;
@@ -835,17 +850,19 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_small(const T* __restrict
             special++;
             continue;
         }
-        uint32_t s = (uint32_t)(((uint64_t)lds_hash((uint64_t)key) * S) >> 32);
-        // at most n < S keys: a free slot or the key itself is always found
-        for (;;) {
+        const uint32_t h = lds_hash<false>((uint64_t)key), step = 6 * (h & 255) + 1;
+        uint32_t s = (uint32_t)(((uint64_t)h * S) >> 32);
+        int left = kSmallProbes;
+        for (; left > 0; left--) {
             KT k = skey[s];
             if (k == kFree) k = atomicCAS(&skey[s], kFree, key);
             if (k == kFree || k == key) {
                 atomicAdd(&scnt[s], 1u);
                 break;
             }
-            s = s + 1 < (uint32_t)S ? s + 1 : 0;
+            s = s + step < (uint32_t)S ? s + step : s + step - S;
         }
+        if (left == 0) s_over = 1;
     }
     __syncthreads();
     Cand top[kMaxK];
@@ -880,7 +897,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_small(const T* __restrict
         for (uint32_t r = 0; r < nan_n; r++)  // every NaN row is a bin of count 1
             push<T>(b, K, Cand{1ull, ubits(from_order_key<T>(nan_keys[r]))});
         HistResult* out = reinterpret_cast<HistResult*>(host.dst);
-        out->ctl = HistCtl{s_distinct, s_special, s_nans, 0, 0, s_negzero};
+        out->ctl = HistCtl{s_distinct, s_special, s_nans, 0, s_over ? kTooSmall : 0u, s_negzero};
 #pragma unroll
         for (int i = 0; i < kMaxK; i++) out->top[i] = b[i];
     }
@@ -934,7 +951,7 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
             }
             HIPC(hipGetLastError());
             memcpy(&found, wait_host_out(c, ho), sizeof found);
-            return take(found);
+            if (!found.ctl.overflow) return take(found);
         }
         size_t g = (n + 16 * kHistThreads - 1) / (16 * kHistThreads);  // at most one workgroup per tile and per CU
         g = std::max<size_t>(1, std::min<size_t>(g, (size_t)c->cu_count));

@@ -92,6 +92,48 @@ def test_most_frequent_all_counts_tie(ctx):
     assert sorted(np.frombuffer(meta[16:32], np.int32)) == [-50_000, -49_999, -49_998, -49_997]
 
 
+def _hist_ms(ctx, x, dtype):
+    """The histogram kernels' time in one dictionary encode, the least of five."""
+    buf, enc = ctx.upload(x), g.Encoding(ctx, g.DICT)
+    enc.Encode(buf, dtype)
+    best = math.inf
+    ctx.profile(True)
+    for _ in range(5):
+        ctx.profile_reset()
+        enc.Encode(buf, dtype)
+        best = min(best, sum(t[0] for k, t in ctx.kernel_table().items() if k.startswith("k_hist")))
+    ctx.profile(False)
+    return best
+
+
+# strides that one multiplication by the golden ratio's bits packs together
+@pytest.mark.parametrize("stride", [1, 5_473, 10_946, 50_549, 61_495])
+@pytest.mark.parametrize("dtype", [g.D_INT, g.D_TIME])
+@pytest.mark.parametrize("distinct,n", [(10_000, 10_000)])
+def test_most_frequent_of_arithmetic_progressions(ctx, dtype, stride, distinct, n):
+    """Right, and no slower than random keys: 3 is far above the spread of a
+    kernel's time and far below what clustered keys cost (5 to 200)."""
+    npdt = g.NP_DTYPE[dtype]
+    r = np.random.default_rng(stride)
+    at = np.arange(n) if n == distinct else r.integers(0, distinct, n)
+    x = (1_400_000_000 + at * stride).astype(npdt)
+    assert [o.to_bytes() for o in g.Encoding(ctx, g.DICT).Encode(ctx.upload(x), dtype)] == O.encode(g.DICT, dtype, x)
+    other = r.choice(np.iinfo(npdt).max, distinct, replace=False) if dtype == g.D_INT else \
+        np.unique(r.integers(0, np.iinfo(npdt).max, distinct + 10))[:distinct]
+    assert _hist_ms(ctx, x, dtype) <= 3 * _hist_ms(ctx, r.permutation(other)[at].astype(npdt), dtype)
+
+
+@pytest.mark.parametrize("n", [10_000, 40_000])
+def test_most_frequent_of_keys_with_one_hash(ctx, n):
+    """Keys whose folded halves are equal start at one slot with one step; each
+    table gives up on them in turn, up to the one that takes every column."""
+    hi = np.arange(1, n + 1, dtype=np.uint64)
+    lo = (hi * np.uint64(0x85EBCA6B) ^ np.uint64(0x1234567)) & np.uint64(0xFFFFFFFF)
+    x = np.random.default_rng(n).permutation(((hi << np.uint64(32)) | lo).astype(np.int64))
+    x[::7] = x[3]
+    assert [o.to_bytes() for o in g.Encoding(ctx, g.DICT).Encode(ctx.upload(x), g.D_TIME)] == O.encode(g.DICT, g.D_TIME, x)
+
+
 # 4096-row tiles; up to 1024 of them are scanned by the counting pass's last
 # workgroup (its ticket groups begin past 64), more by a launch of their own
 @pytest.mark.parametrize("tiles", [1, 2, 64, 65, 1_023, 1_024, 1_025])
