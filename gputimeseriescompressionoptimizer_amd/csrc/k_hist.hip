@@ -5,14 +5,15 @@
 // reference's stable sort of key-sorted bins yields).
 //
 // Counting: each workgroup aggregates its rows in LDS (plain LDS atomics; the
-// 16 rows a thread loads at once keep HBM busy while they wait): integers
+// up to 16 rows a thread loads at once keep HBM busy while they wait): integers
 // near the first row by offset, other keys in a hash table of kHistParts
 // partitions, each key's partition fixed by its hash.  The workgroups write
 // their keys and counts out; the last of them adds them up in LDS if they are
 // few, else k_hist_merge does, one workgroup per partition, so that no key is
-// counted through device-scope atomics.  A column with more distinct keys than these tables
-// hold is counted again into a global open-addressing table (64-bit keys, ~0 =
-// empty).  A value equal to a table's empty marker is counted on the side.
+// counted through device-scope atomics.  A column with more distinct keys than
+// these tables hold is counted again by more workgroups of fewer rows each,
+// and, past what those or the merge's tables hold, into a global
+// open-addressing table (64-bit keys, ~0 = empty).  A value equal to a table's empty marker is counted on the side.
 // Floats count -0.0 with +0.0 (operator==), reporting -0.0 when one was seen
 // (it sorts first in the reference).  A NaN equals nothing, so each NaN row is
 // a bin of count 1: they stay out of the tables, and every workgroup keeps the
@@ -198,9 +199,24 @@ struct HistInfo {
     uint64_t nan_keys[kMaxK];
 };
 
-// Workgroups of 1024 threads, one per CU, stride over tiles of 16384 rows,
-// each thread taking 16 rows with their loads issued together.
+// Workgroups of 1024 threads, one per CU, stride over tiles of 16 rows a
+// thread, whose loads are issued together.
+//
+// Columns that leave a workgroup no more than few_rows a thread are counted in
+// tiles of that many, one a workgroup: distinct or not, their keys fit its table
+// (two thirds and half of its slots), so that only the merge's tables can be
+// too small.  With 16 rows a thread every column of more than 5,500 random keys
+// (3,500 of 8 bytes) was counted in vain and then again in the global table.  A
+// dictionary encode of 100,000 int32 rows with 16,000 keys 231 us, of int64 rows
+// 251, now 85 and 81 (in the global table alone 184 and 185); of 1M rows with
+// 60,000 keys 1187 and 1247, now 126 and 106; of 100,000 rows with 50 keys 55 and
+// 56, now 52.
 constexpr int kHistThreads = 1024;
+template <typename T> constexpr int few_rows() { return sizeof(T) == 8 ? 4 : sizeof(T) == 1 ? 16 : 8; }
+// Entries a workgroup may write out.
+template <typename T, int PER> constexpr int seg_slots() {
+    return PER < 16 ? PER * kHistThreads : kHistParts * part_slots<T>();
+}
 
 // Integer columns: keys within kWindow / 2 of the first row's (dictionary
 // codes, categories, most small integers) are counted by their offset, in
@@ -358,19 +374,20 @@ __device__ __forceinline__ uint32_t segment_of(const uint32_t* first, uint32_t s
 
 // GLOBAL: the tables are flushed into, and keys without a slot added to, the
 // global table, which k_hist_topk searches.  Else the workgroup's used slots
-// go to segs (its kHistParts * part_slots entries from blockIdx.x on, partition
+// go to segs (its seg_slots entries from blockIdx.x on, partition
 // by partition, partition p from off[p * grid + workgroup] on), and a key
 // without a slot ends the count (info[].overflow: the host counts again with
 // GLOBAL).  With a tail, if all workgroups' entries are few (columns of few
 // distinct values), the last workgroup adds them up itself and hands the best K
-// to the host; else (kNeedMerge) k_hist_merge does.
-constexpr uint32_t kTailEntries = 8192;
+// to the host; else (kNeedMerge) k_hist_merge does (1M int32 rows of 130 values,
+// 16,000 entries: 37 us, in two launches 42).
+constexpr uint32_t kTailEntries = 16384;
 struct HistTail {
     uint32_t* tickets = nullptr;
     int K = 0;
     HostOut host;
 };
-template <typename T, bool GLOBAL>
+template <typename T, int PER, bool GLOBAL>
 __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict__ x, size_t n, GlobalTable table,
                                                              HistEntry<HistKey<T>>* __restrict__ segs,
                                                              uint32_t* __restrict__ off, HistInfo* __restrict__ info,
@@ -405,13 +422,19 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
     Small4 nan4;
     unsigned long long special = 0, nans = 0;
     bool negzero = false;
+    // Probes for a slot: with few rows, whose keys all have one, the whole
+    // partition; 48 let 7,500 random keys of 4 bytes and 5,000 of 8 find one (24:
+    // 5,500 and 3,500; 96: 500 more, but a table that overflows all the same does
+    // so after twice the time); before the global table, which most rows of a
+    // column with that many keys end up in anyway, 8 (24: 30 us more of 270).
+    constexpr int probes = GLOBAL ? 8 : PER < 16 ? PS : 48;
     // Adds `add` rows of `key` to its partition; a key without a slot goes to
     // the global table, or ends the count.
     auto lds_add = [&](KT key, uint32_t add) {
-        const uint64_t at = (uint64_t)lds_hash<true>((uint64_t)key) * kHistParts;
+        const uint64_t at = (uint64_t)lds_hash<(PER == 16 && !GLOBAL)>((uint64_t)key) * kHistParts;
         const uint32_t base = (uint32_t)(at >> 32) * PS;
         uint32_t h = (uint32_t)(((uint64_t)(uint32_t)at * PS) >> 32);
-        for (int p = 0; p < 24; p++) {
+        for (int p = 0; p < probes; p++) {
             const uint32_t s = base + h;
             h = h + 1 < (uint32_t)PS ? h + 1 : 0;
             KT k = skey[s];
@@ -465,13 +488,14 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
             lds_add(key, 1u);
         }
     };
-    constexpr int kPer = 16, kRows = kPer * kHistThreads;
+    auto gave_up = [&] { return !GLOBAL && *(volatile uint32_t*)&s_over != 0; };
+    constexpr int kPer = PER, kRows = kPer * kHistThreads;
     constexpr int V = 16 / sizeof(T);
     constexpr int Q = kRows / V / kHistThreads;  // 16-byte loads per thread and tile
     const size_t tiles = (n + kRows - 1) / kRows;
     const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
     for (size_t t = blockIdx.x; t < tiles; t += gridDim.x) {  // uniform per workgroup
-        if (!GLOBAL && *(volatile uint32_t*)&s_over) break;  // (each wave by itself: the count is dropped)
+        if (gave_up()) break;  // (each wave by itself: the count is dropped)
         const size_t base = t * kRows;
         if (aligned && base + kRows <= n) {
             const u32x4* s4 = reinterpret_cast<const u32x4*>(x + base);
@@ -480,6 +504,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
             for (int q = 0; q < Q; q++) w[q] = s4[threadIdx.x + kHistThreads * q];
 #pragma unroll
             for (int q = 0; q < Q; q++) {
+                if (Q >= 4 && q == Q / 2 && gave_up()) break;
                 T v[V];
                 __builtin_memcpy(v, &w[q], 16);
 #pragma unroll
@@ -494,8 +519,10 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
                 if (i < cnt) v[k] = x[base + i];
             }
 #pragma unroll
-            for (int k = 0; k < kPer; k++)
+            for (int k = 0; k < kPer; k++) {
+                if (k == kPer / 2 && gave_up()) break;
                 if ((int)threadIdx.x + k * kHistThreads < cnt) count(v[k]);
+            }
         }
     }
     if (rk0 != kFree) lds_add(rk0, rc0);
@@ -549,7 +576,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
             if (lane == kWave - 1) s_off[kHistParts] = upto;
         }
         __syncthreads();
-        HistEntry<KT>* mine = segs + (size_t)blockIdx.x * kLdsSlots;
+        HistEntry<KT>* mine = segs + (size_t)blockIdx.x * seg_slots<T, PER>();
         for (int p = wid; p < kHistParts; p += kHistThreads / kWave) {
             uint32_t at = s_off[p];
 #pragma unroll
@@ -614,27 +641,39 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
         fold_info<kHistThreads>(info, blocks, &ctl);
         HistResult* out = reinterpret_cast<HistResult*>(tail.host.dst);
         const bool few = total <= kTailEntries && n < (1ull << 32);
-        if (few)
-            for (uint32_t e = threadIdx.x; e < total; e += kHistThreads) {
-                const uint32_t w = segment_of(first, blocks, e);
-                const HistEntry<KT>* en = segs + (size_t)w * kLdsSlots + (e - first[w]);
-                const KT key = ld_agent(&en->key);
-                const uint32_t c = ld_agent(&en->count);
-                uint32_t s = (uint32_t)(((uint64_t)lds_hash<true>((uint64_t)key) * kLdsSlots) >> 32);
+        constexpr int F = 4;  // entries in flight a thread
+        for (uint32_t e0 = threadIdx.x; few && e0 < total; e0 += F * kHistThreads) {
+            KT key[F];
+            uint32_t cnt[F];
+#pragma unroll
+            for (int f = 0; f < F; f++) {
+                const uint32_t e = e0 + f * kHistThreads;
+                cnt[f] = 0;
+                if (e < total) {
+                    const uint32_t w = segment_of(first, blocks, e);
+                    const HistEntry<KT>* en = segs + (size_t)w * seg_slots<T, PER>() + (e - first[w]);
+                    key[f] = ld_agent(&en->key);
+                    cnt[f] = ld_agent(&en->count);
+                }
+            }
+#pragma unroll
+            for (int f = 0; f < F; f++) {
+                if (!cnt[f]) continue;
+                uint32_t s = (uint32_t)(((uint64_t)lds_hash<false>((uint64_t)key[f]) * kLdsSlots) >> 32);
                 int left = 256;
                 for (; left > 0; left--) {
                     KT k = skey[s];
-                    if (k == kFree) k = atomicCAS(&skey[s], kFree, key);
-                    if (k == kFree || k == key) {
-                        atomicAdd(&scnt[s], c);
+                    if (k == kFree) k = atomicCAS(&skey[s], kFree, key[f]);
+                    if (k == kFree || k == key[f]) {
+                        atomicAdd(&scnt[s], cnt[f]);
                         break;
                     }
                     s = s + 1 < (uint32_t)kLdsSlots ? s + 1 : 0;
                 }
                 if (left == 0) atomicOr(&ctl.overflow, kNeedMerge);
             }
-        else if (threadIdx.x == 0)
-            atomicOr(&ctl.overflow, kNeedMerge);
+        }
+        if (!few && threadIdx.x == 0) atomicOr(&ctl.overflow, kNeedMerge);
         __syncthreads();
         if (ctl.overflow) {  // uniform
             if (threadIdx.x == 0) out->ctl = ctl;
@@ -685,12 +724,13 @@ constexpr int kMergeThreads = 1024, kMergeSlots = 4096;
 template <typename T>
 __global__ __launch_bounds__(kMergeThreads) void k_hist_merge(const HistEntry<HistKey<T>>* __restrict__ segs,
                                                               const uint32_t* __restrict__ off,
-                                                              const HistInfo* __restrict__ info, uint32_t blocks, int K,
+                                                              const HistInfo* __restrict__ info, uint32_t blocks,
+                                                              uint32_t slots /* entries a workgroup */, int K,
                                                               Cand* partials, uint32_t* part_ctl, uint32_t* tickets,
                                                               HostOut host) {
     using KT = HistKey<T>;
     constexpr KT kFree = (KT)~(KT)0;
-    constexpr int kSegSlots = kHistParts * part_slots<T>(), W = kMergeThreads / kWave;
+    constexpr int W = kMergeThreads / kWave;
     __shared__ __attribute__((aligned(16))) KT skey[kMergeSlots];
     __shared__ unsigned long long scnt[kMergeSlots];
     __shared__ Cand sc[W * kMaxK];
@@ -702,6 +742,18 @@ __global__ __launch_bounds__(kMergeThreads) void k_hist_merge(const HistEntry<Hi
     __shared__ uint32_t red[W];
     __shared__ bool last;
     const uint32_t* row = off + (size_t)blockIdx.x * blocks;  // blocks <= kMergeThreads
+    // a counting workgroup's table was too small (the same in every workgroup
+    // here): nothing to add up, and no tickets are taken
+    if (__syncthreads_or(threadIdx.x < blocks && info[threadIdx.x].overflow)) {
+        if (blockIdx.x != 0) return;
+        if (threadIdx.x == 0) {
+            ctl = HistCtl{};
+            ctl.overflow = kTooSmall;
+            reinterpret_cast<HistResult*>(host.dst)->ctl = ctl;
+        }
+        host_out_done(host);
+        return;
+    }
     const uint32_t at = threadIdx.x < blocks ? row[threadIdx.x] : 0u;
     const uint32_t mine = threadIdx.x < blocks ? row[blocks + threadIdx.x] - at : 0u;
     for (int i = threadIdx.x; i < kMergeSlots; i += kMergeThreads) {
@@ -726,7 +778,7 @@ __global__ __launch_bounds__(kMergeThreads) void k_hist_merge(const HistEntry<Hi
             en[f].count = 0;
             if (e < total) {
                 const uint32_t w = segment_of(first, blocks, e);
-                en[f] = segs[(size_t)w * kSegSlots + begin[w] + (e - first[w])];
+                en[f] = segs[(size_t)w * slots + begin[w] + (e - first[w])];
             }
         }
 #pragma unroll
@@ -953,22 +1005,27 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
             memcpy(&found, wait_host_out(c, ho), sizeof found);
             if (!found.ctl.overflow) return take(found);
         }
-        size_t g = (n + 16 * kHistThreads - 1) / (16 * kHistThreads);  // at most one workgroup per tile and per CU
-        g = std::max<size_t>(1, std::min<size_t>(g, (size_t)c->cu_count));
-        DevBuf info(c, sizeof(HistInfo) * g);
+        using Entry = HistEntry<HistKey<T>>;
         auto xs = static_cast<const T*>(x);
-        {
-            using Entry = HistEntry<HistKey<T>>;
-            DevBuf segs(c, sizeof(Entry) * part_slots<T>() * kHistParts * g), off(c, 4 * (kHistParts + 1) * g);
-            // up to 64 workgroups (1M rows) the last of them merges (50 codes:
-            // one launch of 22 us for two of 9 + 16); more of them have too many
-            // entries for one workgroup (64M rows 70 us, two launches 53 + 17)
+        // One count in tiles of PER rows a thread by at most max_g workgroups, and
+        // the merge: whether the tables held the keys.
+        auto counted = [&](auto per, size_t max_g) {
+            constexpr int PER = decltype(per)::value;
+            const size_t rows = (size_t)PER * kHistThreads, g = std::min((n + rows - 1) / rows, max_g);
+            // in four sizes, so that columns of every length share their blocks
+            size_t room = 16;
+            while (room < g) room *= 4;
+            DevBuf info(c, sizeof(HistInfo) * g), off(c, 4 * (kHistParts + 1) * g),
+                segs(c, sizeof(Entry) * seg_slots<T, PER>() * room);
+            // up to 1M rows of 4 bytes the last workgroup merges (50 codes: one launch
+            // of 22 us for two of 9 + 16); more workgroups have too many entries for
+            // one (64M rows 70 us, two launches 53 + 17)
             HistTail tail;
-            if (g <= 64) tail = HistTail{c->control->tickets, K, host_out(c)};
+            if (g <= (PER < 16 ? 128 : 64)) tail = HistTail{c->control->tickets, K, host_out(c)};
             {
                 KernelTimer kt_(c, "k_hist_count");
-                hipLaunchKernelGGL((k_hist_count<T, false>), dim3((unsigned)g), dim3(kHistThreads), 0, c->stream, xs, n,
-                                   GlobalTable{}, segs.get<Entry>(), off.get<uint32_t>(), info.get<HistInfo>(), tail);
+                hipLaunchKernelGGL((k_hist_count<T, PER, false>), dim3((unsigned)g), dim3(kHistThreads), 0, c->stream, xs,
+                                   n, GlobalTable{}, segs.get<Entry>(), off.get<uint32_t>(), info.get<HistInfo>(), tail);
             }
             HIPC(hipGetLastError());
             if (tail.tickets) memcpy(&found, wait_host_out(c, tail.host), sizeof found);
@@ -978,14 +1035,27 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
                 {
                     KernelTimer kt_(c, "k_hist_merge");
                     hipLaunchKernelGGL(k_hist_merge<T>, dim3(kHistParts), dim3(kMergeThreads), 0, c->stream,
-                                       segs.get<Entry>(), off.get<uint32_t>(), info.get<HistInfo>(), (uint32_t)g, K,
-                                       partials.get<Cand>(), part_ctl.get<uint32_t>(), c->control->tickets, ho);
+                                       segs.get<Entry>(), off.get<uint32_t>(), info.get<HistInfo>(), (uint32_t)g,
+                                       (uint32_t)seg_slots<T, PER>(), K, partials.get<Cand>(), part_ctl.get<uint32_t>(),
+                                       c->control->tickets, ho);
                 }
                 HIPC(hipGetLastError());
                 memcpy(&found, wait_host_out(c, ho), sizeof found);
             }
-            if (!found.ctl.overflow) return take(found);
+            return !found.ctl.overflow;
+        };
+        using Few = std::integral_constant<int, few_rows<T>()>;
+        const size_t few = (size_t)Few::value * kHistThreads, cus = std::min<size_t>(c->cu_count, kMergeThreads);
+        if (n <= few * cus) {
+            if (counted(Few{}, cus)) return take(found);
+        } else {
+            if (counted(std::integral_constant<int, 16>{}, cus)) return take(found);
+            // the merge takes the entries of up to kMergeThreads workgroups (4M int32
+            // rows of 30,000 keys 287 us, 422 through the global table)
+            if (Few::value < 16 && n <= few * kMergeThreads && counted(Few{}, kMergeThreads)) return take(found);
         }
+        const size_t g = std::min((n + 16 * kHistThreads - 1) / (16 * kHistThreads), cus);
+        DevBuf info(c, sizeof(HistInfo) * g);
         // more distinct keys than the LDS tables hold
         const uint64_t all_distinct = pow2_at_least(2 * (uint64_t)n + 2);
         uint64_t cap = std::min<uint64_t>(std::max<uint64_t>(1024, all_distinct), 1u << 16);
@@ -1001,7 +1071,7 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
             }
             {
                 KernelTimer kt_(c, "k_hist_count");
-                hipLaunchKernelGGL((k_hist_count<T, true>), dim3((unsigned)g), dim3(kHistThreads), 0, c->stream, xs, n,
+                hipLaunchKernelGGL((k_hist_count<T, 16, true>), dim3((unsigned)g), dim3(kHistThreads), 0, c->stream, xs, n,
                                    table, nullptr, nullptr, info.get<HistInfo>(), HistTail{});
             }
             HIPC(hipGetLastError());

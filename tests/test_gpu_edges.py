@@ -109,7 +109,7 @@ def _hist_ms(ctx, x, dtype):
 # strides that one multiplication by the golden ratio's bits packs together
 @pytest.mark.parametrize("stride", [1, 5_473, 10_946, 50_549, 61_495])
 @pytest.mark.parametrize("dtype", [g.D_INT, g.D_TIME])
-@pytest.mark.parametrize("distinct,n", [(10_000, 10_000)])
+@pytest.mark.parametrize("distinct,n", [(10_000, 10_000), (2_000, 100_000)])
 def test_most_frequent_of_arithmetic_progressions(ctx, dtype, stride, distinct, n):
     """Right, and no slower than random keys: 3 is far above the spread of a
     kernel's time and far below what clustered keys cost (5 to 200)."""
@@ -132,6 +132,43 @@ def test_most_frequent_of_keys_with_one_hash(ctx, n):
     x = np.random.default_rng(n).permutation(((hi << np.uint64(32)) | lo).astype(np.int64))
     x[::7] = x[3]
     assert [o.to_bytes() for o in g.Encoding(ctx, g.DICT).Encode(ctx.upload(x), g.D_TIME)] == O.encode(g.DICT, g.D_TIME, x)
+
+
+# 8,192 rows a workgroup (4,096 of 8 bytes) up to 256 of them; past that 16,384
+# first, and where its table does not hold the keys, 8,192 in up to 1024 workgroups
+@pytest.mark.parametrize("dtype,n,distinct,tables", [
+    (g.D_INT, 12_289, 12_289, True), (g.D_INT, 100_000, 16_000, True), (g.D_SHORT, 100_000, 60_000, True),
+    (g.D_INT, 256 * 8_192, 30_000, True), (g.D_INT, 256 * 8_192 + 1, 30_000, True),
+    (g.D_INT, 1_024 * 8_192, 12_000, True), (g.D_INT, 1_024 * 8_192 + 1, 12_000, False),
+    (g.D_TIME, 10_241, 10_241, True), (g.D_DOUBLE, 13_000, 13_000, True), (g.D_FLOAT, 300_000, 30_000, True),
+    (g.D_TIME, 256 * 4_096, 30_000, True), (g.D_TIME, 256 * 4_096 + 1, 30_000, True),
+    (g.D_DOUBLE, 1_024 * 4_096, 12_000, True), (g.D_TIME, 1_024 * 4_096 + 1, 12_000, False),
+])
+def test_most_frequent_of_many_keys(ctx, dtype, n, distinct, tables):
+    """Columns whose keys the workgroups' tables hold are not counted again in
+    the global one (k_hist_init empties that)."""
+    npdt = g.NP_DTYPE[dtype]
+    r = np.random.default_rng(n)
+    if dtype in (g.D_FLOAT, g.D_DOUBLE):
+        values = np.unique(r.standard_normal(distinct + 100).astype(npdt))
+    else:
+        i = np.iinfo(npdt)
+        values = np.unique(r.integers(i.min, i.max, 2 * distinct, dtype=npdt)) if dtype != g.D_SHORT else \
+            np.arange(-30_000, 30_000).astype(npdt)
+    values = r.permutation(values)[:distinct]
+    x = r.permutation(np.concatenate([values, values[r.integers(0, values.size, n - values.size)]]))
+    x[::113] = values[5]
+    x[7::211] = values[6]
+    buf, enc = ctx.upload(x), g.Encoding(ctx, g.DICT)
+    ctx.profile(True)
+    ctx.profile_reset()
+    meta = enc.Encode(buf, dtype)[1].to_bytes()
+    ran = ctx.kernel_table()
+    ctx.profile(False)
+    v, c = np.unique(x, return_counts=True)
+    want = [v[j] for j in np.lexsort((v, -c))[:4]]
+    assert sorted(np.frombuffer(meta[16:16 + 4 * npdt().itemsize], npdt)) == sorted(want)
+    assert ("k_hist_init" not in ran) == tables
 
 
 # 4096-row tiles; up to 1024 of them are scanned by the counting pass's last
