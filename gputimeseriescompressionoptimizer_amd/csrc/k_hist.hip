@@ -21,9 +21,10 @@
 // from them.  Columns of a few thousand rows are counted whole in one
 // workgroup's LDS (k_hist_small).  The global table starts at 2n slots (at
 // least 1024, at most 64K); if it ends up more than 70% full the host retries
-// once with a table of twice the keys seen (the exact count, or with a full
-// table the keys seen plus the rows it dropped, each possibly a new key), and
-// a second retry, never needed in practice, sizes it for every row distinct.
+// once with a table of twice the keys seen (the exact count, and with a full
+// table the HyperLogLog estimate of the keys that it turned away), and a second
+// retry, never needed in practice, sizes it for every row distinct.
+#include <cmath>
 #include <type_traits>
 
 #include "dispatch.h"
@@ -42,7 +43,6 @@ struct HistCtl {
     unsigned long long distinct;
     unsigned long long special;  // rows whose bit pattern (4- and 8-byte types) marks an empty slot
     unsigned long long nans;     // NaN rows (floats)
-    unsigned long long dropped;  // rows that found no slot in a full global table
     uint32_t overflow;           // kTooSmall: a table was; kNeedMerge
     uint32_t negzero;
 };
@@ -68,43 +68,66 @@ template <typename T> __device__ __forceinline__ uint64_t hist_key(T v, bool& ne
 
 // The global table.  New keys are counted per thread and summed (a counter
 // bumped once per new key serializes every workgroup on one address, which for
-// a column of 10^4 distinct rows was most of the count's time).  A table that fills is dropped and counted again in a larger one, so a thread that
-// once found no slot (no free one within kProbes: far past what a table
-// 70% full needs) only counts the rows it drops.
+// a column of 10^4 distinct rows was most of the count's time).  A table that
+// fills is dropped and counted again in a larger one, so a thread that once
+// found no slot (no free one within kProbes: far past what a table 70% full
+// needs) adds no more keys and only notes them for the estimate that sizes the
+// next table.  Sized by the rows turned away, every one of them possibly a new
+// key, 64M rows of 65,536 values took tables of 2 GiB and 23.5 ms; by the
+// estimate 4 MiB and 21.2 ms.
 constexpr uint64_t kProbes = 512;
+constexpr int kHllBits = 10, kHllRegs = 1 << kHllBits;  // within 3% (one sigma)
 struct GlobalTable {
     unsigned long long* keys = nullptr;
     unsigned long long* counts = nullptr;
     uint64_t mask = 0;
     HistCtl* ctl = nullptr;
-    uint32_t fresh = 0;               // keys this thread brought in
-    unsigned long long dropped = 0;   // rows it found no slot for
+    uint32_t* hll = nullptr;  // kHllRegs registers: the keys turned away
+    uint32_t fresh = 0;       // keys this thread brought in
+    bool full = false;        // it found no slot for one
     __device__ __forceinline__ uint64_t home(uint64_t key) const { return hmix(key) & mask; }
     __device__ __forceinline__ unsigned long long peek(uint64_t s) const {
         return __hip_atomic_load(&keys[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    __device__ __forceinline__ void add(uint64_t key, unsigned long long cnt) {
-        if (dropped) {
-            dropped += cnt;
-            return;
-        }
-        uint64_t s = home(key);
-        for (uint64_t p = 0; p <= mask && p < kProbes; p++) {
-            unsigned long long seen = peek(s);
-            if (seen == kEmpty) {
-                const unsigned long long prev = atomicCAS(&keys[s], kEmpty, (unsigned long long)key);
-                if (prev == kEmpty) fresh++;
-                seen = prev == kEmpty ? key : prev;
+    // regs: the workgroup's registers (LDS)
+    __device__ __forceinline__ void add(uint64_t key, unsigned long long cnt, volatile uint32_t* regs) {
+        if (!full) {
+            uint64_t s = home(key);
+            for (uint64_t p = 0; p <= mask && p < kProbes; p++) {
+                unsigned long long seen = peek(s);
+                if (seen == kEmpty) {
+                    const unsigned long long prev = atomicCAS(&keys[s], kEmpty, (unsigned long long)key);
+                    if (prev == kEmpty) fresh++;
+                    seen = prev == kEmpty ? key : prev;
+                }
+                if (seen == key) {
+                    atomicAdd(&counts[s], cnt);
+                    return;
+                }
+                s = (s + 1) & mask;
             }
-            if (seen == key) {
-                atomicAdd(&counts[s], cnt);
-                return;
-            }
-            s = (s + 1) & mask;
+            full = true;
         }
-        dropped += cnt;
+        // the high bits: the keys that meet a full stretch share low ones
+        const uint64_t h = hmix(key);
+        const uint32_t r = (uint32_t)(h >> (64 - kHllBits));
+        const uint32_t rank = (uint32_t)__clzll((h << kHllBits) | (1ull << (kHllBits - 1))) + 1;
+        if (rank > regs[r]) atomicMax(const_cast<uint32_t*>(&regs[r]), rank);
     }
 };
+
+// How many keys the registers have seen.
+double hll_estimate(const uint32_t* regs) {
+    const double m = kHllRegs;
+    double sum = 0;
+    int zeros = 0;
+    for (int i = 0; i < kHllRegs; i++) {
+        sum += std::ldexp(1.0, -(int)regs[i]);
+        zeros += regs[i] == 0;
+    }
+    const double e = 0.7213 / (1.0 + 1.079 / m) * m * m / sum;
+    return e <= 2.5 * m && zeros ? m * std::log(m / zeros) : e;
+}
 
 // Ascending list of the (up to) four smallest keys seen, with multiplicity.
 struct Small4 {
@@ -401,6 +424,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
     __shared__ int s_nc[kHistThreads / kWave];
     __shared__ uint32_t s_new;   // keys this workgroup brought into the global table
     __shared__ uint32_t s_over;  // a key found no slot
+    __shared__ uint32_t s_hll[GLOBAL ? kHllRegs : 1];  // keys that the global table turned away
     __shared__ unsigned long long s_special, s_nans;
     __shared__ uint32_t s_negzero;
     constexpr bool kInt = !std::is_floating_point<T>::value;
@@ -414,6 +438,8 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
     if (kInt) fill(win, sizeof win, 0u);
     fill(skey, sizeof skey, ~0u);
     fill(scnt, sizeof scnt, 0u);
+    static_assert(!GLOBAL || kHllRegs == kHistThreads, "a register a thread");
+    if (GLOBAL) s_hll[threadIdx.x] = 0;
     if (threadIdx.x == 0) {
         s_new = s_over = s_negzero = 0;
         s_special = s_nans = 0;
@@ -445,7 +471,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
             }
         }
         if (GLOBAL)
-            table.add((uint64_t)key, add);
+            table.add((uint64_t)key, add, s_hll);
         else
             s_over = 1;
     };
@@ -546,17 +572,14 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
     const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
     if (GLOBAL) {
         for (int s = threadIdx.x; s < kLdsSlots; s += kHistThreads)
-            if (skey[s] != kFree) table.add((uint64_t)skey[s], scnt[s]);
+            if (skey[s] != kFree) table.add((uint64_t)skey[s], scnt[s], s_hll);
         const uint32_t fresh = wave_sum(table.fresh);
-        const unsigned long long dropped = wave_sum(table.dropped);
-        if (lane == 0) {
-            if (fresh) atomicAdd(&s_new, fresh);
-            if (dropped) {
-                atomicOr(&table.ctl->overflow, 1u);
-                atomicAdd(&table.ctl->dropped, dropped);
-            }
+        if (lane == 0 && fresh) atomicAdd(&s_new, fresh);
+        if (__syncthreads_or(table.full)) {
+            if (threadIdx.x == 0) atomicOr(&table.ctl->overflow, kTooSmall);
+            const uint32_t rank = s_hll[threadIdx.x];
+            if (rank > ld_agent(&table.hll[threadIdx.x])) atomicMax(&table.hll[threadIdx.x], rank);
         }
-        __syncthreads();
         if (threadIdx.x == 0 && s_new) atomicAdd(&table.ctl->distinct, (unsigned long long)s_new);
     } else {
         // partitions' used slots, where each begins, then the entries
@@ -949,7 +972,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_small(const T* __restrict
         for (uint32_t r = 0; r < nan_n; r++)  // every NaN row is a bin of count 1
             push<T>(b, K, Cand{1ull, ubits(from_order_key<T>(nan_keys[r]))});
         HistResult* out = reinterpret_cast<HistResult*>(host.dst);
-        out->ctl = HistCtl{s_distinct, s_special, s_nans, 0, s_over ? kTooSmall : 0u, s_negzero};
+        out->ctl = HistCtl{s_distinct, s_special, s_nans, s_over ? kTooSmall : 0u, s_negzero};
 #pragma unroll
         for (int i = 0; i < kMaxK; i++) out->top[i] = b[i];
     }
@@ -958,13 +981,15 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_small(const T* __restrict
 
 // The histogram's global table emptied (keys ~0, counts 0) and its control
 // block cleared, in one launch.
-__global__ void k_hist_init(unsigned long long* keys, unsigned long long* counts, size_t cap, HistCtl* ctl) {
+__global__ __launch_bounds__(kBlock) void k_hist_init(GlobalTable table) {
     const size_t stride = (size_t)gridDim.x * kBlock;
-    for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < cap; i += stride) {
-        keys[i] = kEmpty;
-        counts[i] = 0;
+    for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i <= table.mask; i += stride) {
+        table.keys[i] = kEmpty;
+        table.counts[i] = 0;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) *ctl = HistCtl{};
+    if (blockIdx.x != 0) return;
+    for (int i = threadIdx.x; i < kHllRegs; i += kBlock) table.hll[i] = 0;
+    if (threadIdx.x == 0) *table.ctl = HistCtl{};
 }
 
 uint64_t pow2_at_least(uint64_t v) {
@@ -1060,14 +1085,14 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
         const uint64_t all_distinct = pow2_at_least(2 * (uint64_t)n + 2);
         uint64_t cap = std::min<uint64_t>(std::max<uint64_t>(1024, all_distinct), 1u << 16);
         for (int attempt = 0; attempt < 3; attempt++) {
-            DevBuf keys(c, 8 * cap), counts(c, 8 * cap), ctl(c, sizeof(HistCtl));
+            DevBuf keys(c, 8 * cap), counts(c, 8 * cap), ctl(c, sizeof(HistCtl)), hll(c, 4 * kHllRegs);
             const GlobalTable table{keys.get<unsigned long long>(), counts.get<unsigned long long>(), cap - 1,
-                                    ctl.get<HistCtl>()};
+                                    ctl.get<HistCtl>(), hll.get<uint32_t>()};
+            kernel_bytes(c, "k_hist_init", 16.0 * (double)cap);
             const unsigned fg = (unsigned)std::min<uint64_t>((cap + kBlock - 1) / kBlock, (uint64_t)c->cu_count * 16);
             {
                 KernelTimer kt_(c, "k_hist_init");
-                hipLaunchKernelGGL(k_hist_init, dim3(fg), dim3(kBlock), 0, c->stream, table.keys, table.counts, cap,
-                                   table.ctl);
+                hipLaunchKernelGGL(k_hist_init, dim3(fg), dim3(kBlock), 0, c->stream, table);
             }
             {
                 KernelTimer kt_(c, "k_hist_count");
@@ -1090,7 +1115,12 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
             const HistCtl& h = found.ctl;
             if (h.overflow || h.distinct * 10 > cap * 7) {
                 if (attempt == 2 || cap >= all_distinct) fail(DDJ_ENOMEM, "histogram table overflow");
-                const uint64_t seen = h.distinct + (h.overflow ? h.dropped : 0);
+                uint64_t seen = h.distinct;
+                if (h.overflow) {
+                    uint32_t regs[kHllRegs];
+                    d2h(c, regs, hll.get(), sizeof regs);
+                    seen += (uint64_t)hll_estimate(regs);
+                }
                 const uint64_t next = attempt == 0 ? std::min(all_distinct, pow2_at_least(2 * seen + 2)) : all_distinct;
                 cap = std::max(next, std::min(all_distinct, 2 * cap));  // always grows
                 continue;

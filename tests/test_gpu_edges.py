@@ -171,6 +171,28 @@ def test_most_frequent_of_many_keys(ctx, dtype, n, distinct, tables):
     assert ("k_hist_init" not in ran) == tables
 
 
+@pytest.mark.parametrize("dtype,n,distinct", [(g.D_INT, 9_000_000, 100_000), (g.D_TIME, 4_200_000, 60_000),
+                                              (g.D_INT, 400_000, 400_000)])
+def test_most_frequent_table_is_sized_by_keys(ctx, dtype, n, distinct):
+    """The second global table has room for a few times the keys (the first holds
+    65,536 and turns the others away), however many rows they have."""
+    npdt = g.NP_DTYPE[dtype]
+    r = np.random.default_rng(n)
+    values = r.permutation(np.arange(distinct, dtype=np.int64) * 5_003 - 7).astype(npdt)
+    x = r.permutation(np.concatenate([values, values[r.integers(0, distinct, n - distinct)]]))
+    x[::1_113], x[7::2_211] = values[5], values[6]
+    buf, enc = ctx.upload(x), g.Encoding(ctx, g.DICT)
+    ctx.profile(True)
+    ctx.profile_reset()
+    meta = enc.Encode(buf, dtype)[1].to_bytes()
+    _, tables, nbytes = ctx.kernel_table()["k_hist_init"]
+    ctx.profile(False)
+    assert sorted(np.frombuffer(meta[16:16 + 4 * npdt().itemsize], npdt)) == sorted(_top(x, 4))
+    # 16 bytes a slot; at most twice the keys that the first held or turned away,
+    # estimated within 20% (six sigma), rounded up to a power of two
+    assert tables == 2 and 16 * 65_536 < nbytes <= 16 * (65_536 + 2 * 2 * 1.2 * (65_536 + distinct))
+
+
 # 4096-row tiles; up to 1024 of them are scanned by the counting pass's last
 # workgroup (its ticket groups begin past 64), more by a launch of their own
 @pytest.mark.parametrize("tiles", [1, 2, 64, 65, 1_023, 1_024, 1_025])
