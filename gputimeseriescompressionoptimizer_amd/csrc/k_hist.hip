@@ -20,7 +20,8 @@
 // four smallest (radix order) NaN rows, which is all the top-K can ever take
 // from them.  Columns of a few thousand rows are counted whole in one
 // workgroup's LDS (k_hist_small).  The global table starts at 2n slots (at
-// least 1024, at most 64K); if it ends up more than 70% full the host retries
+// least 1024, at most 64K, or what k_hist_merge's tables found too many keys
+// for); if it ends up more than 70% full the host retries
 // once with a table of twice the keys seen (the exact count, and with a full
 // table the HyperLogLog estimate of the keys that it turned away), and a second
 // retry, never needed in practice, sizes it for every row distinct.
@@ -77,6 +78,19 @@ template <typename T> __device__ __forceinline__ uint64_t hist_key(T v, bool& ne
 // estimate 4 MiB and 21.2 ms.
 constexpr uint64_t kProbes = 512;
 constexpr int kHllBits = 10, kHllRegs = 1 << kHllBits;  // within 3% (one sigma)
+// Notes a key in a workgroup's registers (LDS).  By the high bits of its hash:
+// the keys that meet a full stretch of a table share low ones.
+__device__ __forceinline__ void hll_note(uint64_t key, volatile uint32_t* regs) {
+    const uint64_t h = hmix(key);
+    const uint32_t r = (uint32_t)(h >> (64 - kHllBits));
+    const uint32_t rank = (uint32_t)__clzll((h << kHllBits) | (1ull << (kHllBits - 1))) + 1;
+    if (rank > regs[r]) atomicMax(const_cast<uint32_t*>(&regs[r]), rank);
+}
+// A workgroup's register into the column's.
+__device__ __forceinline__ void hll_merge(uint32_t* hll, int r, uint32_t rank) {
+    if (rank > __hip_atomic_load(&hll[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&hll[r], rank);
+}
+
 struct GlobalTable {
     unsigned long long* keys = nullptr;
     unsigned long long* counts = nullptr;
@@ -108,11 +122,7 @@ struct GlobalTable {
             }
             full = true;
         }
-        // the high bits: the keys that meet a full stretch share low ones
-        const uint64_t h = hmix(key);
-        const uint32_t r = (uint32_t)(h >> (64 - kHllBits));
-        const uint32_t rank = (uint32_t)__clzll((h << kHllBits) | (1ull << (kHllBits - 1))) + 1;
-        if (rank > regs[r]) atomicMax(const_cast<uint32_t*>(&regs[r]), rank);
+        hll_note(key, regs);
     }
 };
 
@@ -234,7 +244,7 @@ struct HistInfo {
 // 251, now 85 and 81 (in the global table alone 184 and 185); of 1M rows with
 // 60,000 keys 1187 and 1247, now 126 and 106; of 100,000 rows with 50 keys 55 and
 // 56, now 52.
-constexpr int kHistThreads = 1024;
+constexpr int kHistThreads = 1024, kMergeThreads = 1024, kMergeSlots = 4096;
 template <typename T> constexpr int few_rows() { return sizeof(T) == 8 ? 4 : sizeof(T) == 1 ? 16 : 8; }
 // Entries a workgroup may write out.
 template <typename T, int PER> constexpr int seg_slots() {
@@ -400,11 +410,13 @@ __device__ __forceinline__ uint32_t segment_of(const uint32_t* first, uint32_t s
 // go to segs (its seg_slots entries from blockIdx.x on, partition
 // by partition, partition p from off[p * grid + workgroup] on), and a key
 // without a slot ends the count (info[].overflow: the host counts again with
-// GLOBAL).  With a tail, if all workgroups' entries are few (columns of few
-// distinct values), the last workgroup adds them up itself and hands the best K
-// to the host; else (kNeedMerge) k_hist_merge does (1M int32 rows of 130 values,
-// 16,000 entries: 37 us, in two launches 42).
-constexpr uint32_t kTailEntries = 16384;
+// GLOBAL).  With a tail, if all workgroups' entries are no more than its table's
+// slots (columns of few distinct values), the last workgroup adds them up itself
+// and hands the best K to the host; else (kNeedMerge), or if too many of them turn
+// out distinct, k_hist_merge does.  1M int32 rows of 60 values, 7,400 entries: 30
+// us in one launch, 42 in two; the other way round from about 20,000 entries on.
+// 13,000 distinct rows, all of them entries: 47 us in two launches, and after a
+// tail that took 256 probes to find its table full 401.
 struct HistTail {
     uint32_t* tickets = nullptr;
     int K = 0;
@@ -414,7 +426,7 @@ template <typename T, int PER, bool GLOBAL>
 __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict__ x, size_t n, GlobalTable table,
                                                              HistEntry<HistKey<T>>* __restrict__ segs,
                                                              uint32_t* __restrict__ off, HistInfo* __restrict__ info,
-                                                             HistTail tail) {
+                                                             uint32_t* __restrict__ hll, HistTail tail) {
     using KT = HistKey<T>;
     constexpr KT kFree = (KT)~(KT)0;  // an empty slot; rows of that bit pattern are counted on the side
     constexpr int PS = part_slots<T>(), kLdsSlots = kHistParts * PS;
@@ -438,8 +450,11 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
     if (kInt) fill(win, sizeof win, 0u);
     fill(skey, sizeof skey, ~0u);
     fill(scnt, sizeof scnt, 0u);
-    static_assert(!GLOBAL || kHllRegs == kHistThreads, "a register a thread");
-    if (GLOBAL) s_hll[threadIdx.x] = 0;
+    static_assert(kHllRegs == kHistThreads && kHllRegs == kMergeThreads, "a register a thread");
+    if (GLOBAL)
+        s_hll[threadIdx.x] = 0;
+    else if (blockIdx.x == 0)
+        hll[threadIdx.x] = 0;  // k_hist_merge's
     if (threadIdx.x == 0) {
         s_new = s_over = s_negzero = 0;
         s_special = s_nans = 0;
@@ -577,8 +592,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
         if (lane == 0 && fresh) atomicAdd(&s_new, fresh);
         if (__syncthreads_or(table.full)) {
             if (threadIdx.x == 0) atomicOr(&table.ctl->overflow, kTooSmall);
-            const uint32_t rank = s_hll[threadIdx.x];
-            if (rank > ld_agent(&table.hll[threadIdx.x])) atomicMax(&table.hll[threadIdx.x], rank);
+            hll_merge(table.hll, threadIdx.x, s_hll[threadIdx.x]);
         }
         if (threadIdx.x == 0 && s_new) atomicAdd(&table.ctl->distinct, (unsigned long long)s_new);
     } else {
@@ -663,7 +677,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
         __syncthreads();
         fold_info<kHistThreads>(info, blocks, &ctl);
         HistResult* out = reinterpret_cast<HistResult*>(tail.host.dst);
-        const bool few = total <= kTailEntries && n < (1ull << 32);
+        const bool few = total <= (uint32_t)kLdsSlots && n < (1ull << 32);
         constexpr int F = 4;  // entries in flight a thread
         for (uint32_t e0 = threadIdx.x; few && e0 < total; e0 += F * kHistThreads) {
             KT key[F];
@@ -682,8 +696,9 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
 #pragma unroll
             for (int f = 0; f < F; f++) {
                 if (!cnt[f]) continue;
-                uint32_t s = (uint32_t)(((uint64_t)lds_hash<false>((uint64_t)key[f]) * kLdsSlots) >> 32);
-                int left = 256;
+                const uint32_t h = lds_hash<false>((uint64_t)key[f]), step = 6 * (h & 255) + 1;  // as k_hist_small's
+                uint32_t s = (uint32_t)(((uint64_t)h * kLdsSlots) >> 32);
+                int left = 32;
                 for (; left > 0; left--) {
                     KT k = skey[s];
                     if (k == kFree) k = atomicCAS(&skey[s], kFree, key[f]);
@@ -691,10 +706,11 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
                         atomicAdd(&scnt[s], cnt[f]);
                         break;
                     }
-                    s = s + 1 < (uint32_t)kLdsSlots ? s + 1 : 0;
+                    s = s + step < (uint32_t)kLdsSlots ? s + step : s + step - kLdsSlots;
                 }
                 if (left == 0) atomicOr(&ctl.overflow, kNeedMerge);
             }
+            if (*(volatile uint32_t*)&ctl.overflow) break;  // (each wave by itself: the sums are dropped)
         }
         if (!few && threadIdx.x == 0) atomicOr(&ctl.overflow, kNeedMerge);
         __syncthreads();
@@ -743,14 +759,13 @@ __device__ __forceinline__ bool best_of_grid(Cand* top, int K, Cand* sc, Cand* b
 // atomics, the launch that cleared it and the one that searched its 64K slots:
 // 5M rows of long-tailed volumes 2 + 72 + 11 us, now 20 + 22; 16M rows, whose
 // table overflowed and was counted again, 2.5 ms, now 38 + 32 us.
-constexpr int kMergeThreads = 1024, kMergeSlots = 4096;
 template <typename T>
 __global__ __launch_bounds__(kMergeThreads) void k_hist_merge(const HistEntry<HistKey<T>>* __restrict__ segs,
                                                               const uint32_t* __restrict__ off,
                                                               const HistInfo* __restrict__ info, uint32_t blocks,
                                                               uint32_t slots /* entries a workgroup */, int K,
-                                                              Cand* partials, uint32_t* part_ctl, uint32_t* tickets,
-                                                              HostOut host) {
+                                                              Cand* partials, uint32_t* part_ctl, uint32_t* hll,
+                                                              uint32_t* tickets, HostOut host) {
     using KT = HistKey<T>;
     constexpr KT kFree = (KT)~(KT)0;
     constexpr int W = kMergeThreads / kWave;
@@ -760,6 +775,7 @@ __global__ __launch_bounds__(kMergeThreads) void k_hist_merge(const HistEntry<Hi
     __shared__ Cand best[kMaxK];
     __shared__ HistCtl ctl;
     __shared__ uint32_t s_distinct, s_over;
+    __shared__ uint32_t s_hll[kHllRegs];  // keys turned away
     __shared__ uint32_t first[kMergeThreads];  // of the partition's entries, where each workgroup's begin
     __shared__ uint32_t begin[kMergeThreads];  // and where they are among the workgroup's
     __shared__ uint32_t red[W];
@@ -783,6 +799,7 @@ __global__ __launch_bounds__(kMergeThreads) void k_hist_merge(const HistEntry<Hi
         skey[i] = kFree;
         scnt[i] = 0;
     }
+    s_hll[threadIdx.x] = 0;
     if (threadIdx.x == 0) {
         s_distinct = s_over = 0;
         ctl = HistCtl{};
@@ -807,8 +824,12 @@ __global__ __launch_bounds__(kMergeThreads) void k_hist_merge(const HistEntry<Hi
 #pragma unroll
         for (int f = 0; f < F; f++) {
             if (!en[f].count) continue;
-            uint32_t s = (uint32_t)hmix((uint64_t)en[f].key) & (kMergeSlots - 1);
-            int left = 256;  // past 90% full the count runs again with the global table
+            const uint64_t h = hmix((uint64_t)en[f].key);
+            const uint32_t step = (uint32_t)(h >> 32) | 1;  // odd: visits every slot
+            uint32_t s = (uint32_t)h & (kMergeSlots - 1);
+            // past 85% full the count runs again with the global table, and the
+            // keys left over only go into the estimate that sizes it
+            int left = *(volatile uint32_t*)&s_over ? 0 : 64;
             for (; left > 0; left--) {
                 KT have = skey[s];
                 if (have == kFree) have = atomicCAS(&skey[s], kFree, en[f].key);
@@ -816,13 +837,16 @@ __global__ __launch_bounds__(kMergeThreads) void k_hist_merge(const HistEntry<Hi
                     atomicAdd(&scnt[s], (unsigned long long)en[f].count);
                     break;
                 }
-                s = (s + 1) & (kMergeSlots - 1);
+                s = (s + step) & (kMergeSlots - 1);
             }
-            if (left == 0) s_over = 1;
+            if (left == 0) {
+                s_over = 1;
+                hll_note((uint64_t)en[f].key, s_hll);
+            }
         }
-        if (*(volatile uint32_t*)&s_over) break;  // the count is dropped
     }
     __syncthreads();
+    if (s_over) hll_merge(hll, threadIdx.x, s_hll[threadIdx.x]);
     Cand top[kMaxK];
     take_table<T, kMergeSlots, kMergeThreads>(skey, scnt, top, K, &s_distinct);
     block_best<T, kMergeThreads>(top, K, sc, best);  // its barriers complete s_distinct
@@ -1032,6 +1056,13 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
         }
         using Entry = HistEntry<HistKey<T>>;
         auto xs = static_cast<const T*>(x);
+        // The keys that a full table (or k_hist_merge's) holds and has turned away.
+        auto keys_seen = [&](const HistCtl& ctl, const DevBuf& hll) {
+            uint32_t regs[kHllRegs];
+            d2h(c, regs, hll.get(), sizeof regs);
+            return ctl.distinct + (uint64_t)hll_estimate(regs);
+        };
+        uint64_t seen = 0;
         // One count in tiles of PER rows a thread by at most max_g workgroups, and
         // the merge: whether the tables held the keys.
         auto counted = [&](auto per, size_t max_g) {
@@ -1040,7 +1071,7 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
             // in four sizes, so that columns of every length share their blocks
             size_t room = 16;
             while (room < g) room *= 4;
-            DevBuf info(c, sizeof(HistInfo) * g), off(c, 4 * (kHistParts + 1) * g),
+            DevBuf info(c, sizeof(HistInfo) * g), off(c, 4 * (kHistParts + 1) * g), hll(c, 4 * kHllRegs),
                 segs(c, sizeof(Entry) * seg_slots<T, PER>() * room);
             // up to 1M rows of 4 bytes the last workgroup merges (50 codes: one launch
             // of 22 us for two of 9 + 16); more workgroups have too many entries for
@@ -1050,7 +1081,8 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
             {
                 KernelTimer kt_(c, "k_hist_count");
                 hipLaunchKernelGGL((k_hist_count<T, PER, false>), dim3((unsigned)g), dim3(kHistThreads), 0, c->stream, xs,
-                                   n, GlobalTable{}, segs.get<Entry>(), off.get<uint32_t>(), info.get<HistInfo>(), tail);
+                                   n, GlobalTable{}, segs.get<Entry>(), off.get<uint32_t>(), info.get<HistInfo>(),
+                                   hll.get<uint32_t>(), tail);
             }
             HIPC(hipGetLastError());
             if (tail.tickets) memcpy(&found, wait_host_out(c, tail.host), sizeof found);
@@ -1062,11 +1094,12 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
                     hipLaunchKernelGGL(k_hist_merge<T>, dim3(kHistParts), dim3(kMergeThreads), 0, c->stream,
                                        segs.get<Entry>(), off.get<uint32_t>(), info.get<HistInfo>(), (uint32_t)g,
                                        (uint32_t)seg_slots<T, PER>(), K, partials.get<Cand>(), part_ctl.get<uint32_t>(),
-                                       c->control->tickets, ho);
+                                       hll.get<uint32_t>(), c->control->tickets, ho);
                 }
                 HIPC(hipGetLastError());
                 memcpy(&found, wait_host_out(c, ho), sizeof found);
             }
+            if (found.ctl.overflow && found.ctl.distinct) seen = keys_seen(found.ctl, hll);  // the merge's tables filled
             return !found.ctl.overflow;
         };
         using Few = std::integral_constant<int, few_rows<T>()>;
@@ -1083,7 +1116,8 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
         DevBuf info(c, sizeof(HistInfo) * g);
         // more distinct keys than the LDS tables hold
         const uint64_t all_distinct = pow2_at_least(2 * (uint64_t)n + 2);
-        uint64_t cap = std::min<uint64_t>(std::max<uint64_t>(1024, all_distinct), 1u << 16);
+        uint64_t cap = std::min<uint64_t>(std::max<uint64_t>(1024, all_distinct),
+                                          std::max<uint64_t>(1u << 16, pow2_at_least(2 * seen + 2)));
         for (int attempt = 0; attempt < 3; attempt++) {
             DevBuf keys(c, 8 * cap), counts(c, 8 * cap), ctl(c, sizeof(HistCtl)), hll(c, 4 * kHllRegs);
             const GlobalTable table{keys.get<unsigned long long>(), counts.get<unsigned long long>(), cap - 1,
@@ -1097,7 +1131,7 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
             {
                 KernelTimer kt_(c, "k_hist_count");
                 hipLaunchKernelGGL((k_hist_count<T, 16, true>), dim3((unsigned)g), dim3(kHistThreads), 0, c->stream, xs, n,
-                                   table, nullptr, nullptr, info.get<HistInfo>(), HistTail{});
+                                   table, nullptr, nullptr, info.get<HistInfo>(), nullptr, HistTail{});
             }
             HIPC(hipGetLastError());
             // the top-K runs before the table's state is known, so that one
@@ -1115,12 +1149,7 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
             const HistCtl& h = found.ctl;
             if (h.overflow || h.distinct * 10 > cap * 7) {
                 if (attempt == 2 || cap >= all_distinct) fail(DDJ_ENOMEM, "histogram table overflow");
-                uint64_t seen = h.distinct;
-                if (h.overflow) {
-                    uint32_t regs[kHllRegs];
-                    d2h(c, regs, hll.get(), sizeof regs);
-                    seen += (uint64_t)hll_estimate(regs);
-                }
+                seen = h.overflow ? keys_seen(h, hll) : h.distinct;
                 const uint64_t next = attempt == 0 ? std::min(all_distinct, pow2_at_least(2 * seen + 2)) : all_distinct;
                 cap = std::max(next, std::min(all_distinct, 2 * cap));  // always grows
                 continue;

@@ -171,11 +171,14 @@ def test_most_frequent_of_many_keys(ctx, dtype, n, distinct, tables):
     assert ("k_hist_init" not in ran) == tables
 
 
-@pytest.mark.parametrize("dtype,n,distinct", [(g.D_INT, 9_000_000, 100_000), (g.D_TIME, 4_200_000, 60_000),
-                                              (g.D_INT, 400_000, 400_000)])
-def test_most_frequent_table_is_sized_by_keys(ctx, dtype, n, distinct):
-    """The second global table has room for a few times the keys (the first holds
-    65,536 and turns the others away), however many rows they have."""
+# past 8M rows (4M of 8 bytes) a first global table of 65,536 slots turns keys
+# away, before that the merge's do; the next table holds the column
+@pytest.mark.parametrize("dtype,n,distinct,tables", [
+    (g.D_INT, 9_000_000, 100_000, 2), (g.D_TIME, 4_200_000, 60_000, 2), (g.D_INT, 400_000, 400_000, 1),
+    (g.D_TIME, 2_000_000, 700_000, 1), (g.D_INT, 9_000_000, 40_000, 1), (g.D_INT, 9_000_000, 46_000, 2)])
+def test_most_frequent_table_is_sized_by_keys(ctx, dtype, n, distinct, tables):
+    """A larger global table has room for a few times the keys, however many
+    rows they have."""
     npdt = g.NP_DTYPE[dtype]
     r = np.random.default_rng(n)
     values = r.permutation(np.arange(distinct, dtype=np.int64) * 5_003 - 7).astype(npdt)
@@ -185,12 +188,13 @@ def test_most_frequent_table_is_sized_by_keys(ctx, dtype, n, distinct):
     ctx.profile(True)
     ctx.profile_reset()
     meta = enc.Encode(buf, dtype)[1].to_bytes()
-    _, tables, nbytes = ctx.kernel_table()["k_hist_init"]
+    _, launches, nbytes = ctx.kernel_table()["k_hist_init"]
     ctx.profile(False)
     assert sorted(np.frombuffer(meta[16:16 + 4 * npdt().itemsize], npdt)) == sorted(_top(x, 4))
-    # 16 bytes a slot; at most twice the keys that the first held or turned away,
-    # estimated within 20% (six sigma), rounded up to a power of two
-    assert tables == 2 and 16 * 65_536 < nbytes <= 16 * (65_536 + 2 * 2 * 1.2 * (65_536 + distinct))
+    # 16 bytes a slot; twice the keys that the tables before it held and turned
+    # away (none of them more than once each), estimated within 20% (six sigma),
+    # rounded up to a power of two
+    assert launches == tables and nbytes <= 16 * (65_536 + 2 * 2 * 1.2 * 2 * distinct)
 
 
 # 4096-row tiles; up to 1024 of them are scanned by the counting pass's last
