@@ -194,7 +194,9 @@ __device__ __forceinline__ int stage_fl_words(const uint8_t* __restrict__ in, si
     const uint8_t* base = in + B0;
     const int a = (int)(reinterpret_cast<uintptr_t>(base) & 15);
     const u32x4* wp4 = reinterpret_cast<const u32x4*>(base - a);
-    const int n4_valid = (a + avail + 15) / 16;
+    // past the stream's end (rows that a corrupt stencil asks for) no chunk holds
+    // a byte of it, and none may be read
+    const int n4_valid = avail > 0 ? (a + avail + 15) / 16 : 0;
     const int n4_fill = n4_valid + 1;  // <= fl_stage_words<MAXB>() / 4 for b <= MAXB
     u32x4* w4 = reinterpret_cast<u32x4*>(w);
     constexpr int U = 4;

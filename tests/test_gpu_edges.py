@@ -235,6 +235,26 @@ def test_merge_outputs_too_short(ctx, n):
     assert np.array_equal(enc.Decode([stencil, codes, rest], g.D_INT).to_numpy(np.int32), x)
 
 
+# scanned with the count (up to 4096 tiles of 4096 rows), and by a launch of its own
+@pytest.mark.parametrize("n", [5_000, 1_000_001, 4_096 * 4_096 + 1])
+@pytest.mark.parametrize("flip", [0xFF, 0x55])
+def test_patch_streams_too_short(ctx, n, flip):
+    """The same for a patch whose two sides are FL streams: most tiles ask for
+    rows far past the end of one, which are not read."""
+    r = np.random.default_rng(n)
+    x = np.where(r.random(n) < 0.01, r.integers(20_000, 30_000, n), 500 + np.arange(n) % 90).astype(np.int16)
+    path = [g.PATCH, g.AFL, g.NONE, g.AFL, g.NONE]
+    tree = g.CompressionTree(ctx, path, g.D_SHORT)
+    blob = np.frombuffer(tree.Compress(ctx.upload(x)).to_bytes(), np.uint8)
+    stencil = slice(8 + 1, 8 + int(blob[4:8].view(np.int32)[0]))  # after the node's header and the padding's count
+    bad = blob.copy()
+    bad[stencil] ^= flip
+    with pytest.raises(g.DdjError) as e:
+        tree.Decompress(ctx.upload(bad))
+    assert e.value.status == 3
+    assert np.array_equal(tree.Decompress(ctx.upload(blob)).to_numpy(np.int16), x)
+
+
 @pytest.mark.parametrize("begin,count", [(0, 1), (0, 4097), (1, 1), (4095, 2), (4096, 4096), (4097, 1), (99_999, 1),
                                          (70_001, 29_999), (0, 100_000)])
 def test_delta_row_ranges(ctx, begin, count):
