@@ -927,6 +927,7 @@ void batch_run(ddj_ctx* ctx, const ddj_column* cols, uint32_t n_cols, const ddj_
         std::unique_ptr<OwnedCtx> w(new OwnedCtx);
         const hipError_t e = init_ctx(w->c, ctx->c.device);
         if (e != hipSuccess) fail(e == hipErrorOutOfMemory ? DDJ_ENOMEM : DDJ_EHIP, hipGetErrorString(e));
+        w->c.alloc->share(*ctx->c.alloc);
         ctx->pool.push_back(std::move(w));
     }
     for (uint32_t i = 0; i < n_cols; i++) blobs[i] = ddj_buf{nullptr, 0};

@@ -48,12 +48,22 @@ public:
     // (its stream work on the block must be complete).
     void adopt(void* p, size_t cls);
     void trim();
+    // From now on either of the two, and whoever shares with them, has the
+    // others give their cached blocks back before an allocation fails.  Before
+    // this one is used; the other may be in use.
+    void share(Allocator& other);
     size_t in_use() const { return in_use_; }
 
 private:
+    struct Group {
+        std::mutex mu;
+        std::vector<Allocator*> members;
+    };
     static size_t round_size(size_t bytes);
+    void* take_locked(size_t size_class);  // null: no memory
     void trim_locked();
     std::mutex mu_;
+    std::shared_ptr<Group> group_;
     int device_;
     std::map<size_t, std::vector<void*>> free_;
     std::map<void*, size_t> live_;

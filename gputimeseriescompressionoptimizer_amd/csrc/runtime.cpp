@@ -1,4 +1,4 @@
-// Context, stream, caching allocator and copies.
+// Errors, read-backs and copies.
 #include "ddj_internal.h"
 #include "kernels.h"
 
@@ -30,90 +30,6 @@ size_t dtype_size(int dtype) {
     case DDJ_D_CHAR: return 1;
     default: return 0;
     }
-}
-
-// Size classes: powers of two up to 1 MiB, then multiples of 2 MiB.  Every
-// block also has 64 spare bytes so kernels may touch whole 16-byte vectors
-// past a logical end.
-size_t Allocator::round_size(size_t bytes) {
-    bytes += 64;
-    if (bytes <= (1u << 20)) {
-        size_t s = 256;
-        while (s < bytes) s <<= 1;
-        return s;
-    }
-    const size_t g = 2u << 20;
-    return (bytes + g - 1) / g * g;
-}
-
-void* Allocator::alloc(size_t bytes) {
-    std::lock_guard<std::mutex> lk(mu_);
-    size_t s = round_size(bytes);
-    auto it = free_.find(s);
-    if (it != free_.end() && !it->second.empty()) {
-        void* p = it->second.back();
-        it->second.pop_back();
-        live_[p] = s;
-        in_use_ += s;
-        return p;
-    }
-    void* p = nullptr;
-    hipError_t e = hipMalloc(&p, s);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        trim_locked();  // give cached blocks back and retry once
-        e = hipMalloc(&p, s);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            fail(DDJ_ENOMEM, "device allocation of " + std::to_string(s) + " bytes failed");
-        }
-    }
-    live_[p] = s;
-    in_use_ += s;
-    return p;
-}
-
-void Allocator::free(void* p) {
-    if (!p) return;
-    std::lock_guard<std::mutex> lk(mu_);
-    auto it = live_.find(p);
-    if (it == live_.end()) return;
-    free_[it->second].push_back(p);
-    in_use_ -= it->second;
-    live_.erase(it);
-}
-
-bool Allocator::detach(void* p, size_t* cls) {
-    std::lock_guard<std::mutex> lk(mu_);
-    auto it = live_.find(p);
-    if (it == live_.end()) return false;
-    if (cls) *cls = it->second;
-    in_use_ -= it->second;
-    live_.erase(it);
-    return true;
-}
-
-void Allocator::adopt(void* p, size_t cls) {
-    std::lock_guard<std::mutex> lk(mu_);
-    live_[p] = cls;
-    in_use_ += cls;
-}
-
-void Allocator::trim() {
-    std::lock_guard<std::mutex> lk(mu_);
-    trim_locked();
-}
-
-void Allocator::trim_locked() {
-    (void)hipDeviceSynchronize();
-    for (auto& kv : free_)
-        for (void* p : kv.second) (void)hipFree(p);
-    free_.clear();
-}
-
-Allocator::~Allocator() {
-    trim_locked();
-    for (auto& kv : live_) (void)hipFree(kv.first);
 }
 
 void d2h_any(Ctx* c, void* dst, const void* src, size_t bytes) {
