@@ -69,8 +69,8 @@ def _top(x, k):
     return [int(v[i]) for i in np.lexsort((v, -c))[:k]]
 
 
-# 16384 rows a workgroup, 12288 LDS slots (6144 of 8 bytes), 64K slots in the
-# first global table (70% of it full makes the count run again)
+# 8192 rows a workgroup (4096 of 8 bytes), 64 tables of 4096 slots in the merge;
+# 300,000 keys need the global one
 @pytest.mark.parametrize("distinct", [1, 3, 4, 63, 2_049, 6_144, 12_289, 45_875, 45_876, 70_000, 300_000])
 @pytest.mark.parametrize("dtype", [g.D_INT, g.D_TIME])
 def test_most_frequent(ctx, dtype, distinct):
@@ -197,9 +197,10 @@ def test_most_frequent_table_is_sized_by_keys(ctx, dtype, n, distinct, tables):
     assert launches == tables and nbytes <= 16 * (65_536 + 2 * 2 * 1.2 * 2 * distinct)
 
 
-# 4096-row tiles; up to 1024 of them are scanned by the counting pass's last
-# workgroup (its ticket groups begin past 64), more by a launch of their own
-@pytest.mark.parametrize("tiles", [1, 2, 64, 65, 1_023, 1_024, 1_025])
+# 4096-row tiles; up to 4096 of them are scanned by the counting pass's last
+# workgroup (its ticket groups begin past 64, its steps take 1024), more by a
+# launch of their own
+@pytest.mark.parametrize("tiles", [1, 2, 64, 65, 1_023, 1_024, 1_025, 4_096])
 @pytest.mark.parametrize("path,dtype", [
     ([g.PATCH, g.AFL, g.NONE, g.AFL, g.NONE], g.D_SHORT),
     ([g.PATCH, g.NONE, g.NONE], g.D_SHORT),
@@ -212,7 +213,7 @@ def test_most_frequent_table_is_sized_by_keys(ctx, dtype, n, distinct, tables):
 def test_tile_scan(ctx, path, dtype, tiles):
     npdt = g.NP_DTYPE[dtype]
     r = np.random.default_rng(tiles)
-    for n in (4096 * tiles - 1, 4096 * tiles, 4096 * tiles + 1):
+    for n in (4096 * tiles - 1, 4096 * tiles, 4096 * tiles + 1):  # one tile more with the last
         x = (r.integers(0, 100, n) + (r.random(n) < 0.02) * r.integers(0, 27, n)).astype(npdt)
         x[n // 5: n // 4] = 3
         tree = g.CompressionTree(ctx, path, dtype)
@@ -221,21 +222,24 @@ def test_tile_scan(ctx, path, dtype, tiles):
         assert np.array_equal(tree.Decompress(blob).to_numpy(npdt), x)
 
 
-@pytest.mark.parametrize("n", [5_000, 5_000_000])  # scanned with the count, and by a launch of its own
-def test_merge_outputs_too_short(ctx, n):
+# scanned with the count (up to 4096 tiles of 4096 rows), whose result says so,
+# and by a launch of its own, after which the merge's error flag does
+@pytest.mark.parametrize("n,dtype", [(5_000, g.D_INT), (5_000_000, g.D_INT), (4_096 * 4_096, g.D_SHORT),
+                                     (4_096 * 4_096 + 1, g.D_SHORT)])
+def test_merge_outputs_too_short(ctx, n, dtype):
     """A stencil with more set or clear bits than the outputs hold is refused."""
-    x = (np.arange(n) % 5).astype(np.int32)
+    npdt = g.NP_DTYPE[dtype]
+    x = (np.arange(n) % 5).astype(npdt)
     enc = g.Encoding(ctx, g.DICT)
-    stencil, codes, rest = enc.Encode(ctx.upload(x), g.D_INT)
+    stencil, codes, rest = enc.Encode(ctx.upload(x), dtype)
     flipped = ctx.upload(np.bitwise_xor(np.frombuffer(stencil.to_bytes(), np.uint8),
                                         np.r_[np.zeros(1, np.uint8), np.full(stencil.nbytes - 1, 255, np.uint8)]))
     with pytest.raises(g.DdjError) as e:
-        enc.Decode([flipped, codes, rest], g.D_INT)
+        enc.Decode([flipped, codes, rest], dtype)
     assert e.value.status == 3
-    assert np.array_equal(enc.Decode([stencil, codes, rest], g.D_INT).to_numpy(np.int32), x)
+    assert np.array_equal(enc.Decode([stencil, codes, rest], dtype).to_numpy(npdt), x)
 
 
-# scanned with the count (up to 4096 tiles of 4096 rows), and by a launch of its own
 @pytest.mark.parametrize("n", [5_000, 1_000_001, 4_096 * 4_096 + 1])
 @pytest.mark.parametrize("flip", [0xFF, 0x55])
 def test_patch_streams_too_short(ctx, n, flip):
