@@ -162,11 +162,6 @@ template <typename T> __device__ __forceinline__ T wave_sum(T v) {
         return v;
     }
 }
-__device__ __forceinline__ uint64_t wave_or(uint64_t v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v |= __shfl_xor(v, o, kWave);
-    return v;
-}
 
 // Block-wide exclusive scan of one value per thread (NT threads).
 // Returns the exclusive prefix; *total receives the block sum.

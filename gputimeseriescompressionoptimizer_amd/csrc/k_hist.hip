@@ -350,7 +350,8 @@ template <typename T, int NT = kBlock> __device__ void block_best(Cand* top, int
 // workgroup) and the counting workgroups' records: rows of the empty markers'
 // bit pattern (all ones), and every NaN row as a bin of count 1.
 template <typename T>
-__device__ void finish_topk(const Cand* best, int K, HistCtl ctl, const HistInfo* info, uint32_t blocks, HistResult* out) {
+__device__ void finish_topk(const Cand* best, int K, HistCtl ctl, const HistInfo* info, uint32_t blocks,
+                            HistResult* out) {
     Cand b[kMaxK];
 #pragma unroll
     for (int i = 0; i < kMaxK; i++) b[i] = i < K ? best[i] : Cand{0, 0};

@@ -77,7 +77,6 @@ template <typename K> K* radix_sort(Ctx* c, K* keys, K* tmp, size_t n, int key_b
 // device-side check) arm it first; the call then reads and clears it.
 void arm_error_flag(Ctx* c);
 
-
 // The floatToInt encoder's inputs for a float / double column: min/max keys
 // and the float precision (maximum over the rows, as DevStats::precision).
 struct FloatScanResult {
@@ -189,7 +188,6 @@ void launch_sub_scalar(Ctx* c, int elem_size, const void* x, size_t n, uint64_t 
 void launch_float_split(Ctx* c, const float* x, size_t n, int32_t* mant, int32_t* expo, int32_t* sign);
 void launch_float_compose(Ctx* c, const int32_t* mant, const int32_t* expo, const uint8_t* stencil_bits,
                           int sign_const, size_t n, float* out);
-void launch_precision(Ctx* c, int dtype, const void* x, size_t n, uint32_t* d_max);
 void launch_float_to_int(Ctx* c, int dtype, const void* x, size_t n, int precision, int32_t* out);
 void launch_int_to_float(Ctx* c, int dtype, const uint8_t* x, size_t n, int precision, void* out);
 
