@@ -411,13 +411,14 @@ __device__ __forceinline__ uint32_t segment_of(const uint32_t* first, uint32_t s
 // go to segs (its seg_slots entries from blockIdx.x on, partition
 // by partition, partition p from off[p * grid + workgroup] on), and a key
 // without a slot ends the count (info[].overflow: the host counts again with
-// GLOBAL).  With a tail, if all workgroups' entries are no more than its table's
-// slots (columns of few distinct values), the last workgroup adds them up itself
-// and hands the best K to the host; else (kNeedMerge), or if too many of them turn
-// out distinct, k_hist_merge does.  1M int32 rows of 60 values, 7,400 entries: 30
-// us in one launch, 42 in two; the other way round from about 20,000 entries on.
-// 13,000 distinct rows, all of them entries: 47 us in two launches, and after a
-// tail that took 256 probes to find its table full 401.
+// GLOBAL).  With a tail, the last workgroup adds all workgroups' entries up itself
+// and hands the best K to the host, if its table has a slot for each or, up to
+// kTailEntries, no workgroup has more than kTailKeys (columns of few distinct
+// values); else (kNeedMerge), or if too many turn out distinct, k_hist_merge does.
+// 300,000 int64 rows of 130 values, 9,600 entries: 62 us encoded, through the merge
+// 71.  13,000 distinct rows, all of them entries: 47 us counted in two launches, and
+// after a tail that took 256 probes to find its table full 401.
+constexpr uint32_t kTailEntries = 16384, kTailKeys = 512;
 struct HistTail {
     uint32_t* tickets = nullptr;
     int K = 0;
@@ -465,11 +466,11 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
     unsigned long long special = 0, nans = 0;
     bool negzero = false;
     // Probes for a slot: with few rows, whose keys all have one, the whole
-    // partition; 48 let 7,500 random keys of 4 bytes and 5,000 of 8 find one (24:
-    // 5,500 and 3,500; 96: 500 more, but a table that overflows all the same does
-    // so after twice the time); before the global table, which most rows of a
-    // column with that many keys end up in anyway, 8 (24: 30 us more of 270).
-    constexpr int probes = GLOBAL ? 8 : PER < 16 ? PS : 48;
+    // partition; 24 let 5,500 random keys of 4 bytes and 3,500 of 8 find one (48:
+    // 7,500 and 5,000, but twice the loop unrolled into every row's place: 20M
+    // int16 rows of 60 values 28 us for 19); before the global table, which most
+    // rows of a column with that many keys end up in anyway, 8.
+    constexpr int probes = GLOBAL ? 8 : PER < 16 ? PS : 24;
     // Adds `add` rows of `key` to its partition; a key without a slot goes to
     // the global table, or ends the count.
     auto lds_add = [&](KT key, uint32_t add) {
@@ -662,23 +663,25 @@ __global__ __launch_bounds__(kHistThreads) void k_hist_count(const T* __restrict
         __shared__ uint32_t first[kHistThreads + 1];
         __shared__ uint32_t red[kHistThreads / kWave];
         __shared__ HistCtl ctl;
-        __shared__ uint32_t s_distinct;
+        __shared__ uint32_t s_distinct, s_most;
         __shared__ Cand sc[kHistThreads / kWave * kMaxK];
         __shared__ Cand best[kMaxK];
         const uint32_t blocks = gridDim.x;  // <= kHistThreads
         const uint32_t have = threadIdx.x < blocks ? ld_agent(&off[(size_t)kHistParts * blocks + threadIdx.x]) : 0u;
         if (threadIdx.x == 0) {
             ctl = HistCtl{};
-            s_distinct = 0;
+            s_distinct = s_most = 0;
         }
         fill(skey, sizeof skey, ~0u);
         fill(scnt, sizeof scnt, 0u);
         uint32_t total;
         first[threadIdx.x] = block_exclusive_scan<uint32_t, kHistThreads>(have, &total, red);
+        const uint32_t most = wave_max(have);
+        if (lane == 0) atomicMax(&s_most, most);
         __syncthreads();
         fold_info<kHistThreads>(info, blocks, &ctl);
         HistResult* out = reinterpret_cast<HistResult*>(tail.host.dst);
-        const bool few = total <= (uint32_t)kLdsSlots && n < (1ull << 32);
+        const bool few = (total <= (uint32_t)kLdsSlots || (total <= kTailEntries && s_most <= kTailKeys)) && n < (1ull << 32);
         constexpr int F = 4;  // entries in flight a thread
         for (uint32_t e0 = threadIdx.x; few && e0 < total; e0 += F * kHistThreads) {
             KT key[F];
