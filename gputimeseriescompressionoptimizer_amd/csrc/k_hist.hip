@@ -241,9 +241,9 @@ struct HistInfo {
 // too small.  With 16 rows a thread every column of more than 5,500 random keys
 // (3,500 of 8 bytes) was counted in vain and then again in the global table.  A
 // dictionary encode of 100,000 int32 rows with 16,000 keys 231 us, of int64 rows
-// 251, now 85 and 81 (in the global table alone 184 and 185); of 1M rows with
-// 60,000 keys 1187 and 1247, now 126 and 106; of 100,000 rows with 50 keys 55 and
-// 56, now 52.
+// 251, now 86 and 82 (in the global table alone 184 and 185); of 1M rows with
+// 60,000 keys 1187 and 1247, now 125 and 106; of 100,000 rows with 50 keys 55 and
+// 56, now 53 and 52.
 constexpr int kHistThreads = 1024, kMergeThreads = 1024, kMergeSlots = 4096;
 template <typename T> constexpr int few_rows() { return sizeof(T) == 8 ? 4 : sizeof(T) == 1 ? 16 : 8; }
 // Entries a workgroup may write out.
@@ -1113,7 +1113,7 @@ void topk_most_frequent(Ctx* c, int dtype, const void* x, size_t n, int K, uint6
         } else {
             if (counted(std::integral_constant<int, 16>{}, cus)) return take(found);
             // the merge takes the entries of up to kMergeThreads workgroups (4M int32
-            // rows of 30,000 keys 287 us, 422 through the global table)
+            // rows of 16,000 keys 244 us, 416 through the global table)
             if (Few::value < 16 && n <= few * kMergeThreads && counted(Few{}, kMergeThreads)) return take(found);
         }
         const size_t g = std::min((n + 16 * kHistThreads - 1) / (16 * kHistThreads), cus);

@@ -7,9 +7,11 @@
  * are ddj_buf handles allocated from the context's caching allocator.  All
  * GPU work of a context runs on its own HIP stream; calls on one context
  * are serialised by the caller, separate contexts are independent.  A call
- * may return with its last kernels still queued on that stream: copies to the
- * host through this interface come after them, and a caller's own stream waits
- * on ddj_ctx_stream.
+ * may return with its last kernels still queued on that stream, its outputs
+ * not yet written and its inputs not yet read: copies through this interface,
+ * ddj_buf_free and later calls on the context come after them; a caller's own
+ * stream waits on ddj_ctx_stream before it reads the outputs, and before it
+ * changes or frees an input.
  *
  * Status codes replace the reference's exit(1) / print-and-continue error
  * handling (core/macros.h:8-17).
